@@ -263,9 +263,10 @@ int fla_hip_dsgesv(int n, int nrhs, double* A, int lda, int* p, const double* B,
    [3] FP64 products with A, [4] ||A||_inf, [5] GMRES iterations, [6] the
    reduced-precision factorization's info. */
 int fla_hip_mp_last_stats(double* out, int nout);
-/* Panel solve of the reduced-precision factor: 0 blocked substitution,
-   1 (default) multiplication by the inverse of each 128 x 128 diagonal
-   factor. */
+/* Panel solve of the reduced-precision factor: 0 backward-stable, 1 product
+   with the diagonal factors' inverses.  One panel solve serves both (inverse
+   product corrected to substitution's accuracy), so the choice has no effect
+   any more. */
 int fla_hip_mp_set_panel(int inverse);
 /* CUs left out of the reduced-precision factor's update stream for its panel
    chain (default 64; 0 = no mask). */

@@ -11,12 +11,16 @@
 // (FLA_Chol_u_blk_var3.c:38-54) is the lower algorithm on A' (the triangles
 // are exchanged in place before and after).
 #include "fla_hip_internal.h"
-#include "fla_hip_lds_tri.h"
+
+#include <utility>
 
 namespace {
 
-constexpr int PB = 128;  // panel sub-block width (diagonal block order)
-constexpr int LB = 32;   // leaf width of the panel triangular solve
+constexpr int PB = 128;       // panel sub-block width (diagonal block order)
+constexpr int NT16 = PB / 16;  // 16-blocks of a diagonal block
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ double readlane_d(double v, int lane) {
   const long long b = __double_as_longlong(v);
@@ -25,171 +29,315 @@ __device__ __forceinline__ double readlane_d(double v, int lane) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-constexpr int DLD = PB + 1;  // LDS leading dimension of the diagonal block
-
-// Single-workgroup Cholesky of the nb x nb lower block at A (nb <= 128),
-// blocked by 32 inside the workgroup (the reference's var3 structure one
-// level down, FLA_Chol_l_blk_var3.c:13-66):
-//   1. wave 0 factors the 32x32 diagonal block, lane = row, pivots broadcast
-//      with readlane (no barriers): d = sqrt(a_jj) with bl1_dsqrte's failure
-//      rule, l_ij = a_ij * (1/d), a_ic -= l_ij l_cj;
-//   2. the rows below are solved against it (lane = row, row in VGPRs, the
-//      32x32 factor read from LDS by broadcast), dtrsm's update order;
-//   3. the trailing part is updated on MFMA (16x16 lower tiles, rank 32).
-// The block lives in LDS (129 KB); padding beyond nb is the identity.
-// INV: after a successful factor, also writes inv(L) (lower, ld 128, zero
-// upper part) to W, inverted in LDS (fla_hip_lds_tri.h).
-template <bool INV>
-__global__ __launch_bounds__(256) void potrf_blk_kernel(int nb, double* __restrict__ A, long lda,
-                                                        int col_offset, int* __restrict__ info,
-                                                        double* __restrict__ W) {
-  if (*info >= 0) return;
-  __shared__ double S[PB * DLD];
-  __shared__ int fail;
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  // 64 elements per thread, 16 loads in flight at a time
-  for (int q0 = 0; q0 < PB * PB / 256; q0 += 16) {
-    double v[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int e = t + (q0 + q) * 256;
-      const int i = e & (PB - 1), c = e >> 7;
-      v[q] = (i < nb && c < nb) ? A[(long)i + (long)c * lda] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int e = t + (q0 + q) * 256;
-      const int i = e & (PB - 1), c = e >> 7;
-      S[c * DLD + i] = (i < c) ? 0.0 : ((i < nb) ? v[q] : (i == c ? 1.0 : 0.0));
-    }
-  }
-  if (t == 0) fail = -1;
-  __syncthreads();
-  for (int b = 0; b < PB; b += LB) {
-    // 1. diagonal 32x32 block: wave 0, lanes 0..31
-    if (wave == 0) {
-      const int r = b + (lane & 31);
-      double x[LB];
-#pragma unroll
-      for (int c = 0; c < LB; ++c) x[c] = S[(b + c) * DLD + r];
-      int f = -1;
-#pragma unroll
-      for (int j = 0; j < LB; ++j) {
-        if (f >= 0) continue;  // uniform: a failed column stops the sweep
-        const double ajj = readlane_d(x[j], j);
-        if (!(ajj > 0.0)) {  // <= 0 or NaN, as bl1_dsqrte
-          f = j;
-          continue;
-        }
-        const double d = sqrt(ajj);
-        const double inv = 1.0 / d;
-        if ((lane & 31) > j) x[j] *= inv;
-        if ((lane & 31) == j) x[j] = d;
-        // entries above the diagonal (lane < c) take garbage here and are
-        // never stored or read, so the update needs no per-lane predicate
-#pragma unroll
-        for (int c = j + 1; c < LB; ++c) x[c] -= x[j] * readlane_d(x[j], c);
-      }
-      if (lane < 32) {
-#pragma unroll
-        for (int c = 0; c < LB; ++c)
-          if (lane >= c && (f < 0 || c < f)) S[(b + c) * DLD + r] = x[c];
-      }
-      if (lane == 0 && f >= 0) fail = b + f;
-    }
-    __syncthreads();
-    if (fail >= 0) break;
-    // 2. rows below the diagonal block: X := X * inv(L_bb)'
-    const int nrow = PB - b - LB;
-    if (t < nrow) {
-      const int r = b + LB + t;
-      double x[LB];
-#pragma unroll
-      for (int c = 0; c < LB; ++c) x[c] = S[(b + c) * DLD + r];
-#pragma unroll
-      for (int j = 0; j < LB; ++j) {
-        x[j] *= 1.0 / S[(b + j) * DLD + b + j];
-#pragma unroll
-        for (int c = j + 1; c < LB; ++c) x[c] -= S[(b + j) * DLD + b + c] * x[j];
-      }
-#pragma unroll
-      for (int c = 0; c < LB; ++c) S[(b + c) * DLD + r] = x[c];
-    }
-    __syncthreads();
-    // 3. trailing update A(i, c) -= sum_k L(i, k) L(c, k), i >= c >= b + 32,
-    //    on v_mfma_f64_16x16x4f64: 16 x 16 lower tiles spread over the waves;
-    //    lane (li, lk), register q holds D(16 ti + li, 16 tj + lk + 4 q).
-    {
-      const int T16 = nrow / 16;
-      const int ntile = T16 * (T16 + 1) / 2;
-      const int i0 = b + LB;
-      const int li = lane & 15, lk = lane >> 4;
-      for (int tt = wave; tt < ntile; tt += 4) {
-        int ti = (int)((sqrt(8.0 * tt + 1.0) - 1.0) * 0.5);
-        while (ti * (ti + 1) / 2 > tt) --ti;
-        while ((ti + 1) * (ti + 2) / 2 <= tt) ++ti;
-        const int tj = tt - ti * (ti + 1) / 2;
-        fla_lds::d4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int ks = 0; ks < LB / 4; ++ks) {
-          const double* col = S + (b + 4 * ks + lk) * DLD;
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(col[i0 + 16 * tj + li], col[i0 + 16 * ti + li],
-                                                     acc, 0, 0, 0);
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int row = i0 + 16 * ti + li, cc = i0 + 16 * tj + lk + 4 * q;
-          if (row >= cc) S[cc * DLD + row] -= acc[q];
-        }
-      }
-    }
-    __syncthreads();
-  }
-  const int ncols = (fail >= 0) ? fail : nb;
-  for (int e = t; e < PB * PB; e += 256) {
-    const int i = e & (PB - 1), c = e >> 7;
-    if (i >= c && i < nb && c < ncols) A[(long)i + (long)c * lda] = S[c * DLD + i];
-  }
-  if (t == 0 && fail >= 0) *info = col_offset + fail;
-  if (INV && fail < 0) {
-    // the strictly upper part of S is zero and the padding the identity
-    __syncthreads();
-    fla_lds::trtri_lower_lds(S, t);
-    for (int e = t; e < PB * PB; e += 256) {
-      const int i = e & (PB - 1), c = e >> 7;
-      W[i + c * PB] = (i >= c) ? S[c * DLD + i] : 0.0;
-    }
-  }
+// Barrier that orders LDS accesses only: __syncthreads would also wait for
+// the global stores in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// Leaf of the panel solve: X := X * inv(L)' for an m x nb strip (nb <= 32),
-// L lower non-unit.  One lane per row with the row in VGPRs, L through
-// uniform loads; the update order of dtrsm_('R','L','T','N')
-// (src/flablas/f2c/dtrsm.c): x_j *= 1/l_jj, then x_c -= l_cj * x_j.
-template <bool FULL>
-__global__ __launch_bounds__(64) void trsm_rlt_leaf_kernel(int m, int nb,
-                                                           const double* __restrict__ L, long ldl,
-                                                           double* __restrict__ X, long ldx,
-                                                           const int* __restrict__ abort_flag) {
-  if (abort_flag && *abort_flag >= 0) return;
-  const int r = blockIdx.x * 64 + threadIdx.x;
-  if (r >= m) return;
-  double x[LB];
+// 16 x 16 blocks in fragment order.  v_mfma_f64_16x16x4f64 leaves D(x, y) in
+// lane 16*(x%4) + y, register x/4; with x the column and y the row of a
+// block X, lane (li = lane%16, lk = lane/16) holds X(li, lk + 4 s) in
+// register s.  That register is at the same time the lane's operand of step
+// s of a product over X's columns, as the row operand (X Z') and as the
+// column operand (Z X'), so blocks move between products without any
+// shuffle.  In memory a block is 128 d2: entry [p][lane] = steps 2p, 2p+1.
+__device__ __forceinline__ d4 mfma_step(double colf, double rowf, d4 acc) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(colf, rowf, acc, 0, 0, 0);
+}
+// acc + R C' for blocks R (row operand) and C (column operand: c0, c1).
+__device__ __forceinline__ d4 mfma_block(d2 c0, d2 c1, d4 r, d4 acc) {
+  acc = mfma_step(c0.x, r[0], acc);
+  acc = mfma_step(c0.y, r[1], acc);
+  acc = mfma_step(c1.x, r[2], acc);
+  return mfma_step(c1.y, r[3], acc);
+}
+// X := T inv(L)' for a block T, given inv(L) (y) and -L (l): the product with
+// the explicit inverse, then one correction with its residual,
+// X += (T - X L') inv(L)', which brings the backward error of the inverse
+// (eps cond(L)) to that of substitution.  12 matrix steps against 136
+// dependent vector operations per row.
+__device__ __forceinline__ d4 solve_block(const d2 (&y)[2], const d2 (&l)[2], d4 t) {
+  const d4 zero = {0.0, 0.0, 0.0, 0.0};
+  const d4 x0 = mfma_block(y[0], y[1], t, zero);
+  const d4 r = mfma_block(l[0], l[1], x0, t);
+  return mfma_block(y[0], y[1], r, x0);
+}
+
+// The blocks of a factored 128 x 128 diagonal block L as the panel solve
+// reads them: for 16-column block jb the negated blocks left of the diagonal
+// -L(jb, 0..jb-1), then inv(L(jb, jb)), then -L(jb, jb).
+constexpr int frag_q0(int jb) { return jb * (jb - 1) / 2 + 2 * jb; }
+constexpr int NFRAG = frag_q0(NT16);
+static_assert(NFRAG * 256 <= PB * PB, "the fragments fit the 128 x 128 scratch block");
+
+// One wave factors a 16 x 16 symmetric block and inverts the factor.  Lane li
+// of each row of 16 lanes holds row li (x[c] = a(li, c), both triangles) and
+// column li of the identity (w): the sweep of Cholesky is also the forward
+// substitution of L Y = I, so w ends as column li of inv(L).  Column j's
+// multiplier of column c, a_jc, is broadcast from lane j's upper half by the
+// update instruction itself (DPP row_newbcast):
+//   x_c -= a_jc (x_j / a_jj),  w_c -= a_jc (w_j / d) / d,
+// two instructions per column.  (Through lane reads the pivot alone took 80
+// cycles from its update to its first use, and every multiplier two reads.)
+// A VALU result is a DPP source only two wait states later: the statements
+// below keep other instructions in between, or carry the s_nop.
+template <int J, int C>
+__device__ __forceinline__ void sweep_update(double& w, double& x, double nw, double nx) {
+  asm volatile(
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %1, %1, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf"
+      : "+v"(w), "+v"(x)
+      : "v"(nw), "v"(nx), "i"(J));
+}
+// Updates of column J for C0 <= C < C1 (none past 15).
+template <int J, int C0, int C1>
+__device__ __forceinline__ void sweep_updates(double (&x)[16], double (&w)[16], double nw,
+                                              double nx) {
+  if constexpr (C0 < C1 && C0 < 16) {
+    sweep_update<J, C0>(w[C0], x[C0], nw, nx);
+    sweep_updates<J, C0 + 1, C1>(x, w, nw, nx);
+  }
+}
+template <int J>
+__device__ __forceinline__ double bcast16(double x) {
+  double a;
+  asm volatile("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+               : "=v"(a)
+               : "v"(x), "i"(J));
+  return a;
+}
+
+// Column J with the pivot a already broadcast.  Goldschmidt's iteration from
+// v_rsq_f64 gives g -> sqrt(a) and h -> 1/(2 sqrt(a)) with the common error
+// e = 1/2 - g h, which also corrects the reciprocal; the root takes two
+// residual corrections (Markstein).  The updates of column J - 1 right of
+// column J (multipliers nxp, nwp) fill the chain's latencies; column J + 1 is
+// updated first, so that the next pivot is on its way at the end.  piv: lane
+// J's root, checked once after the sweep.
+template <int J>
+__device__ __forceinline__ void sweep_column(double (&x)[16], double (&w)[16], int li, double& piv,
+                                             double& a, double& nxp, double& nwp) {
+  constexpr int N = J > 0 ? 15 - J : 0, C1 = J + 1 + (N + 2) / 3, C2 = J + 1 + (2 * N + 2) / 3;
+  constexpr int JP = J > 0 ? J - 1 : 0;
+  const double y = __builtin_amdgcn_rsq(a);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (J > 0) sweep_updates<JP, J + 1, C1>(x, w, nwp, nxp);
+  __builtin_amdgcn_sched_barrier(0);
+  double g = a * y, h = 0.5 * y;
+  double e = fma(-h, g, 0.5);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (J > 0) sweep_updates<JP, C1, C2>(x, w, nwp, nxp);
+  __builtin_amdgcn_sched_barrier(0);
+  h = fma(h, e, h);
+  g = fma(g, e, g);
+  e = fma(-h, g, 0.5);
+  const double h2 = h + h;
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (J > 0) sweep_updates<JP, C2, 16>(x, w, nwp, nxp);
+  __builtin_amdgcn_sched_barrier(0);
+  const double inv = fma(h2, e, h2);
+  const double xs = x[J] * inv, ws = w[J] * inv;
+  nxp = -(xs * inv);
+  nwp = -(ws * inv);
+  const double a0 = a;
+  if constexpr (J < 15) {
+    sweep_update<J, J + 1>(w[J + 1], x[J + 1], nwp, nxp);
+    a = bcast16<J + 1>(x[J + 1]);
+  }
+  g = fma(fma(-g, g, a0), h, g);
+  const double d = fma(fma(-g, g, a0), h, g);
+  x[J] = li == J ? d : xs;
+  w[J] = ws;
+  piv = li == J ? d : piv;
+}
+template <int... J>
+__device__ __forceinline__ void sweep16(double (&x)[16], double (&w)[16], int li, double& piv,
+                                        std::integer_sequence<int, J...>) {
+  double a = bcast16<0>(x[0]), nxp = 0.0, nwp = 0.0;
+  (sweep_column<J>(x, w, li, piv, a, nxp, nwp), ...);
+}
+
+// The same with the library's root and division, any pivot range; returns the
+// first column whose pivot is <= 0 or NaN (bl1_dsqrte's rule), else -1.
+__device__ __noinline__ int sweep16_any(double* z, int lane) {
+  const int li = lane & 15;
+  double x[16], w[16];
 #pragma unroll
-  for (int c = 0; c < LB; ++c) x[c] = (FULL || c < nb) ? X[(long)r + (long)c * ldx] : 0.0;
+  for (int c = 0; c < 16; ++c) {
+    x[c] = z[li * 18 + c];
+    w[c] = c == li ? 1.0 : 0.0;
+  }
+  int f = -1;
 #pragma unroll
-  for (int j = 0; j < LB; ++j) {
-    if (FULL || j < nb) {
-      x[j] *= 1.0 / L[(long)j + (long)j * ldl];
+  for (int j = 0; j < 16; ++j) {
+    const double a = readlane_d(x[j], j);
+    if (f < 0 && !(a > 0.0)) f = j;
+    const double d = sqrt(a), inv = 1.0 / d;
+    const double xs = x[j] * inv, ws = w[j] * inv;
 #pragma unroll
-      for (int c = j + 1; c < LB; ++c)
-        if (FULL || c < nb) x[c] -= L[(long)c + (long)j * ldl] * x[j];
+    for (int c = j + 1; c < 16; ++c) {
+      const double l = readlane_d(x[c], j) * inv;
+      w[c] = fma(-ws, l, w[c]);
+      x[c] = fma(-xs, l, x[c]);
     }
+    x[j] = li == j ? d : xs;
+    w[j] = ws;
+  }
+  if (lane < 32) {
+#pragma unroll
+    for (int q = 0; q < 16; ++q) z[lane * 18 + q] = lane < 16 ? x[q] : w[q];
+  }
+  return f;
+}
+
+// A factored 16 x 16 diagonal block in LDS: rows 0..15 hold L (below and on
+// the diagonal), row 16 + c column c of inv(L).  The row length keeps 16-byte
+// accesses aligned and spreads the rows over the banks.
+constexpr int ZLD = 18;
+
+// Factors the symmetric block dg (fragment order) into z, one wave.  Returns
+// the first failing column or -1.  Pivots outside [2^-700, 2^1000] (products
+// of the fast sweep could under- or overflow) and failing ones take the
+// general sweep.
+__device__ __forceinline__ int factor16(d4 dg, double* z, int lane) {
+  const int li = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) z[li * ZLD + lk + 4 * r] = dg[r];
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  double x[16], w[16], piv = 0.0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const d2 v = *reinterpret_cast<const d2*>(z + li * ZLD + 2 * q);
+    x[2 * q] = v.x;
+    x[2 * q + 1] = v.y;
+    w[2 * q] = 2 * q == li ? 1.0 : 0.0;
+    w[2 * q + 1] = 2 * q + 1 == li ? 1.0 : 0.0;
+  }
+  // every x is written two wait states before the first broadcast reads it
+  asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]),
+               "+v"(x[6]), "+v"(x[7]));
+  asm volatile("s_nop 1" : "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]),
+               "+v"(x[13]), "+v"(x[14]), "+v"(x[15]));
+  sweep16(x, w, li, piv, std::make_integer_sequence<int, 16>{});
+  if (!__all(piv >= 0x1p-350 && piv <= 0x1p500)) return sweep16_any(z, lane);
+  if (lane < 32) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      *reinterpret_cast<d2*>(z + lane * ZLD + 2 * q) =
+          lane < 16 ? d2{x[2 * q], x[2 * q + 1]} : d2{w[2 * q], w[2 * q + 1]};
+  }
+  return -1;
+}
+
+// Single-workgroup Cholesky of the nb x nb lower block at A (nb <= 128, padded
+// with the identity) over 16-column blocks with the whole block in registers:
+// wave w owns block row w (blocks (w, 0..w) in fragment order).  Step b, after
+// one barrier: every wave below applies the previous step's update to its
+// block (w, b), solves it against the factored diagonal block b, applies it
+// to its own diagonal block, and publishes it through LDS; wave b + 1 then
+// factors its diagonal block (factor16) while the others apply the previous
+// step's update to their remaining blocks.
+// Bound: the serial chain of 128 pivots (broadcast, root, reciprocal, scale,
+// update: about 240 cycles each) plus 20 matrix steps (about 2000 cycles with
+// their operands' LDS reads) per 16 columns.  128 columns take 28 us alone, 73
+// with the block in LDS, lane reads for the multipliers and three barriers
+// per 32 columns.
+// W receives the blocks of L for the panel solve (see frag_q0).  A failed
+// block leaves its columns from the failing one on unwritten.
+__global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restrict__ A, long lda,
+                                                        int col_offset, int* __restrict__ info,
+                                                        d2* __restrict__ W) {
+  if (*info >= 0) return;
+  __shared__ d2 Xf[2][NT16][2][64];  // the solved blocks (negated) of a block column, by parity
+  __shared__ __attribute__((aligned(16))) double Z[2][32 * ZLD];
+  __shared__ int fail;
+  const int t = threadIdx.x, lane = t & 63;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  if (t == 0) fail = -1;
+  // c[i]: block (w, b + i) at step b (i < w - b); dg: block (w, w)
+  d4 c[NT16 - 1], dg;
+  const int row = 16 * w + li;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int col = 16 * w + lk + 4 * r;
+    const int i = row > col ? row : col, j = row > col ? col : row;  // the lower triangle's copy
+    dg[r] = i < nb ? A[(long)i + (long)j * lda] : (row == col ? 1.0 : 0.0);
   }
 #pragma unroll
-  for (int c = 0; c < LB; ++c)
-    if (FULL || c < nb) X[(long)r + (long)c * ldx] = x[c];
+  for (int k = 0; k < NT16 - 1; ++k) {
+    if (k >= w) break;  // uniform
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      c[k][r] = row < nb ? A[(long)row + (long)(16 * k + lk + 4 * r) * lda] : 0.0;
+  }
+  if (w == 0) {
+    const int f = factor16(dg, Z[0], lane);
+    if (lane == 0 && f >= 0) fail = f;
+  }
+  d4 xr = {0.0, 0.0, 0.0, 0.0};  // this row's block of the previous block column
+  for (int b = 0; b < NT16; ++b) {
+    lds_barrier();
+    const int par = b & 1;
+    const double* const z = Z[par];
+    const int flim = fail;
+    if (w > b && flim < 0) {
+      __builtin_amdgcn_s_setprio(2);
+      d2 y[2], l[2];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int k = lk + 4 * s;
+        y[s >> 1][s & 1] = z[(16 + k) * ZLD + li];
+        const double v = z[li * ZLD + k];
+        l[s >> 1][s & 1] = k <= li ? -v : 0.0;
+      }
+      d4 cur = c[0];
+      if (b > 0) cur = mfma_block(Xf[par ^ 1][b][0][lane], Xf[par ^ 1][b][1][lane], xr, cur);
+      const d4 xn = solve_block(y, l, cur);
+      const d2 n0 = d2{-xn[0], -xn[1]}, n1 = d2{-xn[2], -xn[3]};
+      Xf[par][w][0][lane] = n0;
+      Xf[par][w][1][lane] = n1;
+      dg = mfma_block(n0, n1, xn, dg);
+      if (w == b + 1) {
+        __builtin_amdgcn_s_setprio(3);
+        const int f = factor16(dg, Z[par ^ 1], lane);
+        if (lane == 0 && f >= 0) fail = 16 * w + f;
+      }
+      __builtin_amdgcn_s_setprio(0);
+      // the previous step's update of the blocks right of b, moved one place
+#pragma unroll
+      for (int i = 1; i < NT16 - 1; ++i) {
+        if (i >= w - b) break;  // uniform
+        c[i - 1] = b > 0 ? mfma_block(Xf[par ^ 1][b + i][0][lane], Xf[par ^ 1][b + i][1][lane], xr,
+                                      c[i])
+                         : c[i];
+      }
+      xr = xn;
+      d2* const Wq = W + (frag_q0(w) + b) * 128;
+      Wq[lane] = n0;
+      Wq[64 + lane] = n1;
+      if (row < nb) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) A[(long)row + (long)(16 * b + lk + 4 * r) * lda] = xn[r];
+      }
+    } else if (w == b) {
+      // the diagonal block: L to A (up to a failing column), inv(L) and -L to W
+      const int jend = flim < 0 ? 16 : flim - 16 * b;
+      d2* const Wq = W + (frag_q0(b) + b) * 128;
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int k0 = lk + 8 * p, k1 = k0 + 4;
+        const double v0 = z[li * ZLD + k0], v1 = z[li * ZLD + k1];
+        if (k0 <= li && row < nb && k0 < jend) A[(long)row + (long)(16 * b + k0) * lda] = v0;
+        if (k1 <= li && row < nb && k1 < jend) A[(long)row + (long)(16 * b + k1) * lda] = v1;
+        Wq[64 * p + lane] = d2{z[(16 + k0) * ZLD + li], z[(16 + k1) * ZLD + li]};
+        Wq[128 + 64 * p + lane] = d2{k0 <= li ? -v0 : 0.0, k1 <= li ? -v1 : 0.0};
+      }
+    }
+    if (flim >= 0) break;
+  }
+  if (t == 0 && fail >= 0) *info = col_offset + fail;
 }
 
 // Exchanges A(i,j) and A(j,i) for all i > j, 32x32 tile pairs through LDS.
@@ -224,134 +372,85 @@ __global__ void set_int_kernel(int* p, int v) { *p = v; }
 
 }  // namespace
 
-bool g_trsm_rows = true;
-
-int launch_potrf_diag(hipStream_t s, int nb, double* A, long lda, int col_offset, int* info) {
-  if (nb <= 0) return FLA_HIP_OK;
-  if (nb > PB) return FLA_HIP_EARG;
-  hipLaunchKernelGGL(potrf_blk_kernel<false>, dim3(1), dim3(256), 0, s, nb, A, lda, col_offset,
-                     info, nullptr);
-  FLA_HIP_CHECK(hipGetLastError());
-  return FLA_HIP_OK;
-}
-
-// The same, and W (128 x 128, ld 128) := inv(L) when the factor succeeds.
-int launch_potrf_diag_inv(hipStream_t s, int nb, double* A, long lda, int col_offset, int* info,
-                          double* W) {
-  if (nb <= 0) return FLA_HIP_OK;
-  if (nb > PB) return FLA_HIP_EARG;
-  hipLaunchKernelGGL(potrf_blk_kernel<true>, dim3(1), dim3(256), 0, s, nb, A, lda, col_offset,
-                     info, W);
-  FLA_HIP_CHECK(hipGetLastError());
-  return FLA_HIP_OK;
-}
-
-// A21 := A21 * inv(L11)' for an m x nb strip, L11 lower non-unit (nb <= 128):
-// one launch, one thread per row of the strip.  Columns are solved in blocks
-// of 32 held in VGPRs: first the contributions of the already solved columns
-// k (ascending, re-read by the thread that wrote them), then the 32 x 32
-// diagonal block by substitution -- dtrsm_('R','L','T','N')'s update order
-// (src/flablas/f2c/dtrsm.c), temp = 1/a_kk multiplied in.  L's columns
-// below the diagonal blocks are read with wave-uniform (scalar) loads, 32
-// at a time; the four 32 x 32 diagonal blocks, whose substitution would
-// otherwise wait on dozens of dependent scalar loads each, are first copied
-// into LDS (16.5 KB packed, small enough to share a CU with the update
-// kernel).
-template <bool FULL>
-__global__ __launch_bounds__(256) void trsm_rlt_rows_kernel(int m, int nb,
-                                                            const double* __restrict__ L,
-                                                            long ldl, double* __restrict__ X,
-                                                            long ldx, const int* __restrict__ abort) {
-  // diagonal block b, lower triangle packed by columns: (r, c), r >= c, at
-  // Ld[b][c*LB - c*(c-1)/2 + (r - c)]
-  __shared__ double Ld[PB / LB][LB * (LB + 1) / 2];
+// A21 := A21 inv(L11)' for an m x 128 strip, L11 given by the blocks that
+// potrf_blk_kernel left in W.  Each wave owns 16 rows, all 128 columns in
+// registers in fragment order; per 16-column block the contributions of the
+// solved blocks, then the diagonal block (solve_block).  L's blocks stream
+// from memory (88 KB, shared by every wave through the caches) PF blocks
+// ahead of their use; no LDS, so the workgroups fit beside the update
+// kernel's.  (32 rows per wave, with half the reads of L, spilled registers.)
+// Bound: one wave's chain of 208 matrix steps (5.8 us) while the rows fit the
+// chip once.  n = 5003: 11.5 us a launch on average against 87 for one thread
+// per row with substitution.
+__global__ __launch_bounds__(256, 2) void trsm_rlt_kernel(int m, const d2* __restrict__ W,
+                                                          double* __restrict__ X, long ldx,
+                                                          const int* __restrict__ abort) {
+  constexpr int PF = 6;
   if (abort && *abort >= 0) return;
-  const int nbk = FULL ? PB : nb;
-  {
-    // 16 elements per thread, all loads issued before the LDS stores
-    double v[(PB / LB) * LB * LB / 256];
+  const int lane = threadIdx.x & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const int row0 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * 16;
+  if (row0 >= m) return;
+  const bool in = row0 + li < m;
+  double* const xp = X + (in ? row0 + li : m - 1) + (long)lk * ldx;
+  d4 c[NT16];
+  d2 ring[PF][2];
+  const d2* const Wl = W + lane;
 #pragma unroll
-    for (int q = 0; q < (PB / LB) * LB * LB / 256; ++q) {
-      const int e = threadIdx.x + 256 * q;
-      const int b = e / (LB * LB), r = e % LB, c = (e / LB) % LB;
-      const int gr = b * LB + r, gc = b * LB + c;
-      v[q] = (gr < nbk && gc < nbk && r >= c) ? L[gr + (long)gc * ldl] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < (PB / LB) * LB * LB / 256; ++q) {
-      const int e = threadIdx.x + 256 * q;
-      const int b = e / (LB * LB), r = e % LB, c = (e / LB) % LB;
-      if (b * LB + r < nbk && b * LB + c < nbk && r >= c)
-        Ld[b][c * LB - (c * (c - 1)) / 2 + (r - c)] = v[q];
-    }
+  for (int q = 0; q < PF; ++q) {
+    ring[q][0] = Wl[q * 128];
+    ring[q][1] = Wl[q * 128 + 64];
   }
-  __syncthreads();
-  const int row = blockIdx.x * 256 + threadIdx.x;
-  if (row >= m) return;
-  double* xr = X + row;
-  for (int jb = 0; jb < nbk; jb += LB) {
-    const int w = FULL ? LB : ((nbk - jb) < LB ? (nbk - jb) : LB);
-    double x[LB];
 #pragma unroll
-    for (int c = 0; c < LB; ++c) x[c] = (FULL || c < w) ? xr[(long)(jb + c) * ldx] : 0.0;
+  for (int k = 0; k < NT16; ++k)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) c[k][r] = xp[(long)(16 * k + 4 * r) * ldx];
+#pragma unroll
+  for (int jb = 0; jb < NT16; ++jb) {
+#pragma unroll
     for (int k = 0; k < jb; ++k) {
-      const double xk = xr[(long)k * ldx];
-      const double* lk = L + (long)k * ldl + jb;
-#pragma unroll
-      for (int c = 0; c < LB; ++c)
-        if (FULL || c < w) x[c] -= lk[c] * xk;
-    }
-    const double* Lb = Ld[jb / LB];
-#pragma unroll
-    for (int j = 0; j < LB; ++j) {
-      if (FULL || j < w) {
-        const double* lj = Lb + (j * LB - (j * (j - 1)) / 2);  // column j from its diagonal
-        x[j] *= 1.0 / lj[0];
-#pragma unroll
-        for (int c = j + 1; c < LB; ++c)
-          if (FULL || c < w) x[c] -= lj[c - j] * x[j];
+      const int q = frag_q0(jb) + k;
+      c[jb] = mfma_block(ring[q % PF][0], ring[q % PF][1], c[k], c[jb]);
+      if (q + PF < NFRAG) {
+        ring[q % PF][0] = Wl[(q + PF) * 128];
+        ring[q % PF][1] = Wl[(q + PF) * 128 + 64];
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
+    const int q = frag_q0(jb) + jb;
+    c[jb] = solve_block(ring[q % PF], ring[(q + 1) % PF], c[jb]);
 #pragma unroll
-    for (int c = 0; c < LB; ++c)
-      if (FULL || c < w) xr[(long)(jb + c) * ldx] = x[c];
+    for (int u = 0; u < 2; ++u)
+      if (q + u + PF < NFRAG) {
+        ring[(q + u) % PF][0] = Wl[(q + u + PF) * 128];
+        ring[(q + u) % PF][1] = Wl[(q + u + PF) * 128 + 64];
+      }
+    if (in) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) xp[(long)(16 * jb + 4 * r) * ldx] = c[jb][r];
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-int launch_trsm_rlt(hipStream_t s, int m, int nb, const double* L11, long ldl, double* A21,
-                    long lda, const int* abort_flag) {
-  if (m <= 0 || nb <= 0) return FLA_HIP_OK;
+// Single-workgroup Cholesky of an nb x nb lower diagonal block (nb <= 128);
+// the blocks of L for launch_trsm_rlt go to W.
+static int launch_potrf_diag(hipStream_t s, int nb, double* A, long lda, int col_offset, int* info,
+                             double* W) {
+  if (nb <= 0) return FLA_HIP_OK;
   if (nb > PB) return FLA_HIP_EARG;
-  if (g_trsm_rows) {
-    const unsigned g = (unsigned)((m + 255) / 256);
-    if (nb == PB)
-      hipLaunchKernelGGL(trsm_rlt_rows_kernel<true>, dim3(g), dim3(256), 0, s, m, nb, L11, ldl,
-                         A21, lda, abort_flag);
-    else
-      hipLaunchKernelGGL(trsm_rlt_rows_kernel<false>, dim3(g), dim3(256), 0, s, m, nb, L11, ldl,
-                         A21, lda, abort_flag);
-    FLA_HIP_CHECK(hipGetLastError());
-    return FLA_HIP_OK;
-  }
-  for (int b0 = 0; b0 < nb; b0 += LB) {
-    const int w = (nb - b0) < LB ? (nb - b0) : LB;
-    const double* Lbb = L11 + (long)b0 + (long)b0 * ldl;
-    double* Xb = A21 + (long)b0 * lda;
-    if (w == LB)
-      hipLaunchKernelGGL(trsm_rlt_leaf_kernel<true>, dim3((m + 63) / 64), dim3(64), 0, s, m, w,
-                         Lbb, ldl, Xb, lda, abort_flag);
-    else
-      hipLaunchKernelGGL(trsm_rlt_leaf_kernel<false>, dim3((m + 63) / 64), dim3(64), 0, s, m, w,
-                         Lbb, ldl, Xb, lda, abort_flag);
-    FLA_HIP_CHECK(hipGetLastError());
-    const int rest = nb - b0 - w;
-    if (rest > 0) {
-      // X[:, b0+w:] -= X_b * L11[b0+w:, b0:b0+w]'
-      FLA_TRY(launch_dgemm_mfma(s, false, true, 0, m, rest, w, -1.0, Xb, lda,
-                                L11 + (long)(b0 + w) + (long)b0 * ldl, ldl, 1.0,
-                                Xb + (long)w * lda, lda, abort_flag));
-    }
-  }
+  hipLaunchKernelGGL(potrf_blk_kernel, dim3(1), dim3(512), 0, s, nb, A, lda, col_offset, info,
+                     reinterpret_cast<d2*>(W));
+  FLA_HIP_CHECK(hipGetLastError());
+  return FLA_HIP_OK;
+}
+
+static int launch_trsm_rlt(hipStream_t s, int m, const double* W, double* A21, long lda,
+                           const int* abort_flag) {
+  if (m <= 0) return FLA_HIP_OK;
+  hipLaunchKernelGGL(trsm_rlt_kernel, dim3((unsigned)((m + 63) / 64)), dim3(256), 0, s, m,
+                     reinterpret_cast<const d2*>(W), A21, lda, abort_flag);
+  FLA_HIP_CHECK(hipGetLastError());
   return FLA_HIP_OK;
 }
 
@@ -365,47 +464,22 @@ int launch_transpose_swap(hipStream_t s, int n, double* A, long lda) {
 }
 
 // Factors columns [k, k+kb) of the lower matrix (rows k..n-1): per 128-column
-// sub-block, the diagonal factor, the blocked panel solve of everything
-// below it, and the update of the panel's remaining columns.  All on stream s.
+// sub-block, the diagonal factor, the panel solve of everything below it
+// (only a matrix's last sub-block is narrower than 128, and nothing is below
+// it), and the update of the panel's remaining columns.  All on stream s.
 int chol_panel_f64(hipStream_t s, int n, double* A, long lda, int k, int kb, int* info) {
-  for (int kk = k; kk < k + kb; kk += PB) {
-    const int ib = (k + kb - kk) < PB ? (k + kb - kk) : PB;
-    double* Akk = A + (long)kk + (long)kk * lda;
-    FLA_TRY(launch_potrf_diag(s, ib, Akk, lda, kk, info));
-    const int mb = n - kk - ib;
-    if (mb <= 0) continue;
-    FLA_TRY(launch_trsm_rlt(s, mb, ib, Akk, lda, Akk + ib, lda, info));
-    const int w = k + kb - kk - ib;  // remaining columns of this panel
-    if (w > 0) {
-      const double* P = Akk + ib;  // mb x ib
-      FLA_TRY(launch_dgemm_mfma(s, false, true, 1, mb, w, ib, -1.0, P, lda, P, lda, 1.0,
-                                A + (long)(kk + ib) + (long)(kk + ib) * lda, lda, info));
-    }
-  }
-  return FLA_HIP_OK;
-}
-
-// Same factor with fewer launches, for callers that only need a
-// preconditioner-quality panel (the mixed-precision solver): each 128-block's
-// panel solve multiplies by the explicit inverse of its diagonal factor,
-// A21 := A21 * inv(L11)^T, one in-place MFMA GEMM instead of the blocked
-// substitution (every workgroup of that GEMM owns whole 128-wide rows).
-int chol_panel_f64_inv(hipStream_t s, int n, double* A, long lda, int k, int kb, int* info) {
   double* W = fla_ctx().dlinv;
   for (int kk = k; kk < k + kb; kk += PB) {
     const int ib = (k + kb - kk) < PB ? (k + kb - kk) : PB;
     double* Akk = A + (long)kk + (long)kk * lda;
+    FLA_TRY(launch_potrf_diag(s, ib, Akk, lda, kk, info, W));
     const int mb = n - kk - ib;
-    if (mb <= 0) {
-      FLA_TRY(launch_potrf_diag(s, ib, Akk, lda, kk, info));
-      continue;
-    }
-    FLA_TRY(launch_potrf_diag_inv(s, ib, Akk, lda, kk, info, W));
-    FLA_TRY(launch_dgemm_mfma(s, false, true, 0, mb, ib, ib, 1.0, Akk + ib, lda, W, PB, 0.0,
-                              Akk + ib, lda, info));
-    const int w = k + kb - kk - ib;
+    if (mb <= 0) continue;
+    if (ib != PB) return FLA_HIP_EARG;
+    FLA_TRY(launch_trsm_rlt(s, mb, W, Akk + ib, lda, info));
+    const int w = k + kb - kk - ib;  // remaining columns of this panel
     if (w > 0) {
-      const double* P = Akk + ib;
+      const double* P = Akk + ib;  // mb x ib
       FLA_TRY(launch_dgemm_mfma(s, false, true, 1, mb, w, ib, -1.0, P, lda, P, lda, 1.0,
                                 A + (long)(kk + ib) + (long)(kk + ib) * lda, lda, info));
     }
@@ -487,10 +561,5 @@ extern "C" int fla_hip_dpotrf(int uplo, int n, double* A, int lda, int* info) {
   FLA_HIP_CHECK(hipStreamSynchronize(c.s_update));
   fla_stats_harvest();
   *info = h;
-  return FLA_HIP_OK;
-}
-
-extern "C" int fla_hip_set_panel_solve(int rows) {
-  g_trsm_rows = rows != 0;
   return FLA_HIP_OK;
 }

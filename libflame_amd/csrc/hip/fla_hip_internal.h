@@ -61,7 +61,7 @@ struct FlaHipCtx {
   // move lists; then the triangular solve's copy of the finished right-hand-side
   // blocks (16 columns of n <= kUcSolveRows rows).
   char* uc = nullptr;
-  // 128 x 128 FP64 block: inverse of the current Cholesky diagonal block.
+  // The current Cholesky diagonal block as the panel solve reads it.
   double* dlinv = nullptr;
   int chol_nb = 0;  // 0: chosen from n (fla_chol_nb)
   int mp_nb = 0;    // reduced-precision factor block; 0: fla_chol_nb
@@ -198,12 +198,6 @@ extern int g_tile_group;
 int launch_dgemm_mfma(hipStream_t s, bool ta, bool tb, int mode, int m, int n, int k,
                       double alpha, const double* A, long lda, const double* B, long ldb,
                       double beta, double* C, long ldc, const int* abort_flag);
-// Single-workgroup Cholesky of an nb x nb lower diagonal block (nb <= 128).
-int launch_potrf_diag(hipStream_t s, int nb, double* A, long lda, int col_offset,
-                      int* info);
-// A21 := A21 * inv(L11)' for an m x nb strip, L11 lower non-unit (nb <= 128).
-int launch_trsm_rlt(hipStream_t s, int m, int nb, const double* L11, long ldl, double* A21,
-                    long lda, const int* abort_flag);
 // A12 := inv(L11) * A12, L11 unit lower nb x nb (nb <= 128): one lane per column.
 int launch_trsm_llnu(hipStream_t s, int ncols, int nb, const double* L11, long ldl, double* A12,
                      long lda);
@@ -234,9 +228,6 @@ int launch_trtri_blocks(hipStream_t s, int na, const double* A, long lda, bool u
 // FP64 factor of columns [k, k+kb) of a lower matrix (rows k..n-1): diagonal
 // factors, panel solves and in-panel updates, all on stream s.
 int chol_panel_f64(hipStream_t s, int n, double* A, long lda, int k, int kb, int* info);
-// The same with the panel solve done as a product with the explicit inverse
-// of each 128 x 128 diagonal factor (fewer launches, preconditioner quality).
-int chol_panel_f64_inv(hipStream_t s, int n, double* A, long lda, int k, int kb, int* info);
 // LU panel building blocks (fla_hip_getrf.hip) for the reduced-precision LU:
 // two alternating buffer sets for panel launches on matrices of up to m
 // rows; derr is the device int set when a bounded wait expires.

@@ -393,13 +393,6 @@ inline unsigned nblocks(long total) { return (unsigned)((total + 255) / 256); }
 
 // ---- reduced-precision factorization ------------------------------------------
 
-// Panel solve of the reduced-precision factor: the product with the inverse
-// of each 128 x 128 diagonal factor (default: an MFMA product instead of a
-// latency-bound substitution on the panel chain; the diagonal factors of a
-// matrix that the reduced precision can factor are well conditioned), or
-// blocked substitution (backward stable for any triangle).
-bool g_mp_panel_inverse = true;
-
 struct LpFactor {
   float* As = nullptr;      // FP32 trailing matrix (lower), ld n
   void* P[2] = {};          // packed panels (double-buffered across steps)
@@ -415,10 +408,7 @@ int lp_panel(hipStream_t s, int n, LpFactor& f, double* L, long ldl, int k, int 
                      f.As + (long)k + (long)k * n, (long)n, L + (long)k + (long)k * ldl, ldl,
                      f.amax + slot, 1);
   FLA_HIP_CHECK(hipGetLastError());
-  if (g_mp_panel_inverse)
-    FLA_TRY(chol_panel_f64_inv(s, n, L, ldl, k, kb, dinfo));
-  else
-    FLA_TRY(chol_panel_f64(s, n, L, ldl, k, kb, dinfo));
+  FLA_TRY(chol_panel_f64(s, n, L, ldl, k, kb, dinfo));
   const int m2 = m - kb;
   if (m2 > 0) {
     const double* L21 = L + (long)(k + kb) + (long)k * ldl;
@@ -1201,7 +1191,4 @@ extern "C" int fla_hip_mp_last_stats(double* out, int nout) {
   return FLA_HIP_OK;
 }
 
-extern "C" int fla_hip_mp_set_panel(int inverse) {
-  g_mp_panel_inverse = inverse != 0;
-  return FLA_HIP_OK;
-}
+extern "C" int fla_hip_mp_set_panel(int) { return FLA_HIP_OK; }

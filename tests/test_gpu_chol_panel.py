@@ -1,0 +1,43 @@
+"""The register-resident diagonal factor and the panel solve of FLA_Chol at the
+sizes and scales where they can go wrong: 16-column block edges inside the
+last 128-block, row counts around a wave's 16 rows, and pivots whose root and
+reciprocal leave the fast iteration's range.  Exact closed forms: every
+factor must come out bit for bit."""
+import numpy as np
+import pytest
+
+import libflame_amd as fla
+from tests.cases import exact_spd
+from tests.gpu_util import gpu_chol
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    fla.FLA_Init()
+    yield
+
+
+@pytest.mark.parametrize("n", [15, 16, 17, 33, 112, 113, 143, 144, 145, 191, 193, 400])
+def test_panel_block_edges_exact(n):
+    A, F = exact_spd(n, seed=3 * n + 1)
+    out, r = gpu_chol(A)
+    assert r == fla.FLA_SUCCESS
+    assert np.array_equal(np.tril(out), F)
+    assert np.array_equal(np.triu(out, 1), np.triu(A, 1))
+
+
+@pytest.mark.parametrize("e", [-400, -348, 420, 500])
+@pytest.mark.parametrize("n", [20, 150])
+def test_scaled_pivots_exact(n, e):
+    """A 2^(2e): L is the closed form times 2^e (pivots below 2^-700 and above
+    2^1000 take the library root and division)."""
+    A, F = exact_spd(n, seed=n)
+    with np.errstate(over="ignore"):
+        S = np.ldexp(A, 2 * e)
+    if not np.all(np.isfinite(S)):
+        pytest.skip("the scaled matrix overflows")
+    out, r = gpu_chol(S)
+    assert r == fla.FLA_SUCCESS
+    assert np.array_equal(np.tril(out), np.ldexp(F, e))

@@ -375,6 +375,133 @@ int launch_kp(hipStream_t s, bool vec, int mode, int m, int n, int k, double alp
   return FLA_HIP_OK;
 }
 
+// C := alpha*A*B' + beta*C for shapes whose 128 x 128 tiles would leave most
+// of the chip idle: 64 x 64 of C per workgroup of 4 waves, each 32 x 32 = 2 x 2
+// MFMA blocks, operands straight from memory into registers (a fragment load
+// is 16 consecutive rows of four columns, four 128-byte lines), no LDS and no
+// barrier.  KU k-steps of 4 are loaded while the previous KU feed the MFMAs.
+// Bound: one workgroup's K chain (K/4 steps of 4 x 64 cycles) plus two memory
+// round trips.  Rows past the edge read the last row and are not stored.
+template <int KU>
+__global__ __launch_bounds__(256, 2) void dgemm_nt_direct_kernel(
+    int mode, int m, int n, int k, double alpha, const double* A, long lda, const double* B,
+    long ldb, double beta, double* C, long ldc, int Tm, int Tn, int rpc,
+    const int* __restrict__ abort_flag) {
+  if (abort_flag && *abort_flag >= 0) return;
+  int ti, tj;
+  fla_tile_of(blockIdx.x, gridDim.x, mode, Tm, Tn, rpc, ti, tj);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  const int i0 = ti * 64 + (wave & 1) * 32, j0 = tj * 64 + (wave >> 1) * 32;
+  if (i0 >= m || j0 >= n || (mode == 1 && i0 + 31 < j0)) return;
+  // uniform column base plus a 32-bit lane offset per fragment
+  unsigned oa[2], ob[2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    const int i = i0 + 16 * a + li, j = j0 + 16 * a + li;
+    oa[a] = (unsigned)(i < m ? i : m - 1) + (unsigned)lk * (unsigned)lda;
+    ob[a] = (unsigned)(j < n ? j : n - 1) + (unsigned)lk * (unsigned)ldb;
+  }
+  typedef double Frag[KU][2];
+  Frag fa0, fb0, fa1, fb1;
+  auto load = [&](Frag& fa, Frag& fb, int s0) {
+#pragma unroll
+    for (int u = 0; u < KU; ++u) {
+      const double* const ca = A + (long)(4 * (s0 + u)) * lda;
+      const double* const cb = B + (long)(4 * (s0 + u)) * ldb;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        fa[u][a] = ca[oa[a]];
+        fb[u][a] = cb[ob[a]];
+      }
+    }
+  };
+  v4d acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = v4d{0.0, 0.0, 0.0, 0.0};
+  auto step = [&](const double (&fa)[2], const double (&fb)[2]) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[b], fa[a], acc[a][b], 0, 0, 0);
+  };
+  // whole chunks of KU steps in pairs; the load past the last chunk reads the
+  // last one again
+  const int nc = k / (4 * KU);
+  if (nc > 0) {
+    load(fa0, fb0, 0);
+    for (int c = 0; c < nc; c += 2) {
+      load(fa1, fb1, KU * (c + 1 < nc ? c + 1 : c));
+#pragma unroll
+      for (int u = 0; u < KU; ++u) step(fa0[u], fb0[u]);
+      if (c + 1 >= nc) break;
+      load(fa0, fb0, KU * (c + 2 < nc ? c + 2 : c));
+#pragma unroll
+      for (int u = 0; u < KU; ++u) step(fa1[u], fb1[u]);
+    }
+  }
+  // the remaining columns, four at a time (slots past k are zero)
+  for (int k0 = 4 * KU * nc; k0 < k; k0 += 4) {
+    const bool in = k0 + lk < k;
+    double ra[2], rb[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      ra[a] = in ? (A + (long)k0 * lda)[oa[a]] : 0.0;
+      rb[a] = in ? (B + (long)k0 * ldb)[ob[a]] : 0.0;
+    }
+    step(ra, rb);
+  }
+  const bool whole = i0 + 32 <= m && j0 + 32 <= n && (mode != 1 || i0 >= j0 + 31);
+  double* const Cl = C + (i0 + li) + (long)(j0 + lk) * ldc;
+  if (whole) {
+    double cv[2][2][4];
+    if (beta != 0.0) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) cv[a][b][r] = Cl[16 * a + (long)(16 * b + 4 * r) * ldc];
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const double v = alpha * acc[a][b][r];
+          Cl[16 * a + (long)(16 * b + 4 * r) * ldc] = beta == 0.0 ? v : v + beta * cv[a][b][r];
+        }
+    return;
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + 16 * a + li, j = j0 + 16 * b + lk + 4 * r;
+        if (i >= m || j >= n || (mode == 1 && i < j)) continue;
+        double* c = Cl + 16 * a + (long)(16 * b + 4 * r) * ldc;
+        const double v = alpha * acc[a][b][r];
+        *c = beta == 0.0 ? v : v + beta * (*c);
+      }
+}
+
+int launch_direct(hipStream_t s, int mode, int m, int n, int k, double alpha, const double* A,
+                  long lda, const double* B, long ldb, double beta, double* C, long ldc,
+                  const int* abort_flag) {
+  const int Tm = (m + 63) / 64, Tn = (n + 63) / 64;
+  const long nblk = (mode == 0) ? (long)Tm * Tn : (long)Tn * Tm - (long)Tn * (Tn - 1) / 2;
+  hipLaunchKernelGGL(dgemm_nt_direct_kernel<8>, dim3((unsigned)nblk), dim3(256), 0, s, mode, m, n,
+                     k, alpha, A, lda, B, ldb, beta, C, ldc, Tm, Tn, g_tile_group, abort_flag);
+  FLA_HIP_CHECK(hipGetLastError());
+  return FLA_HIP_OK;
+}
+
 // Tile configurations (selected by fla_hip_set_gemm_config for tuning):
 // <BM, BN, BK, waves in M, waves in N, fragment double-buffering>.
 int g_gemm_cfg = 0;
@@ -426,6 +553,16 @@ int launch_dgemm_mfma(hipStream_t s, bool ta, bool tb, int mode, int m, int n, i
                       double beta, double* C, long ldc, const int* abort_flag) {
   if (m <= 0 || n <= 0) return FLA_HIP_OK;
   if (mode == 1 && m < n) return FLA_HIP_EARG;  // lower mode expects a tall C
+  // At most one 128 x 128 tile per CU: 64 x 64 tiles without LDS, whose chain is
+  // a quarter as long (K = 128: 12 us a launch against 26-52).  FLA_Chol
+  // n = 1024 0.77 -> 0.63 ms, n = 5003 with its solve 5.4 -> 4.5 ms; a limit
+  // of 64, 600 or 1200 tiles gave 4.54, 4.60 and 4.68 ms on the latter.
+  if (g_gemm_cfg == 0 && !ta && tb && k > 0 && lda < (1L << 26) && ldb < (1L << 26)) {
+    const long Tm = (m + 127) / 128, Tn = (n + 127) / 128;
+    const long t128 = mode == 0 ? Tm * Tn : Tn * Tm - Tn * (Tn - 1) / 2;
+    if (t128 <= fla_ctx().num_cus)
+      return launch_direct(s, mode, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, abort_flag);
+  }
   // Default (0) and 12..15: the k-pair kernel wherever it applies (A and B
   // with the tile rows contiguous, full tiles, K a multiple of the chunk),
   // measured on MI355X at 54.9 TFLOP/s on the n = 32768 Cholesky update

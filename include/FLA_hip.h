@@ -264,12 +264,11 @@ int fla_hip_dsgesv(int n, int nrhs, double* A, int lda, int* p, const double* B,
    reduced-precision factorization's info. */
 int fla_hip_mp_last_stats(double* out, int nout);
 /* Panel solve of the reduced-precision factor: 0 backward-stable, 1 product
-   with the diagonal factors' inverses.  One panel solve serves both (inverse
-   product corrected to substitution's accuracy), so the choice has no effect
-   any more. */
+   with the diagonal factors' inverses.  One panel solve (blocked
+   substitution) serves both, so the choice has no effect any more. */
 int fla_hip_mp_set_panel(int inverse);
 /* CUs left out of the reduced-precision factor's update stream for its panel
-   chain (default 64; 0 = no mask). */
+   chain (default 32; 0 = no mask). */
 int fla_hip_mp_set_reserved_cus(int reserved);
 /* Outer block of the reduced-precision factor (multiple of 128; 0 = the
    FP64 Cholesky's choice for the order). */

@@ -52,51 +52,72 @@ __device__ __forceinline__ d4 mfma_block(d2 c0, d2 c1, d4 r, d4 acc) {
   acc = mfma_step(c1.x, r[2], acc);
   return mfma_step(c1.y, r[3], acc);
 }
-// X := T inv(L)' for a block T, given inv(L) (y) and -L (l): the product with
-// the explicit inverse, then one correction with its residual,
-// X += (T - X L') inv(L)', which brings the backward error of the inverse
-// (eps cond(L)) to that of substitution.  12 matrix steps against 136
-// dependent vector operations per row.
-__device__ __forceinline__ d4 solve_block(const d2 (&y)[2], const d2 (&l)[2], d4 t) {
-  const d4 zero = {0.0, 0.0, 0.0, 0.0};
-  const d4 x0 = mfma_block(y[0], y[1], t, zero);
-  const d4 r = mfma_block(l[0], l[1], x0, t);
-  return mfma_block(y[0], y[1], r, x0);
+// Lanes of row Q of 16 lanes, copied to all four rows (two swaps a word).
+template <int Q>
+__device__ __forceinline__ unsigned row_to_all(unsigned x) {
+  const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);  // {0,0,2,2}, {1,1,3,3}
+  const unsigned p = a[Q & 1];
+  const auto b = __builtin_amdgcn_permlane32_swap(p, p, false, false);  // {0,1,0,1}, {2,3,2,3}
+  return b[Q >> 1];
+}
+template <int Q>
+__device__ __forceinline__ double row_to_all(double x) {
+  return __hiloint2double((int)row_to_all<Q>((unsigned)__double2hiint(x)),
+                          (int)row_to_all<Q>((unsigned)__double2loint(x)));
+}
+
+// X := T inv(L)' for a block T by substitution, dtrsm_'s operations in its
+// order (x_j *= 1/l_jj, then t_c -= x_j l_cj).  The four columns 4r..4r+3 sit
+// in register r of the four rows of 16 lanes: within them the solved column
+// is copied across the rows, then one matrix step updates the later columns.
+// l: -L; cf[r]: of the lane's column c = lk + 4r the reciprocal 1/l_cc and
+// -l_cj for j = 4r..4r+2 (0 where c <= j).  About 1100 cycles; a matrix step
+// per column, whose result has to come back through the vector unit each
+// time, took 3200.
+__device__ __forceinline__ d4 solve_block(d4 l, const d4 (&cf)[4], d4 t, int li, int lk) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    double x = t[r];
+    x *= lk == 0 ? cf[r][0] : 1.0;
+    x = fma(cf[r][1], row_to_all<0>(x), x);
+    x *= lk == 1 ? cf[r][0] : 1.0;
+    x = fma(cf[r][2], row_to_all<1>(x), x);
+    x *= lk == 2 ? cf[r][0] : 1.0;
+    x = fma(cf[r][3], row_to_all<2>(x), x);
+    x *= lk == 3 ? cf[r][0] : 1.0;
+    t[r] = x;
+    if (r < 3) t = mfma_step(li >= 4 * (r + 1) ? l[r] : 0.0, x, t);
+  }
+  return t;
 }
 
 // The blocks of a factored 128 x 128 diagonal block L as the panel solve
 // reads them: for 16-column block jb the negated blocks left of the diagonal
-// -L(jb, 0..jb-1), then inv(L(jb, jb)), then -L(jb, jb).
+// -L(jb, 0..jb-1), then -L(jb, jb), then the coefficients cf[lk][r][4] of
+// solve_block (64 doubles).
 constexpr int frag_q0(int jb) { return jb * (jb - 1) / 2 + 2 * jb; }
 constexpr int NFRAG = frag_q0(NT16);
 static_assert(NFRAG * 256 <= PB * PB, "the fragments fit the 128 x 128 scratch block");
 
-// One wave factors a 16 x 16 symmetric block and inverts the factor.  Lane li
-// of each row of 16 lanes holds row li (x[c] = a(li, c), both triangles) and
-// column li of the identity (w): the sweep of Cholesky is also the forward
-// substitution of L Y = I, so w ends as column li of inv(L).  Column j's
-// multiplier of column c, a_jc, is broadcast from lane j's upper half by the
-// update instruction itself (DPP row_newbcast):
-//   x_c -= a_jc (x_j / a_jj),  w_c -= a_jc (w_j / d) / d,
-// two instructions per column.  (Through lane reads the pivot alone took 80
+// One wave factors a 16 x 16 symmetric block.  Lane li of each row of 16 lanes
+// holds row li (x[c] = a(li, c)).  Column j: d = sqrt(a_jj), x_j *= 1/d, then
+// x_c -= x_j l_cj, with l_cj broadcast from lane c by the update instruction
+// itself (DPP row_newbcast).  (Through lane reads the pivot alone took 80
 // cycles from its update to its first use, and every multiplier two reads.)
 // A VALU result is a DPP source only two wait states later: the statements
 // below keep other instructions in between, or carry the s_nop.
-template <int J, int C>
-__device__ __forceinline__ void sweep_update(double& w, double& x, double nw, double nx) {
-  asm volatile(
-      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
-      "v_fmac_f64_dpp %1, %1, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf"
-      : "+v"(w), "+v"(x)
-      : "v"(nw), "v"(nx), "i"(J));
+template <int C>
+__device__ __forceinline__ void sweep_update(double& x, double xs, double nx) {
+  asm volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+               : "+v"(x)
+               : "v"(xs), "v"(nx), "i"(C));
 }
-// Updates of column J for C0 <= C < C1 (none past 15).
-template <int J, int C0, int C1>
-__device__ __forceinline__ void sweep_updates(double (&x)[16], double (&w)[16], double nw,
-                                              double nx) {
+// Updates of the columns C0 <= C < C1 (none past 15).
+template <int C0, int C1>
+__device__ __forceinline__ void sweep_updates(double (&x)[16], double xs, double nx) {
   if constexpr (C0 < C1 && C0 < 16) {
-    sweep_update<J, C0>(w[C0], x[C0], nw, nx);
-    sweep_updates<J, C0 + 1, C1>(x, w, nw, nx);
+    sweep_update<C0>(x[C0], xs, nx);
+    sweep_updates<C0 + 1, C1>(x, xs, nx);
   }
 }
 template <int J>
@@ -108,93 +129,85 @@ __device__ __forceinline__ double bcast16(double x) {
   return a;
 }
 
-// Column J with the pivot a already broadcast.  Goldschmidt's iteration from
-// v_rsq_f64 gives g -> sqrt(a) and h -> 1/(2 sqrt(a)) with the common error
-// e = 1/2 - g h, which also corrects the reciprocal; the root takes two
-// residual corrections (Markstein).  The updates of column J - 1 right of
-// column J (multipliers nxp, nwp) fill the chain's latencies; column J + 1 is
-// updated first, so that the next pivot is on its way at the end.  piv: lane
-// J's root, checked once after the sweep.
+// Column J with the pivot a already broadcast.  The root by Goldschmidt's
+// iteration from v_rsq_f64 (g -> sqrt(a), h -> 1/(2 sqrt(a))) and a residual
+// correction, the reciprocal by a Newton step against the rounded root
+// (Markstein): exact roots and reciprocals come out exact, as the reference's
+// sqrt and division give them.  The updates of column J - 1 right of column J
+// (xsp, nxp) fill the chain's latencies; column J + 1 is updated first, so
+// that the next pivot is on its way at the end.  piv, pinv: lane J's root and
+// reciprocal.
 template <int J>
-__device__ __forceinline__ void sweep_column(double (&x)[16], double (&w)[16], int li, double& piv,
-                                             double& a, double& nxp, double& nwp) {
+__device__ __forceinline__ void sweep_column(double (&x)[16], int li, double& piv, double& pinv,
+                                             double& a, double& xsp, double& nxp) {
   constexpr int N = J > 0 ? 15 - J : 0, C1 = J + 1 + (N + 2) / 3, C2 = J + 1 + (2 * N + 2) / 3;
-  constexpr int JP = J > 0 ? J - 1 : 0;
   const double y = __builtin_amdgcn_rsq(a);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (J > 0) sweep_updates<JP, J + 1, C1>(x, w, nwp, nxp);
+  if constexpr (J > 0) sweep_updates<J + 1, C1>(x, xsp, nxp);
   __builtin_amdgcn_sched_barrier(0);
   double g = a * y, h = 0.5 * y;
   double e = fma(-h, g, 0.5);
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (J > 0) sweep_updates<JP, C1, C2>(x, w, nwp, nxp);
+  if constexpr (J > 0) sweep_updates<C1, C2>(x, xsp, nxp);
   __builtin_amdgcn_sched_barrier(0);
   h = fma(h, e, h);
   g = fma(g, e, g);
-  e = fma(-h, g, 0.5);
+  e = fma(-g, g, a);
   const double h2 = h + h;
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (J > 0) sweep_updates<JP, C2, 16>(x, w, nwp, nxp);
+  if constexpr (J > 0) sweep_updates<C2, 16>(x, xsp, nxp);
   __builtin_amdgcn_sched_barrier(0);
-  const double inv = fma(h2, e, h2);
-  const double xs = x[J] * inv, ws = w[J] * inv;
-  nxp = -(xs * inv);
-  nwp = -(ws * inv);
-  const double a0 = a;
+  const double d = fma(e, h, g);
+  const double inv = fma(fma(-d, h2, 1.0), h2, h2);
+  xsp = x[J] * inv;
+  nxp = -xsp;
+  asm volatile("s_nop 1" : "+v"(xsp));
   if constexpr (J < 15) {
-    sweep_update<J, J + 1>(w[J + 1], x[J + 1], nwp, nxp);
+    sweep_update<J + 1>(x[J + 1], xsp, nxp);
     a = bcast16<J + 1>(x[J + 1]);
   }
-  g = fma(fma(-g, g, a0), h, g);
-  const double d = fma(fma(-g, g, a0), h, g);
-  x[J] = li == J ? d : xs;
-  w[J] = ws;
+  x[J] = li == J ? d : xsp;
   piv = li == J ? d : piv;
+  pinv = li == J ? inv : pinv;
 }
 template <int... J>
-__device__ __forceinline__ void sweep16(double (&x)[16], double (&w)[16], int li, double& piv,
+__device__ __forceinline__ void sweep16(double (&x)[16], int li, double& piv, double& pinv,
                                         std::integer_sequence<int, J...>) {
-  double a = bcast16<0>(x[0]), nxp = 0.0, nwp = 0.0;
-  (sweep_column<J>(x, w, li, piv, a, nxp, nwp), ...);
+  double a = bcast16<0>(x[0]), xsp = 0.0, nxp = 0.0;
+  (sweep_column<J>(x, li, piv, pinv, a, xsp, nxp), ...);
 }
 
-// The same with the library's root and division, any pivot range; returns the
-// first column whose pivot is <= 0 or NaN (bl1_dsqrte's rule), else -1.
+// A factored 16 x 16 diagonal block in LDS: rows 0..15 hold L (below and on
+// the diagonal), row 16 the reciprocals of its diagonal.  The row length keeps
+// 16-byte accesses aligned and spreads the rows over the banks.
+constexpr int ZLD = 18;
+
+// The sweep with the library's root and division, any pivot range; returns
+// the first column whose pivot is <= 0 or NaN (bl1_dsqrte's rule), else -1.
 __device__ __noinline__ int sweep16_any(double* z, int lane) {
   const int li = lane & 15;
-  double x[16], w[16];
+  double x[16], pinv = 0.0;
 #pragma unroll
-  for (int c = 0; c < 16; ++c) {
-    x[c] = z[li * 18 + c];
-    w[c] = c == li ? 1.0 : 0.0;
-  }
+  for (int c = 0; c < 16; ++c) x[c] = z[li * ZLD + c];
   int f = -1;
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const double a = readlane_d(x[j], j);
     if (f < 0 && !(a > 0.0)) f = j;
     const double d = sqrt(a), inv = 1.0 / d;
-    const double xs = x[j] * inv, ws = w[j] * inv;
+    const double xs = x[j] * inv;
 #pragma unroll
-    for (int c = j + 1; c < 16; ++c) {
-      const double l = readlane_d(x[c], j) * inv;
-      w[c] = fma(-ws, l, w[c]);
-      x[c] = fma(-xs, l, x[c]);
-    }
+    for (int c = j + 1; c < 16; ++c) x[c] = fma(-xs, readlane_d(xs, c), x[c]);
     x[j] = li == j ? d : xs;
-    w[j] = ws;
+    pinv = li == j ? inv : pinv;
   }
-  if (lane < 32) {
+  if (lane < 16) {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) z[lane * 18 + q] = lane < 16 ? x[q] : w[q];
+    for (int q = 0; q < 16; ++q) z[lane * ZLD + q] = x[q];
+    z[16 * ZLD + lane] = pinv;
   }
   return f;
 }
-
-// A factored 16 x 16 diagonal block in LDS: rows 0..15 hold L (below and on
-// the diagonal), row 16 + c column c of inv(L).  The row length keeps 16-byte
-// accesses aligned and spreads the rows over the banks.
-constexpr int ZLD = 18;
 
 // Factors the symmetric block dg (fragment order) into z, one wave.  Returns
 // the first failing column or -1.  Pivots outside [2^-700, 2^1000] (products
@@ -205,27 +218,20 @@ __device__ __forceinline__ int factor16(d4 dg, double* z, int lane) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) z[li * ZLD + lk + 4 * r] = dg[r];
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  double x[16], w[16], piv = 0.0;
+  double x[16], piv = 0.0, pinv = 0.0;
 #pragma unroll
   for (int q = 0; q < 8; ++q) {
     const d2 v = *reinterpret_cast<const d2*>(z + li * ZLD + 2 * q);
     x[2 * q] = v.x;
     x[2 * q + 1] = v.y;
-    w[2 * q] = 2 * q == li ? 1.0 : 0.0;
-    w[2 * q + 1] = 2 * q + 1 == li ? 1.0 : 0.0;
   }
-  // every x is written two wait states before the first broadcast reads it
-  asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]),
-               "+v"(x[6]), "+v"(x[7]));
-  asm volatile("s_nop 1" : "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]),
-               "+v"(x[13]), "+v"(x[14]), "+v"(x[15]));
-  sweep16(x, w, li, piv, std::make_integer_sequence<int, 16>{});
+  sweep16(x, li, piv, pinv, std::make_integer_sequence<int, 16>{});
   if (!__all(piv >= 0x1p-350 && piv <= 0x1p500)) return sweep16_any(z, lane);
-  if (lane < 32) {
+  if (lane < 16) {
 #pragma unroll
     for (int q = 0; q < 8; ++q)
-      *reinterpret_cast<d2*>(z + lane * ZLD + 2 * q) =
-          lane < 16 ? d2{x[2 * q], x[2 * q + 1]} : d2{w[2 * q], w[2 * q + 1]};
+      *reinterpret_cast<d2*>(z + lane * ZLD + 2 * q) = d2{x[2 * q], x[2 * q + 1]};
+    z[16 * ZLD + lane] = pinv;
   }
   return -1;
 }
@@ -239,8 +245,8 @@ __device__ __forceinline__ int factor16(d4 dg, double* z, int lane) {
 // factors its diagonal block (factor16) while the others apply the previous
 // step's update to their remaining blocks.
 // Bound: the serial chain of 128 pivots (broadcast, root, reciprocal, scale,
-// update: about 240 cycles each) plus 20 matrix steps (about 2000 cycles with
-// their operands' LDS reads) per 16 columns.  128 columns take 28 us alone, 73
+// update: about 200 cycles each) plus a block substitution and its updates
+// (about 3000 cycles) per 16 columns.  128 columns take 26 us alone, 73
 // with the block in LDS, lane reads for the multipliers and three barriers
 // per 32 columns.
 // W receives the blocks of L for the panel solve (see frag_q0).  A failed
@@ -250,7 +256,7 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
                                                         d2* __restrict__ W) {
   if (*info >= 0) return;
   __shared__ d2 Xf[2][NT16][2][64];  // the solved blocks (negated) of a block column, by parity
-  __shared__ __attribute__((aligned(16))) double Z[2][32 * ZLD];
+  __shared__ __attribute__((aligned(16))) double Z[2][17 * ZLD];
   __shared__ int fail;
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -284,17 +290,21 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
     const int flim = fail;
     if (w > b && flim < 0) {
       __builtin_amdgcn_s_setprio(2);
-      d2 y[2], l[2];
+      d4 l, cf[4];
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const int k = lk + 4 * s;
-        y[s >> 1][s & 1] = z[(16 + k) * ZLD + li];
-        const double v = z[li * ZLD + k];
-        l[s >> 1][s & 1] = k <= li ? -v : 0.0;
+        const int cc = lk + 4 * s;
+        l[s] = -z[li * ZLD + cc];  // above the diagonal never used
+        cf[s][0] = z[16 * ZLD + cc];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          const double v = z[cc * ZLD + 4 * s + q];
+          cf[s][1 + q] = lk > q ? -v : 0.0;
+        }
       }
       d4 cur = c[0];
       if (b > 0) cur = mfma_block(Xf[par ^ 1][b][0][lane], Xf[par ^ 1][b][1][lane], xr, cur);
-      const d4 xn = solve_block(y, l, cur);
+      const d4 xn = solve_block(l, cf, cur, li, lk);
       const d2 n0 = d2{-xn[0], -xn[1]}, n1 = d2{-xn[2], -xn[3]};
       Xf[par][w][0][lane] = n0;
       Xf[par][w][1][lane] = n1;
@@ -322,7 +332,7 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
         for (int r = 0; r < 4; ++r) A[(long)row + (long)(16 * b + lk + 4 * r) * lda] = xn[r];
       }
     } else if (w == b) {
-      // the diagonal block: L to A (up to a failing column), inv(L) and -L to W
+      // the diagonal block: L to A (up to a failing column), -L and cf to W
       const int jend = flim < 0 ? 16 : flim - 16 * b;
       d2* const Wq = W + (frag_q0(b) + b) * 128;
 #pragma unroll
@@ -331,9 +341,11 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
         const double v0 = z[li * ZLD + k0], v1 = z[li * ZLD + k1];
         if (k0 <= li && row < nb && k0 < jend) A[(long)row + (long)(16 * b + k0) * lda] = v0;
         if (k1 <= li && row < nb && k1 < jend) A[(long)row + (long)(16 * b + k1) * lda] = v1;
-        Wq[64 * p + lane] = d2{z[(16 + k0) * ZLD + li], z[(16 + k1) * ZLD + li]};
-        Wq[128 + 64 * p + lane] = d2{k0 <= li ? -v0 : 0.0, k1 <= li ? -v1 : 0.0};
+        Wq[64 * p + lane] = d2{k0 <= li ? -v0 : 0.0, k1 <= li ? -v1 : 0.0};
       }
+      const int cc = lk + (lane & 12), q = (lane & 3) - 1;  // cf[lk][(lane / 4) % 4][lane % 4]
+      const double v = q < 0 ? z[16 * ZLD + cc] : -z[cc * ZLD + (lane & 12) + (q < 0 ? 0 : q)];
+      reinterpret_cast<double*>(Wq + 128)[lane] = lk > q ? v : 0.0;
     }
     if (flim >= 0) break;
   }
@@ -372,6 +384,19 @@ __global__ void set_int_kernel(int* p, int v) { *p = v; }
 
 }  // namespace
 
+// The panel solve's order of L's blocks: row jb's, left to right (the
+// coefficients after each diagonal block are read separately).
+constexpr int NQ = NT16 * (NT16 + 1) / 2;
+struct Stream {
+  int block[NQ];
+};
+constexpr Stream make_stream() {
+  Stream s{};
+  for (int jb = 0, q = 0; jb < NT16; ++jb)
+    for (int k = 0; k <= jb; ++k, ++q) s.block[q] = frag_q0(jb) + k;
+  return s;
+}
+
 // A21 := A21 inv(L11)' for an m x 128 strip, L11 given by the blocks that
 // potrf_blk_kernel left in W.  Each wave owns 16 rows, all 128 columns in
 // registers in fragment order; per 16-column block the contributions of the
@@ -379,13 +404,14 @@ __global__ void set_int_kernel(int* p, int v) { *p = v; }
 // from memory (88 KB, shared by every wave through the caches) PF blocks
 // ahead of their use; no LDS, so the workgroups fit beside the update
 // kernel's.  (32 rows per wave, with half the reads of L, spilled registers.)
-// Bound: one wave's chain of 208 matrix steps (5.8 us) while the rows fit the
-// chip once.  n = 5003: 11.5 us a launch on average against 87 for one thread
-// per row with substitution.
+// Bound: one wave's chain (112 matrix steps and eight block substitutions)
+// while the rows fit the chip once.  n = 5003: about 12 us a launch on average against 87 for one
+// thread per row.
 __global__ __launch_bounds__(256, 2) void trsm_rlt_kernel(int m, const d2* __restrict__ W,
                                                           double* __restrict__ X, long ldx,
                                                           const int* __restrict__ abort) {
   constexpr int PF = 6;
+  constexpr Stream kStream = make_stream();
   if (abort && *abort >= 0) return;
   const int lane = threadIdx.x & 63;
   const int li = lane & 15, lk = lane >> 4;
@@ -395,36 +421,44 @@ __global__ __launch_bounds__(256, 2) void trsm_rlt_kernel(int m, const d2* __res
   double* const xp = X + (in ? row0 + li : m - 1) + (long)lk * ldx;
   d4 c[NT16];
   d2 ring[PF][2];
+  d4 cf[4];
   const d2* const Wl = W + lane;
+  auto coefs = [&](int jb) {
+    const d2* const p = W + (frag_q0(jb) + jb + 1) * 128 + lk * 8;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const d2 u = p[2 * r], v = p[2 * r + 1];
+      cf[r] = d4{u.x, u.y, v.x, v.y};
+    }
+  };
 #pragma unroll
   for (int q = 0; q < PF; ++q) {
-    ring[q][0] = Wl[q * 128];
-    ring[q][1] = Wl[q * 128 + 64];
+    ring[q][0] = Wl[kStream.block[q] * 128];
+    ring[q][1] = Wl[kStream.block[q] * 128 + 64];
   }
 #pragma unroll
   for (int k = 0; k < NT16; ++k)
 #pragma unroll
     for (int r = 0; r < 4; ++r) c[k][r] = xp[(long)(16 * k + 4 * r) * ldx];
+  coefs(0);
 #pragma unroll
   for (int jb = 0; jb < NT16; ++jb) {
 #pragma unroll
-    for (int k = 0; k < jb; ++k) {
-      const int q = frag_q0(jb) + k;
-      c[jb] = mfma_block(ring[q % PF][0], ring[q % PF][1], c[k], c[jb]);
-      if (q + PF < NFRAG) {
-        ring[q % PF][0] = Wl[(q + PF) * 128];
-        ring[q % PF][1] = Wl[(q + PF) * 128 + 64];
+    for (int k = 0; k < NT16; ++k) {
+      if (k > jb) break;
+      const int q = jb * (jb + 1) / 2 + k;
+      const d2 l0 = ring[q % PF][0], l1 = ring[q % PF][1];
+      if (k < jb)
+        c[jb] = mfma_block(l0, l1, c[k], c[jb]);
+      else
+        c[jb] = solve_block(d4{l0.x, l0.y, l1.x, l1.y}, cf, c[jb], li, lk);
+      if (q + PF < NQ) {
+        ring[q % PF][0] = Wl[kStream.block[q + PF] * 128];
+        ring[q % PF][1] = Wl[kStream.block[q + PF] * 128 + 64];
       }
+      if (k == jb && jb + 1 < NT16) coefs(jb + 1);
       __builtin_amdgcn_sched_barrier(0);
     }
-    const int q = frag_q0(jb) + jb;
-    c[jb] = solve_block(ring[q % PF], ring[(q + 1) % PF], c[jb]);
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-      if (q + u + PF < NFRAG) {
-        ring[(q + u) % PF][0] = Wl[(q + u + PF) * 128];
-        ring[(q + u) % PF][1] = Wl[(q + u + PF) * 128 + 64];
-      }
     if (in) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) xp[(long)(16 * jb + 4 * r) * ldx] = c[jb][r];

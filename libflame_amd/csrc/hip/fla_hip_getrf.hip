@@ -12,50 +12,53 @@
 // scaling are skipped, the update uses the unchanged row j, and the sweep
 // continues.
 //
-// Panel: one cooperative kernel.  The (m-k) x nb panel is spread over P
-// workgroups (256 rows each) and held in VGPRs for the whole panel; every
-// column costs one all-to-all exchange: each workgroup publishes its local
-// pivot candidates (value, row, original row) and their rows, the owner of
-// the diagonal row publishes that row, and every workgroup reads all
-// candidates, picks the same pivot, and reads the two rows it needs.
-// The exchange words live in uncached device memory (no L2 write-back or
-// invalidate across the XCDs) and carry their own tags, so no store needs
-// to be acknowledged before another one and no separate flag is polled:
-// each 8-byte word holds a 32-bit payload and the 32-bit tag of the
+// Panel: 128 columns as sub-panels of 32.  A sub-panel is one kernel that
+// keeps its rows in VGPRs (a thread owns whole rows), 1024 rows a workgroup;
+// up to 1024 rows there is nothing to exchange.  With more rows each column
+// costs one all-to-all exchange: every workgroup publishes its pivot
+// candidate together with the candidate's row, reads all of them, and picks
+// the same pivot.  The exchange words live in uncached device memory (no L2
+// write-back or invalidate across the XCDs) and carry their own tags, so no
+// store needs to be acknowledged before another one and no separate flag is
+// polled: each 8-byte word holds a 32-bit payload and the 32-bit tag of the
 // (launch, column) it belongs to, and a reader takes a word only once its
-// tag is current.  Every wait is bounded.
+// tag is current.  Every wait is bounded.  Between sub-panels one kernel
+// applies the interchanges to the panel's other columns and solves for U12,
+// and a product updates the columns to the right.
 #include <hip/hip_runtime.h>
+
+#include <utility>
 
 #include "fla_hip_internal.h"
 
 namespace {
 
-constexpr int PW = 128;           // maximum panel width
-constexpr int ROWS_PER_WG = 256;  // rows of the panel held by one workgroup
-constexpr int NT = 512;  // 8 waves: wave w owns columns [32(w>>1), +32) of row half w&1
+constexpr int PW = 128;  // maximum panel width
+constexpr int SW = 32;   // sub-panel width
+constexpr int NT = 512;  // threads of a sub-panel workgroup
 constexpr int RQ = 2;    // rows per thread
+constexpr int ROWS_PER_WG = NT * RQ;
 constexpr unsigned long long kSpinTicks = 200000000ULL;  // 2 s of the 100 MHz wall clock
-constexpr int MAX_P = 256;  // panel workgroups (one per CU at most)
-constexpr int HW = 8;       // header entries per workgroup slot (one 128-byte line)
+constexpr int MAX_P = 64;  // sub-panel workgroups
+constexpr int SLOT = 40;   // exchange entries of a slot: 32 values, 3 header entries, padding
 
 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(1))) u64x2 g_u64x2;
 typedef __attribute__((address_space(1))) unsigned long long g_u64;
 
-// Exchange area (tagged 16-byte entries, two parities: column j uses j & 1).
-//   hdr [2][P][HW]: {best |v| over non-NaN rows >= j}, {its row, its orig},
-//                   {last NaN row, its orig}, {best |v| over non-NaN rows
-//                   after the last NaN}, {its row, its orig}   (row -1: none),
-//                   {orig of row j} (workgroup 0), two pad entries
-//   rows[2][P][3][PW]: the best, the last-NaN and the after-NaN row
-//   jrow[2][PW]: the diagonal row's values
-// Every store covers whole 128-byte lines (a wave's lanes write consecutive
-// entries): a partial-line write to uncached memory is a read-modify-write.
+// Exchange area (tagged 16-byte entries, two parities: column j uses j & 1):
+// slots [2][P + 1][SLOT], slot w < P from workgroup w, slot P (the diagonal
+// row j) from workgroup 0.  Entries 0..31: the row's values; 32: {candidate
+// |v|}; 33: {its row, its original row}; 34: {the workgroup's last NaN row or
+// -1}.  The candidate is the first maximum after the last NaN, or the last
+// NaN itself with |v| = -1 when nothing follows it.  A slot is five whole
+// 128-byte lines, stored by one instruction: a partial-line write to uncached
+// memory is a read-modify-write.
 struct PanelComm {
-  u64x2* hdr;
-  u64x2* rows;
-  u64x2* jrow;
-  int* err;  // wait-limit flag
+  u64x2* slots;
+  int* err;       // wait-limit flag
+  int* orig[2];   // original row (in the panel) of every row, before / after a sub-panel
+  int* submoved;  // the current sub-panel's row moves
 };
 
 // Stores need no ordering among themselves (each word carries its tag): a
@@ -66,10 +69,6 @@ __device__ __forceinline__ void put(u64x2* p, unsigned lo, unsigned hi, unsigned
   w.x = (unsigned long long)lo | ((unsigned long long)tag << 32);
   w.y = (unsigned long long)hi | ((unsigned long long)tag << 32);
   *(g_u64x2*)p = w;
-}
-__device__ __forceinline__ void put_d(u64x2* p, double d, unsigned tag) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(d);
-  put(p, (unsigned)b, (unsigned)(b >> 32), tag);
 }
 __device__ __forceinline__ u64x2 get(const u64x2* p) {
   g_u64* q = (g_u64*)p;
@@ -133,431 +132,496 @@ __device__ __forceinline__ int wave_min_i(int x) {
   return __builtin_amdgcn_readlane(x, 63);
 }
 
-// First maximum over the wave of key[i] (the lane's rows lane + 64 i, i =
-// 0..3, so smaller i and then smaller lane means the smaller row); keys below
-// zero take no part.  Returns the local row, or -1, and the maximum.
-__device__ __forceinline__ int first_max(const double (&key)[4], double& best) {
-  const double m = wave_max_d(fmax(fmax(key[0], key[1]), fmax(key[2], key[3])));
-  best = m;
-  if (m < 0.0) return -1;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const unsigned long long b = __ballot(key[i] == m);
-    if (b) return 64 * i + __builtin_ctzll(b);
-  }
-  return -1;
+// Barrier that orders LDS accesses only (the exchange stores stay in flight).
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-__global__ __launch_bounds__(NT) void lu_panel_kernel(int M, int W, double* __restrict__ A,
-                                                      long lda, int k, int* __restrict__ piv,
-                                                      int* __restrict__ info,
-                                                      int* __restrict__ moved, PanelComm cm,
-                                                      unsigned tagbase) {
-  // A wait that expired in an earlier panel of this factorization aborts all later ones.
-  if (__hip_atomic_load(cm.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
-  const int P = gridDim.x;
-  const int wg = blockIdx.x;
-  const int t = threadIdx.x;
-  const int lane = t & 63;
-  const int wave = t >> 6;
-  const int cg = wave >> 1;  // column group (its two waves sit on different SIMDs)
-  const int rh = wave & 1;   // row half
-  const int base = wg * ROWS_PER_WG;
+// a += lane (C & 15) of u (in each row of 16 lanes) times b: one instruction
+// per element of the rank-1 update, with the pivot row spread over the lanes.
+template <int C>
+__device__ __forceinline__ void fmac_bcast(double& a, double u, double b) {
+  asm volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+               : "+v"(a)
+               : "v"(u), "v"(b), "i"(C & 15));
+}
+// The thread rows are held as four chunks of eight columns, rotated so that
+// the current column is position I of chunk 0; finished chunks are at the end.
+// Position I becomes the multiplier l, the positions right of it (in the
+// nlive unfinished chunks) take the rank-1 update, x the next position's value.
+template <int I, int... C>
+__device__ __forceinline__ void update_tail(double (&v)[SW], double u0, double nl,
+                                            std::integer_sequence<int, C...>) {
+  (fmac_bcast<I + 1 + C>(v[I + 1 + C], u0, nl), ...);
+}
+template <int I>
+__device__ __forceinline__ void update_first(double (&v)[SW], double u0, double l, double nl,
+                                             double& x) {
+  v[I] = l;
+  update_tail<I>(v, u0, nl, std::make_integer_sequence<int, 7 - I>{});
+  if constexpr (I < 7) x = v[I + 1];
+}
+template <int CH, int... I>
+__device__ __forceinline__ void update_chunk(double (&v)[SW], double u, double nl,
+                                             std::integer_sequence<int, I...>) {
+  (fmac_bcast<8 * CH + I>(v[8 * CH + I], u, nl), ...);
+}
 
-  __shared__ double colbuf[2][ROWS_PER_WG];  // column j of every row, before its interchange
-  __shared__ int origs[ROWS_PER_WG];         // original row of each local row
-  __shared__ double prow[PW];                // pivot row values
-  __shared__ double jrow[PW];                // old diagonal row values
-  __shared__ int sel[4];                     // pivot row, its orig, orig of the old row j
-  // The panel's pivots and its first null pivot, written to global memory
-  // after the column loop: a global store inside the loop would hold the
-  // storing wave at the next column's wait for outstanding memory operations
-  // until the store is acknowledged, and every workgroup waits on workgroup 0.
-  __shared__ int pivs[PW];
-  __shared__ int first_null;
-  __shared__ double stage[NT / 64][32];      // a row's 32 columns, per wave, to store coalesced
-
-  if (wg == 0 && t == 0) {
-    // The move list is appended to only after every workgroup has read this
-    // workgroup's first header, which is stored after this reset completes.
-    __hip_atomic_store(&moved[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __builtin_amdgcn_s_waitcnt(0);
-    first_null = -1;
+// Copies the row of lane cl (register row cq, uniform) to dst in LDS.
+__device__ __forceinline__ void stage_row(double* dst, const double (&v)[RQ][SW], int cq, int lane,
+                                          int cl) {
+  if (lane != cl) return;
+  if (cq == 0) {
+#pragma unroll
+    for (int c = 0; c < SW; ++c) dst[c] = v[0][c];
+  } else {
+#pragma unroll
+    for (int c = 0; c < SW; ++c) dst[c] = v[1][c];
   }
+}
 
-  // Thread owns local rows rh*128 + 64*q + lane (q = 0..1), columns 32*cg + c.
-  double v[RQ][32];
+__device__ __forceinline__ unsigned wave_max_u(unsigned x) {
+  x = max(x, (unsigned)dpp_i<0x111, 0xf>((int)x));
+  x = max(x, (unsigned)dpp_i<0x112, 0xf>((int)x));
+  x = max(x, (unsigned)dpp_i<0x114, 0xf>((int)x));
+  x = max(x, (unsigned)dpp_i<0x118, 0xf>((int)x));
+  x = max(x, (unsigned)dpp_i<0x142, 0xa>((int)x));
+  x = max(x, (unsigned)dpp_i<0x143, 0xc>((int)x));
+  return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
+}
+// Maximum over lanes 0..7.
+__device__ __forceinline__ double max8_d(double x) {
+  x = fmax(x, dpp_d<0x111, 0xf>(x));
+  x = fmax(x, dpp_d<0x112, 0xf>(x));
+  x = fmax(x, dpp_d<0x114, 0xf>(x));
+  return readlane_d(x, 7);
+}
+
+// The wave's first maximum of the keys (>= 0, or -1 for none) in row order
+// (register row, then lane).  The high words (plus one; 0: none) decide it
+// unless two of the largest agree in them.
+__device__ __forceinline__ void wave_first_max(const double (&key)[RQ], int& cq, int& cl) {
+  unsigned h[RQ];
+#pragma unroll
+  for (int q = 0; q < RQ; ++q)
+    h[q] = key[q] >= 0.0 ? (unsigned)__double2hiint(key[q]) + 1u : 0u;
+  const unsigned m = wave_max_u(max(h[0], h[1]));
+  unsigned long long b0 = __ballot(h[0] == m), b1 = __ballot(h[1] == m);
+  if (__builtin_popcountll(b0) + __builtin_popcountll(b1) > 1) {
+    const double d = wave_max_d(fmax(key[0], key[1]));
+    b0 = __ballot(key[0] == d);
+    b1 = __ballot(key[1] == d);
+  }
+  cq = b0 ? 0 : 1;
+  cl = __builtin_ctzll(b0 ? b0 : b1);
+}
+
+struct SubHead {
+  double val;  // the wave's largest |a|, -1: none
+  int row;     // its row in the sub-panel
+  int nan;     // the wave's last NaN row, -1: none
+};
+
+// LU with partial pivoting of the M x W sub-panel at A (W <= 32), column k of
+// the matrix first.  piv: its pivots; cm.submoved: its row moves; cm.orig:
+// the panel's row origins before (first == 0: the identity) and after;
+// pmoved, when given: the whole panel's row moves.  `first`: the sub-panel's
+// first row in the panel.
+// Per column: every wave's candidate to LDS, a barrier, every wave picks the
+// workgroup's; the candidate's owner copies its row to LDS and (one
+// workgroup) a barrier makes it visible, or (more) publishes it, all waves
+// poll the workgroups' slots into LDS, a barrier, and every wave picks the
+// pivot.  Only the winner's row is copied: a single lane's 16-byte LDS writes
+// cost as much as a full wave's, and all eight waves doing so took 1500
+// cycles.  The column loop is not unrolled (450 KB of code, every column
+// fetched from L2 once, 2-5 us a column); only the update's first chunk
+// depends on the column's position at compile time.
+// Bound: the chain of LDS, cross-lane and scalar steps of the search per
+// column, and with more workgroups the exchange's memory round trip.  32
+// columns take 79 us with one workgroup and 130-155 with 2-16 (n = 16384: 141
+// on average); a 128-column panel as one kernel with a second round trip for
+// the pivot row took 620 us at any height.
+__global__ __launch_bounds__(NT, 2) void lu_sub_kernel(int M, int W, double* __restrict__ A,
+                                                       long lda, int k, int* __restrict__ piv,
+                                                       int* __restrict__ info, PanelComm cm,
+                                                       int flip, int first,
+                                                       int* __restrict__ pmoved,
+                                                       unsigned tagbase) {
+  // A wait that expired in an earlier launch of this factorization aborts all later ones.
+  if (__hip_atomic_load(cm.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
+  constexpr int NW = NT / 64;
+  __shared__ __attribute__((aligned(16))) double crow[2][SW];  // the candidate's row, by parity
+  __shared__ __attribute__((aligned(16))) double jrow[2][SW];  // row j before the interchange
+  __shared__ __attribute__((aligned(16))) double gx[MAX_P + 1][SW];  // the exchanged rows
+  __shared__ SubHead head[2][NW];
+  __shared__ double gval[MAX_P + 1];
+  __shared__ int corg[2], jorg[2];
+  __shared__ int grow[MAX_P + 1], gorg[MAX_P + 1], gnan[MAX_P + 1], dead, pivs[SW], first_null;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int base = blockIdx.x * ROWS_PER_WG, P = gridDim.x;
+  if (t == 0) {
+    dead = 0;
+    first_null = -1;
+    if (base == 0) {
+      // The move lists are appended to only after every workgroup has read
+      // this workgroup's first slot, which is stored after this reset
+      // completes.
+      __hip_atomic_store(&cm.submoved[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (pmoved) __hip_atomic_store(&pmoved[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __builtin_amdgcn_s_waitcnt(0);
+    }
+  }
+  double v[RQ][SW], x[RQ];  // x: the current column
+  int og[RQ];               // original row
 #pragma unroll
   for (int q = 0; q < RQ; ++q) {
-    const int r = base + rh * 128 + 64 * q + lane;
+    const int r = base + q * NT + t;
+    og[q] = r;
+    const double* const a = A + (r < M ? r : M - 1);
+    if (W == SW) {
 #pragma unroll
-    for (int c = 0; c < 32; ++c) {
-      const int col = 32 * cg + c;
-      v[q][c] = (r < M && col < W) ? A[(long)r + (long)col * lda] : 0.0;
+      for (int c = 0; c < SW; ++c) v[q][c] = a[(long)c * lda];
+    } else {
+#pragma unroll
+      for (int c = 0; c < SW; ++c) {
+        const double y = a[(long)(c < W ? c : 0) * lda];
+        v[q][c] = c < W ? y : 0.0;
+      }
     }
-    if (cg == 0) {
-      colbuf[0][rh * 128 + 64 * q + lane] = v[q][0];
-      origs[rh * 128 + 64 * q + lane] = r;
-    }
+    x[q] = v[q][0];
   }
-  // All panel loads complete here, so that inside the column loop no use of
-  // the panel registers waits on memory counters (which also count the
-  // exchange stores in flight).
-  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
 
-  for (int j = 0; j < W; ++j) {
-    const int par = j & 1;
-    const int cgj = j >> 5, cj = j & 31;
-    const unsigned tag = tagbase | (unsigned)(j + 1);
-    __syncthreads();  // column j and the row origins are in LDS
-
-    // ---- local candidates, found by every wave from the LDS copy ----
-    double key[4];
-    unsigned long long nanb[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int lr = lane + 64 * i;
-      const int r = base + lr;
-      const double x = colbuf[par][lr];
-      const bool act = r >= j && r < M;
-      key[i] = (act && x == x) ? fabs(x) : -1.0;
-      nanb[i] = __ballot(act && x != x);
-    }
-    double bv, av = -1.0;
-    const int lb = first_max(key, bv);
-    int ln = -1;
-#pragma unroll
-    for (int i = 3; i >= 0; --i)
-      if (ln < 0 && nanb[i]) ln = 64 * i + 63 - __builtin_clzll(nanb[i]);
-    int la = -1;
-    if (ln >= 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (lane + 64 * i <= ln) key[i] = -1.0;
-      la = first_max(key, av);
-    }
-
-    // ---- publish: the header (wave 0), each candidate row (its owners) ----
-    u64x2* myrows = cm.rows + ((long)par * P + wg) * 3 * PW;
-    u64x2* js = cm.jrow + (long)par * PW;
-    if (wave == 0 && lane < HW) {
-      u64x2* h = cm.hdr + ((long)par * P + wg) * HW;
-      const int br = lb >= 0 ? base + lb : -1, bo = lb >= 0 ? origs[lb] : -1;
-      const int nr = ln >= 0 ? base + ln : -1, no = ln >= 0 ? origs[ln] : -1;
-      const int ar = la >= 0 ? base + la : -1, ao = la >= 0 ? origs[la] : -1;
-      const int jo = (wg == 0) ? origs[j] : -1;
-      const double d = lane == 0 ? bv : av;
-      const unsigned long long db = (unsigned long long)__double_as_longlong(d);
-      unsigned lo = 0, hi = 0;
-      if (lane == 0 || lane == 3) {
-        lo = (unsigned)db;
-        hi = (unsigned)(db >> 32);
-      } else if (lane == 1) {
-        lo = (unsigned)br;
-        hi = (unsigned)bo;
-      } else if (lane == 2) {
-        lo = (unsigned)nr;
-        hi = (unsigned)no;
-      } else if (lane == 4) {
-        lo = (unsigned)ar;
-        hi = (unsigned)ao;
-      } else if (lane == 5) {
-        lo = (unsigned)jo;
-      }
-      put(h + lane, lo, hi, tag);
-    }
-    {
-      // rows lb, ln, la of this workgroup, and row j in workgroup 0: the
-      // owner lane stages its 32 columns, then 32 lanes store them
-      const int jl = (wg == 0) ? j : -1;
-      const int want[4] = {lb, ln, la, jl};
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int lr = want[s];
-        if (lr < 0 || (lr >> 7) != rh) continue;  // uniform
-        u64x2* dst = (s < 3) ? myrows + s * PW : js;
-        if (lane == (lr & 63)) {
-          if (((lr >> 6) & 1) == 0) {
-#pragma unroll
-            for (int c = 0; c < 32; ++c) stage[wave][c] = v[0][c];
-          } else {
-#pragma unroll
-            for (int c = 0; c < 32; ++c) stage[wave][c] = v[1][c];
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (lane < 32 && 32 * cg + lane < W) put_d(&dst[32 * cg + lane], stage[wave][lane], tag);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      }
-    }
-
-    // ---- wave 0: read every header, pick the pivot, read its row and row j ----
-    if (wave == 0) {
-      bool ok = true;
-      const unsigned long long t0 = wall_clock64();
-      auto expired = [&]() {
-        if (__hip_atomic_load(cm.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
-            wall_clock64() - t0 > kSpinTicks) {
-          if (lane == 0) __hip_atomic_store(cm.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          return true;
-        }
-        return false;
-      };
-      const u64x2* hb = cm.hdr + (long)par * P * HW;
-      // pass 1: best of every slab, and the last NaN row overall
-      double gv = 0.0;
-      int grow = -1, go = -1, gw = -1, gslot = 0, gnr = -1, gno = -1, jo = 0;
-      for (int w0 = 0; ok && w0 < P; w0 += 64) {
-        const int w = w0 + lane;
-        u64x2 e0, e1, e2, e3, e4, e5;
-        while (true) {
-          bool done = true;
-          if (w < P) {
-            const u64x2* h = hb + (long)w * HW;
-            e0 = get(h);
-            e1 = get(h + 1);
-            e2 = get(h + 2);
-            e3 = get(h + 3);
-            e4 = get(h + 4);
-            e5 = get(h + 5);
-            done = tagged(e0, tag) && tagged(e1, tag) && tagged(e2, tag) && tagged(e3, tag) &&
-                   tagged(e4, tag) && tagged(e5, tag);
-          }
-          if (__all(done)) break;
-          if (expired()) {
-            ok = false;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-        }
-        if (ok && w == 0) jo = lo_i(e5);
-        if (ok && w < P) {
-          // a lane visits its slabs in row order: keep the first maximum
-          const double cv = as_d(e0);
-          const int cr = lo_i(e1), co = hi_i(e1), hn = lo_i(e2), hno = hi_i(e2);
-          if (hn > gnr) {
-            gnr = hn;
-            gno = hno;
-          }
-          if (cr >= 0 && (grow < 0 || cv > gv)) {
-            gv = cv;
-            grow = cr;
-            go = co;
-            gw = w;
-          }
-        }
-      }
-      if (ok) {
-        const unsigned long long nan_lanes = __ballot(gnr >= 0);
-        if (nan_lanes == 0) {
-          // first maximum over the lanes: the wave's maximum, then the
-          // smallest row among the lanes that hold it
-          const double m = wave_max_d(grow >= 0 ? gv : -1.0);
-          const unsigned long long b = __ballot(grow >= 0 && gv == m);
-          int L = b ? __builtin_ctzll(b) : 0;
-          if (__builtin_popcountll(b) > 1) {
-            const bool in = (b >> lane) & 1ull;
-            const int mr = wave_min_i(in ? grow : 0x7fffffff);
-            L = __builtin_ctzll(__ballot(in && grow == mr));
-          }
-          grow = __builtin_amdgcn_readlane(grow, L);
-          go = __builtin_amdgcn_readlane(go, L);
-          gw = __builtin_amdgcn_readlane(gw, L);
-        } else {
-          // the last NaN row overall, and its orig from the lane holding it
-          const int m = wave_max_i(gnr);
-          gno = __builtin_amdgcn_readlane(gno, __builtin_ctzll(__ballot(gnr == m)));
-          gnr = m;
-          // With the last NaN at row gnr (idamax restarts after it): the
-          // after-NaN candidate of the slab holding gnr plus the best of
-          // every slab wholly below it.  All headers are current by now.
-          gv = 0.0;
-          grow = go = gw = -1;
-          for (int w = lane; w < P; w += 64) {
-            const u64x2* h = hb + (long)w * HW;
-            double cv = 0.0;
-            int cr = -1, co = -1, cs = 0;
-            if (lo_i(get(h + 2)) == gnr) {
-              const u64x2 e3 = get(h + 3), e4 = get(h + 4);
-              cv = as_d(e3);
-              cr = lo_i(e4);
-              co = hi_i(e4);
-              cs = 2;
-            } else if ((long)w * ROWS_PER_WG > (long)gnr) {
-              const u64x2 e0 = get(h), e1 = get(h + 1);
-              cv = as_d(e0);
-              cr = lo_i(e1);
-              co = hi_i(e1);
-            }
-            if (cr >= 0 && (grow < 0 || cv > gv || (cv == gv && cr < grow))) {
-              gv = cv;
-              grow = cr;
-              go = co;
-              gw = w;
-              gslot = cs;
-            }
-          }
-#pragma unroll
-          for (int off = 32; off > 0; off >>= 1) {
-            const double ov = __shfl_xor(gv, off);
-            const int orow = __shfl_xor(grow, off), oo = __shfl_xor(go, off),
-                      ow = __shfl_xor(gw, off), os = __shfl_xor(gslot, off);
-            if (orow >= 0 && (grow < 0 || ov > gv || (ov == gv && orow < grow))) {
-              gv = ov;
-              grow = orow;
-              go = oo;
-              gw = ow;
-              gslot = os;
-            }
-          }
-        }
-        if (grow < 0 && gnr >= 0) {  // nothing after the last NaN: it is the pivot
-          grow = gnr;
-          go = gno;
-          gw = gnr / ROWS_PER_WG;
-          gslot = 1;
-        }
-        if (gw < 0) gw = 0;  // unreachable: row j itself takes part (W <= M)
-        // the winning row and the old diagonal row
-        const u64x2* src = cm.rows + (((long)par * P + gw) * 3 + gslot) * PW;
-        while (true) {
-          bool done = true;
-          for (int e = lane; e < W; e += 64) {
-            const u64x2 a = get(&src[e]), b = get(&js[e]);
-            if (tagged(a, tag) && tagged(b, tag)) {
-              prow[e] = as_d(a);
-              jrow[e] = as_d(b);
-            } else {
-              done = false;
-            }
-          }
-          if (__all(done)) break;
-          if (expired()) {
-            ok = false;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-        }
-        if (lane == 0) {
-          sel[0] = grow;
-          sel[1] = go;
-          sel[2] = jo;
-        }
-      }
-      if (!ok && lane == 0) sel[0] = -2;
-    }
-    __syncthreads();
-    if (sel[0] == -2) return;
-    const int r = sel[0];
-    const double piv_val = prow[j];
-    const bool null_pivot = (piv_val == 0.0);
-    const bool swap = !null_pivot && r != j;
-    if (wg == 0 && t == 0) {
-      pivs[j] = r - j;
-      if (null_pivot && first_null < 0) first_null = j;
-    }
-    // ---- interchange rows j and r (skipped for a null pivot) ----
-    if (swap) {
+#pragma unroll 1
+  for (int j = 0; j < SW; ++j) {
+    const int pos = j & 7, nlive = 4 - (j >> 3);
+    if (j < W) {
+      const int par = j & 1;
+      // ---- this wave's candidate ----
+      double key[RQ];
+      int nanrow = -1;
 #pragma unroll
       for (int q = 0; q < RQ; ++q) {
-        const int rr = base + rh * 128 + 64 * q + lane;
-        if (!__any(rr == j || rr == r)) continue;  // this wave holds neither row
-        if (rr == j) {
+        const int r = base + q * NT + t;
+        const bool act = r >= j && r < M;
+        key[q] = (act && x[q] == x[q]) ? fabs(x[q]) : -1.0;
+        const unsigned long long nb = __ballot(act && x[q] != x[q]);
+        if (nb) nanrow = base + q * NT + 64 * wave + 63 - __builtin_clzll(nb);
+      }
+      int cq, cl;
+      wave_first_max(key, cq, cl);
+      if (lane == cl)
+        head[par][wave] = SubHead{cq ? key[1] : key[0], base + cq * NT + t, nanrow};
+      lds_barrier();
+      // ---- the workgroup's candidate lrow, |a| = lval ----
+      SubHead hd = head[par][lane & (NW - 1)];
+      int lnan = -1;
+      if (__ballot(hd.nan >= 0)) {  // a NaN: the search restarts after the last one (rare)
+        lnan = wave_max_i(hd.nan);
+        lds_barrier();
 #pragma unroll
-          for (int c = 0; c < 32; ++c) v[q][c] = prow[32 * cg + c];
-        } else if (rr == r) {
+        for (int q = 0; q < RQ; ++q)
+          if (base + q * NT + t <= lnan) key[q] = -1.0;
+        wave_first_max(key, cq, cl);
+        if (lane == cl)
+          head[par][wave] = SubHead{cq ? key[1] : key[0], base + cq * NT + t, nanrow};
+        lds_barrier();
+        hd = head[par][lane & (NW - 1)];
+      }
+      const double lval = max8_d(hd.val);
+      int lrow;
+      {
+        const unsigned long long b = __ballot(hd.val == lval && lane < NW);
+        if (!(lval >= 0.0))
+          lrow = lnan;  // nothing but the NaN
+        else if ((b & (b - 1)) == 0)
+          lrow = __builtin_amdgcn_readlane(hd.row, __builtin_ctzll(b));
+        else  // equal maxima: the smallest row
+          lrow = wave_min_i((b >> lane) & 1ull ? hd.row : 0x7fffffff);
+      }
+      // ---- its row (and row j) to LDS ----
+      const int lt = (lrow - base) & (NT - 1);
+      const bool own = wave == (lt >> 6), ownj = base == 0 && wave == 0;
+      if (own) {
+        const int q = (lrow - base) / NT;
+        stage_row(crow[par], v, q, lane, lt & 63);
+        if (lane == (lt & 63)) corg[par] = q ? og[1] : og[0];
+      }
+      if (ownj) {
+        stage_row(jrow[par], v, 0, lane, j);
+        if (lane == j) jorg[par] = og[0];
+      }
+      const double* prow = crow[par];
+      const double* jr = jrow[par];
+      const int *orgs = corg + par, *orgj = jorg + par;
+      int r = lrow;
+      if (P == 1) {
+        lds_barrier();
+      } else {
+        // ---- all-to-all exchange ----
+        const unsigned tag = tagbase | (unsigned)(j + 1);
+        u64x2* const area = cm.slots + (long)par * (MAX_P + 1) * SLOT;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        auto publish = [&](const double* row, int slot, int gr, int go) {
+          unsigned lo = 0, hi = 0;
+          if (lane <= SW) {
+            const double d = lane < SW ? row[lane & (SW - 1)] : lval;
+            const unsigned long long b = (unsigned long long)__double_as_longlong(d);
+            lo = (unsigned)b;
+            hi = (unsigned)(b >> 32);
+          } else if (lane == SW + 1) {
+            lo = (unsigned)gr;
+            hi = (unsigned)go;
+          } else if (lane == SW + 2) {
+            lo = (unsigned)lnan;
+          }
+          if (lane < SLOT) put(area + (long)slot * SLOT + lane, lo, hi, tag);
+        };
+        if (own) publish(prow, base / ROWS_PER_WG, lrow, corg[par]);
+        if (ownj) publish(jr, P, j, jorg[par]);
+        constexpr int U = 3;  // slots polled together
+        for (int s0 = wave; s0 <= P; s0 += U * NW) {
+          u64x2 e[U];
+          unsigned long long t0 = 0;
+          for (unsigned spin = 1;; ++spin) {
+            bool done = true;
 #pragma unroll
-          for (int c = 0; c < 32; ++c) v[q][c] = jrow[32 * cg + c];
+            for (int u = 0; u < U; ++u)
+              if (s0 + u * NW <= P && lane < SW + 3)
+                e[u] = get(area + (long)(s0 + u * NW) * SLOT + lane);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (s0 + u * NW <= P && lane < SW + 3) done = done && tagged(e[u], tag);
+            if (__all(done)) break;
+            // the flag and the clock cost as much as a poll: every 64th
+            if (spin & 63) continue;
+            if (t0 == 0) t0 = wall_clock64();
+            if (__hip_atomic_load(cm.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
+                wall_clock64() - t0 > kSpinTicks) {
+              if (lane == 0) {
+                __hip_atomic_store(cm.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                dead = 1;
+              }
+              break;
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int s = s0 + u * NW;
+            if (s > P) continue;
+            if (lane < SW) gx[s][lane] = as_d(e[u]);
+            if (lane == SW) gval[s] = as_d(e[u]);
+            if (lane == SW + 1) {
+              grow[s] = lo_i(e[u]);
+              gorg[s] = hi_i(e[u]);
+            }
+            if (lane == SW + 2) gnan[s] = lo_i(e[u]);
+          }
         }
+        lds_barrier();
+        if (dead) return;
+        const int sl = lane < P ? lane : 0;
+        const double gv = lane < P ? gval[sl] : -1.0;
+        const int gr = grow[sl], gn = gnan[sl];
+        const unsigned long long nb = __ballot(lane < P && gn >= 0);
+        const int lo = nb ? 63 - __builtin_clzll(nb) : 0;  // the slab of the last NaN
+        // the first of the largest, by the high word unless two agree in it
+        const double kk = lane >= lo ? gv : -1.0;
+        const unsigned h = kk >= 0.0 ? (unsigned)__double2hiint(kk) + 1u : 0u;
+        const unsigned mh = wave_max_u(h);
+        unsigned long long b = __ballot(h == mh);
+        if (b & (b - 1)) b = __ballot(kk == wave_max_d(kk));
+        const int gw = mh ? __builtin_ctzll(b) : lo;
+        prow = gx[gw];
+        jr = gx[P];
+        r = __builtin_amdgcn_readlane(gr, gw);
+        orgs = gorg + gw;
+        orgj = gorg + P;
       }
-      if (t == 0) {
-        if (j >= base && j < base + ROWS_PER_WG) origs[j - base] = sel[1];
-        if (r >= base && r < base + ROWS_PER_WG) origs[r - base] = sel[2];
+      const double piv_val = prow[pos];
+      const bool null_pivot = piv_val == 0.0;
+      const bool swap = !null_pivot && r != j;
+      if (base == 0 && t == 0) {
+        pivs[j] = r - j;
+        if (null_pivot && first_null < 0) first_null = j;
       }
-    }
-    // ---- multipliers (column j scaled by the reciprocal, skipped for a null
-    // pivot or a pivot of 1, as bl1_dinvscalv), then the rank-1 update with
-    // the diagonal row (the old row j when there was no interchange) ----
-    const bool scale = !null_pivot && piv_val != 1.0;
-    const double inv = scale ? 1.0 / piv_val : 1.0;
-    const double* u = swap ? prow : jrow;
-    const int jn = j + 1;
-    if (cg >= cgj) {
-      double l[RQ], xn[RQ] = {0.0, 0.0};
-      bool act[RQ];
-#pragma unroll
-      for (int q = 0; q < RQ; ++q) {
-        const int lr = rh * 128 + 64 * q + lane;
-        const int rr = base + lr;
-        act[q] = rr > j && rr < M;
-        double x = colbuf[par][lr];
-        if (swap && rr == r) x = jrow[j];
-        l[q] = scale ? x * inv : x;
-      }
-      // 8-column chunks [c0, c0 + 8): wholly right of j without selects; the
-      // chunk holding j (only in the waves owning it) with them.  The chunk's
-      // pivot-row values are read once for both rows of the thread.
-#pragma unroll
-      for (int cc = 0; cc < 4; ++cc) {
-        const int c0 = 32 * cg + 8 * cc;
-        if (c0 + 7 < j) continue;  // uniform
-        double uu[8];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) uu[c] = u[c0 + c];
+      // the pivot row (row j when nothing moves) spread over each row of 16 lanes
+      const double* const u = swap ? prow : jr;
+      double u0 = u[lane & 15], u1 = u[16 + (lane & 15)];
+      // ---- interchange rows j and r (skipped for a null pivot) ----
+      if (swap) {
 #pragma unroll
         for (int q = 0; q < RQ; ++q) {
-          double* a = &v[q][8 * cc];
-          if (c0 > j) {
-            if (act[q]) {
+          const int rr = base + q * NT + t;
+          if (!__any(rr == j || rr == r)) continue;
+          const double* const w = rr == j ? prow : jr;
+          if (rr == j || rr == r) {
 #pragma unroll
-              for (int c = 0; c < 8; ++c) a[c] = fma(-l[q], uu[c], a[c]);
-            }
-          } else if (act[q]) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-              const double y = fma(-l[q], uu[c], a[c]);
-              a[c] = (c0 + c > j) ? y : ((c0 + c == j) ? l[q] : a[c]);
-            }
-          }
-          if (jn < W && c0 <= jn && jn < c0 + 8) {  // uniform: the next column's chunk
-#pragma unroll
-            for (int c = 0; c < 8; ++c) xn[q] = (c0 + c == jn) ? a[c] : xn[q];
+            for (int c = 0; c < SW; ++c) v[q][c] = w[c];
+            og[q] = rr == j ? *orgs : *orgj;
+            x[q] = w[pos];
           }
         }
       }
-      if (jn < W && cg == (jn >> 5)) {
+      // ---- multipliers (scaled by the reciprocal, skipped for a null pivot
+      // or a pivot of 1, as bl1_dinvscalv) and the rank-1 update ----
+      const bool scale = !null_pivot && piv_val != 1.0;
+      const double inv = scale ? 1.0 / piv_val : 1.0;
+      double l[RQ], nl[RQ];
 #pragma unroll
-        for (int q = 0; q < RQ; ++q) colbuf[par ^ 1][rh * 128 + 64 * q + lane] = xn[q];
+      for (int q = 0; q < RQ; ++q) {
+        l[q] = scale ? x[q] * inv : x[q];
+        nl[q] = -l[q];
+      }
+      // The finished rows 0..j are lanes of the first wave's first register
+      // row: they keep their values by a zero multiplier or, should the pivot
+      // row hold an infinity or NaN, by selects.
+      bool select = false;
+      if (ownj) {
+        select = !__all(fabs(u0) < __builtin_inf() && fabs(u1) < __builtin_inf());
+        nl[0] = lane > j ? nl[0] : 0.0;
+        l[0] = lane > j ? l[0] : x[0];
+      }
+      if (select) {
+#pragma unroll
+        for (int c = 0; c < SW; ++c) {
+          const double y = fma(-l[0], u[c], v[0][c]);
+          if (c > pos && c < 8 * nlive && lane > j) v[0][c] = y;
+          if (c == pos + 1) x[0] = v[0][c];
+        }
+        nl[0] = 0.0;
+        u0 = fabs(u0) < __builtin_inf() ? u0 : 0.0;
+        u1 = fabs(u1) < __builtin_inf() ? u1 : 0.0;
+      }
+      // (rows past M take garbage here and are never stored or searched)
+      // a VALU result is a DPP source only two wait states later
+      asm volatile("s_nop 1" : "+v"(u0), "+v"(u1));
+#define FLA_LU_POS(I)                                 \
+  case I:                                             \
+    update_first<I>(v[0], u0, l[0], nl[0], x[0]);     \
+    update_first<I>(v[1], u0, l[1], nl[1], x[1]);     \
+    break;
+      switch (pos) {
+        FLA_LU_POS(0)
+        FLA_LU_POS(1)
+        FLA_LU_POS(2)
+        FLA_LU_POS(3)
+        FLA_LU_POS(4)
+        FLA_LU_POS(5)
+        FLA_LU_POS(6)
+        FLA_LU_POS(7)
+      }
+#undef FLA_LU_POS
+      constexpr auto seq = std::make_integer_sequence<int, 8>{};
+      if (nlive > 1) {
+        update_chunk<1>(v[0], u0, nl[0], seq);
+        update_chunk<1>(v[1], u0, nl[1], seq);
+      }
+      if (nlive > 2) {
+        update_chunk<2>(v[0], u1, nl[0], seq);
+        update_chunk<2>(v[1], u1, nl[1], seq);
+      }
+      if (nlive > 3) {
+        update_chunk<3>(v[0], u1, nl[0], seq);
+        update_chunk<3>(v[1], u1, nl[1], seq);
+      }
+    }
+    if (pos == 7) {  // the finished chunk goes to the end
+#pragma unroll
+      for (int q = 0; q < RQ; ++q) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const double f = v[q][c];
+          v[q][c] = v[q][c + 8];
+          v[q][c + 8] = v[q][c + 16];
+          v[q][c + 16] = v[q][c + 24];
+          v[q][c + 24] = f;
+        }
+        x[q] = v[q][0];
       }
     }
   }
   __syncthreads();
-
-  if (wg == 0) {
-    for (int jj = t; jj < W; jj += NT) piv[k + jj] = pivs[jj];
+  if (base == 0) {
+    for (int j = t; j < W; j += NT) piv[k + j] = pivs[j];
     if (t == 0 && first_null >= 0) atomicCAS(info, -1, k + first_null);
   }
-  // ---- write back; record rows whose content moved ----
+  asm volatile("" : "+s"(lda));  // the column offsets are not kept through the loop
+  const int* const before = cm.orig[flip];
+  int* const after = cm.orig[flip ^ 1];
+  auto note = [](int* list, int dst, int src) {
+    const int slot = atomicAdd(&list[0], 1);
+    list[1 + 2 * slot] = dst;
+    list[2 + 2 * slot] = src;
+  };
+  if (pmoved && base == 0 && t < first) {
+    // rows finished by an earlier sub-panel keep the origin that it wrote
+    const int po = cm.orig[((t / SW) & 1) ^ 1][t];
+    if (po != t) note(pmoved, t, po);
+  }
 #pragma unroll
   for (int q = 0; q < RQ; ++q) {
-    const int lr = rh * 128 + 64 * q + lane;
-    const int r = base + lr;
-    if (r < M) {
+    const int r = base + q * NT + t;
+    if (r >= M) continue;
+    double* const a = A + r;
+    if (W == SW) {
 #pragma unroll
-      for (int c = 0; c < 32; ++c) {
-        const int col = 32 * cg + c;
-        if (col < W) A[(long)r + (long)col * lda] = v[q][c];
-      }
-      if (cg == 0 && origs[lr] != r) {
-        const int slot = atomicAdd(&moved[0], 1);
-        moved[1 + 2 * slot] = r;
-        moved[2 + 2 * slot] = origs[lr];
-      }
+      for (int c = 0; c < SW; ++c) a[(long)c * lda] = v[q][c];
+    } else {
+#pragma unroll
+      for (int c = 0; c < SW; ++c)
+        if (c < W) a[(long)c * lda] = v[q][c];
     }
+    if (og[q] != r) note(cm.submoved, r, og[q]);
+    const int pr = first + r, po = first == 0 ? og[q] : before[first + og[q]];
+    after[pr] = po;
+    if (pmoved && po != pr) note(pmoved, pr, po);
+  }
+}
+
+// After a sub-panel of w columns at row and column c0 of the panel: its row
+// moves (at most 64, one per lane) on the panel's columns [0, c0) and
+// [c0 + w, c0 + w + nright), and on the latter U12 := inv(L11) A12 (unit
+// lower), also written transposed to Ut.  One wave per column; lane i holds
+// row i of the solve.
+__global__ __launch_bounds__(256) void lu_sub_apply_kernel(int c0, int w, int nright,
+                                                           double* __restrict__ A, long lda,
+                                                           const int* __restrict__ moved,
+                                                           double* __restrict__ Ut, long ldu) {
+  __shared__ double top[4][SW];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ci = blockIdx.x * 4 + wave;
+  if (ci >= c0 + nright) return;
+  const bool right = ci >= c0;
+  double* const rows = A + c0;  // row c0 of the panel
+  double* const col = rows + (long)(right ? ci + w : ci) * lda;
+  const int i = lane & (SW - 1);
+  double l[SW], a = 0.0;
+  if (right) {
+    a = i < w ? col[i] : 0.0;
+#pragma unroll
+    for (int k = 0; k < SW - 1; ++k) l[k] = (k < i && i < w) ? rows[i + (long)(c0 + k) * lda] : 0.0;
+    top[wave][i] = a;
+  }
+  const int cnt = moved[0];
+  const bool mv = lane < cnt;
+  const int dst = mv ? moved[1 + 2 * lane] : 0, src = mv ? moved[2 + 2 * lane] : 0;
+  const double x = mv ? col[src] : 0.0;
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // every lane has read its row
+  if (mv && (!right || dst >= w)) col[dst] = x;
+  if (!right) return;
+  if (mv && dst < w) top[wave][dst] = x;
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  a = top[wave][i];
+#pragma unroll
+  for (int k = 0; k < SW - 1; ++k) {
+    const double y = fma(-l[k], readlane_d(a, k), a);
+    a = i > k ? y : a;
+  }
+  if (lane < w) {
+    col[lane] = a;
+    Ut[(ci - c0) + (long)lane * ldu] = a;
   }
 }
 
@@ -624,21 +688,23 @@ struct LuBufs {
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-constexpr size_t kHdrBytes = sizeof(u64x2) * 2 * MAX_P * HW;
-constexpr size_t kRowsBytes = sizeof(u64x2) * 2 * MAX_P * 3 * PW;
-constexpr size_t kJrowBytes = sizeof(u64x2) * 2 * PW;
+constexpr int MAX_ROWS = MAX_P * ROWS_PER_WG;
+constexpr size_t kSlotBytes = sizeof(u64x2) * 2 * (MAX_P + 1) * SLOT;
+constexpr size_t kOrigBytes = sizeof(int) * MAX_ROWS;
 constexpr size_t kMovedBytes = sizeof(int) * (1 + 4 * PW);
-static_assert(kHdrBytes + kRowsBytes + kJrowBytes + 256 * 8 + 4 * kMovedBytes < kUcLuBytes,
+static_assert(kSlotBytes + 2 * kOrigBytes + 16 * 256 + 5 * kMovedBytes < kUcLuBytes,
               "LU exchange area");
 
 static void lu_carve(char* p, LuBufs (&b)[4]) {
   PanelComm cm;
-  cm.hdr = reinterpret_cast<u64x2*>(p);
-  p += align256(kHdrBytes);
-  cm.rows = reinterpret_cast<u64x2*>(p);
-  p += align256(kRowsBytes);
-  cm.jrow = reinterpret_cast<u64x2*>(p);
-  p += align256(kJrowBytes);
+  cm.slots = reinterpret_cast<u64x2*>(p);
+  p += align256(kSlotBytes);
+  for (int s = 0; s < 2; ++s) {
+    cm.orig[s] = reinterpret_cast<int*>(p);
+    p += align256(kOrigBytes);
+  }
+  cm.submoved = reinterpret_cast<int*>(p);
+  p += align256(kMovedBytes);
   cm.err = nullptr;  // set by the caller
   for (int s = 0; s < 4; ++s) {
     b[s].cm = cm;
@@ -659,23 +725,36 @@ static unsigned g_lu_epoch = 0;
 
 static int lu_panel(hipStream_t s, int M, int W, double* Ap, long lda, int k, int* piv,
                     int* dinfo, const LuBufs& b) {
-  const int P = (M + ROWS_PER_WG - 1) / ROWS_PER_WG;
-  g_lu_epoch = (g_lu_epoch + 1) & 0xffffffu;
-  if (g_lu_epoch == 0) {
-    const long words = (long)(reinterpret_cast<char*>(b.cm.jrow) + kJrowBytes -
-                              reinterpret_cast<char*>(b.cm.hdr)) / 8;
-    hipLaunchKernelGGL(zero_kernel, dim3(256), dim3(256), 0, s,
-                       reinterpret_cast<unsigned long long*>(b.cm.hdr), words);
-    FLA_HIP_CHECK(hipGetLastError());
-    g_lu_epoch = 1;
-  }
+  double* const Ut = fla_ctx().dlinv;  // transposed U12 of a sub-panel, at most 96 x 32
   void* tok = fla_stats_begin(s);
-  hipLaunchKernelGGL(lu_panel_kernel, dim3(P), dim3(NT), 0, s, M, W, Ap, lda, k, piv, dinfo,
-                     b.moved, b.cm, g_lu_epoch << 8);
+  for (int c0 = 0, sub = 0; c0 < W; c0 += SW, ++sub) {
+    const int w = (W - c0) < SW ? (W - c0) : SW;
+    const int m = M - c0, nright = W - c0 - w;
+    double* As = Ap + (long)c0 + (long)c0 * lda;
+    g_lu_epoch = (g_lu_epoch + 1) & 0xffffffu;
+    if (g_lu_epoch == 0) {
+      hipLaunchKernelGGL(zero_kernel, dim3(256), dim3(256), 0, s,
+                         reinterpret_cast<unsigned long long*>(b.cm.slots),
+                         (long)(kSlotBytes / 8));
+      FLA_HIP_CHECK(hipGetLastError());
+      g_lu_epoch = 1;
+    }
+    hipLaunchKernelGGL(lu_sub_kernel, dim3((m + ROWS_PER_WG - 1) / ROWS_PER_WG), dim3(NT), 0, s, m,
+                       w, As, lda, k + c0, piv, dinfo, b.cm, sub & 1, c0,
+                       nright == 0 ? b.moved : nullptr, g_lu_epoch << 8);
+    FLA_HIP_CHECK(hipGetLastError());
+    if (c0 + nright > 0) {
+      hipLaunchKernelGGL(lu_sub_apply_kernel, dim3((c0 + nright + 3) / 4), dim3(256), 0, s, c0, w,
+                         nright, Ap, lda, b.cm.submoved, Ut, (long)PW);
+      FLA_HIP_CHECK(hipGetLastError());
+    }
+    if (nright > 0 && m > w)
+      FLA_TRY(launch_dgemm_mfma(s, false, true, 0, m - w, nright, w, -1.0, As + w, lda, Ut, PW, 1.0,
+                                As + (long)w + (long)w * lda, lda, nullptr));
+  }
   double fl = 0.0;
   for (int j = 0; j < W; ++j) fl += (double)(M - j - 1) * (1.0 + 2.0 * (W - j - 1));
   fla_stats_end(s, tok, 2, fl);
-  FLA_HIP_CHECK(hipGetLastError());
   return FLA_HIP_OK;
 }
 
@@ -799,7 +878,7 @@ static int lu_update_cols2(hipStream_t s, int m, double* A, long lda, int k, int
 // stream carries the chain: panel A; B's columns updated with A; panel B; B's
 // interchanges on A's columns; the next pair's 256 columns updated with the
 // pair (K = 256), after which the next panel A starts.  The bulk stream
-// (s_update_lp: its CU mask leaves 64 CUs to the panel kernel) updates every
+// (s_update_lp: its CU mask leaves 32 CUs to the panel kernel) updates every
 // column beyond the next pair (K = 256) and applies the pair's
 // interchanges left of it, concurrently with the next pair's two panels; the
 // chain waits for it only before the following pair's columns.  Ut holds the
@@ -883,8 +962,7 @@ extern "C" int fla_hip_dgetrf(int m, int n, double* A, int lda, int* p, int* inf
   const int Pmax = (m + ROWS_PER_WG - 1) / ROWS_PER_WG;
   // Every panel workgroup must be resident at once (one per CU at most).
   if (Pmax > c.num_cus || Pmax > MAX_P) {
-    std::fprintf(stderr, "libflame_amd: dgetrf supports m <= %d on this device\n",
-                 c.num_cus * ROWS_PER_WG);
+    std::fprintf(stderr, "libflame_amd: dgetrf supports m <= %d on this device\n", MAX_ROWS);
     return FLA_HIP_EARG;
   }
   // exchange area in the uncached region, laid out for MAX_P workgroups
@@ -925,7 +1003,7 @@ int fla_lu_panel_setup(int m, int* derr) {
   const int Pmax = (m + ROWS_PER_WG - 1) / ROWS_PER_WG;
   if (Pmax > c.num_cus || Pmax > MAX_P) {
     std::fprintf(stderr, "libflame_amd: the LU panel supports m <= %d on this device\n",
-                 c.num_cus * ROWS_PER_WG);
+                 MAX_ROWS);
     return FLA_HIP_EARG;
   }
   lu_carve(c.uc, g_mp_bufs);

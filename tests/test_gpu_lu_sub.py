@@ -1,0 +1,53 @@
+"""The LU sub-panel kernel where it can go wrong: heights around the 512
+threads and the 1024 rows of a workgroup, ragged last sub-panels, and NaN or
+infinite entries in workgroups other than the pivot's."""
+import numpy as np
+import pytest
+
+import libflame_amd as fla
+from tests.cases import exact_lu
+from tests.gpu_util import gpu_lu
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    fla.FLA_Init()
+    yield
+
+
+@pytest.mark.parametrize("m,n", [(33, 33), (63, 40), (511, 70), (513, 33), (1023, 65), (1024, 32),
+                                 (1025, 97), (2049, 160), (1100, 129)])
+def test_sub_panel_exact(m, n):
+    A, L, U, p = exact_lu(n, seed=m + n, m=m)
+    out, pv, r = gpu_lu(A)
+    assert r == fla.FLA_SUCCESS
+    assert np.array_equal(pv, p)
+    assert np.array_equal(np.tril(out[:, :n], -1), np.tril(L, -1))
+    assert np.array_equal(np.triu(out[:n, :]), U)
+
+
+@pytest.mark.parametrize("rows", [[7], [600], [1500], [40, 2100], [2199]])
+def test_nan_restart_across_workgroups(orc, rows):
+    A = np.asfortranarray(orc.gen_lu_c2(3, 2200, 40))
+    for r in rows:
+        A[r, 0] = np.nan
+    _, pv, _ = gpu_lu(A)
+    _, pref, _ = orc.lu_piv(A)
+    assert pv[0] == pref[0]
+
+
+@pytest.mark.parametrize("m", [100, 1500])
+def test_infinite_row_keeps_finished_rows(orc, m):
+    """An infinity right of the first columns reaches the rows below its pivot
+    row only: finished rows of U and the columns left of it stay finite."""
+    n, c = 32, 9
+    A = np.asfortranarray(orc.gen_lu_c2(5, m, n))
+    A[0, c] = np.inf
+    out, pv, _ = gpu_lu(A)
+    ref, pref, _ = orc.lu_piv(A)
+    assert np.array_equal(pv[:c], pref[:c])
+    assert np.array_equal(np.isfinite(out[:, :c]), np.isfinite(ref[:, :c]))
+    k = next(i for i in range(n) if not np.isfinite(ref[i, c]))
+    assert np.all(np.isfinite(out[:k, :]))

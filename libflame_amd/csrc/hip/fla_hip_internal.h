@@ -34,7 +34,7 @@ struct FlaHipCtx {
   hipStream_t s_panel = nullptr;   // panel factorizations (look-ahead)
   // Trailing updates of the reduced-precision factor: their panel chain, not
   // the update, is the critical path, so this stream leaves more CUs free.
-  // 64 CUs left to the panels: the reduced-precision factor's updates and the
+  // 32 CUs left to the panels: the reduced-precision factor's updates and the
   // LU's bulk updates beside its panel chain
   hipStream_t s_update_lp = nullptr;
   static constexpr int kEvents = 8;

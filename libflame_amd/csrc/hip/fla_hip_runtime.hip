@@ -4,7 +4,7 @@
 // The reference binds one rocBLAS handle per SuperMatrix thread and device
 // (FLASH_Queue_bind_hip, src/base/flamec/supermatrix/hip/main/FLASH_Queue_hip.c:297-318);
 // here one process drives one GPU through three streams: s_update for trailing
-// updates, s_panel for the look-ahead panel chain, and s_update_lp (64 CUs
+// updates, s_panel for the look-ahead panel chain, and s_update_lp (32 CUs
 // left to the panels) for the reduced-precision factor's updates and the
 // LU's bulk updates.
 #include <cstdlib>
@@ -23,16 +23,17 @@ FlaHipCtx& fla_ctx() { return g_ctx; }
 // single-workgroup panel kernel that needs a whole CU's LDS would otherwise
 // wait for a CU to drain completely.
 static int g_reserved_cus = 8;
-// The second update stream leaves 64 CUs to the panels.  It carries the
-// reduced-precision factor's updates (measured on MI355X at n = 16384) and
-// the LU's bulk updates, whose panel kernel needs up to 64 whole CUs with all
-// its workgroups resident (with 8 left, LU panels waited for CUs: 119 ms
-// instead of 87 ms per factorization at n = 16384).  One stream serves both
-// so that the library's three streams, with the null stream, fit the four
-// hardware queues HIP gives a process: two busy streams sharing a queue
-// serialize (an LU with its bulk stream on the panel's queue took 182 ms
-// instead of 134 ms).
-static int g_lp_reserved_cus = 64;
+// The second update stream leaves 32 CUs (four of each XCD) to the panels.
+// It carries the reduced-precision factor's updates and the LU's bulk
+// updates, whose panel kernel needs one whole CU per 1024 rows with all its
+// workgroups resident.  Measured at n = 16384 with 64, 48, 32, 24, 16 and 8
+// CUs left: FLA_LU_piv 120.0, 120.9, 116.6, 124.3, 126.2, 127.4 ms; the mixed
+// solve 32.0, 32.0, 30.5, 31.1, 31.7, 32.0 ms (n = 8000-8192: within 1 %).
+// One stream serves both so that the library's three streams, with the null
+// stream, fit the four hardware queues HIP gives a process: two busy streams
+// sharing a queue serialize (an LU with its bulk stream on the panel's queue
+// took 182 ms instead of 134 ms).
+static int g_lp_reserved_cus = 32;
 
 static int create_masked_stream(hipStream_t* s, int reserved) {
   if (reserved <= 0 || reserved >= g_ctx.num_cus) {

@@ -199,62 +199,6 @@ __global__ __launch_bounds__(256) void trsm_subst_lds_kernel(int nrhs, int nb,
   }
 }
 
-// Diagonal-block solve of the blocked dtrsm, by substitution with the block
-// staged in LDS and one lane per right-hand side:
-//   left side:  M = op(T_kk), the right-hand sides are the columns of B_k;
-//   right side: M = op(T_kk)', the right-hand sides are the rows of B_k
-//               (x op(T) = b  <=>  op(T)' x' = b').
-// M(i, c) = flip ? T(c, i) : T(i, c).  M lower: forward in dtrsm_'s column
-// order (x_c := x_c / M_cc, then x_i -= x_c M_ic for i > c); M upper:
-// backward.  Left-side solves divide by the diagonal and right-side solves
-// multiply by its reciprocal, as dtrsm_ does (src/flablas/f2c/dtrsm.c).
-template <bool MLOWER, bool ROWS>
-__global__ __launch_bounds__(256) void trsm_diag_subst_kernel(int nrhs, int nb,
-                                                              const double* __restrict__ T,
-                                                              long ldt, int flip, int unit,
-                                                              double* __restrict__ B, long ldb) {
-  __shared__ double Ms[TB * TB];  // Ms[c * TB + i] = M(i, c) on the strict triangle, else 0
-  __shared__ double dg[TB];       // M(c, c); 1 for a unit diagonal and beyond nb
-  for (int e = threadIdx.x; e < TB * TB; e += 256) {
-    const int i = e % TB, c = e / TB;
-    const bool in = MLOWER ? (i > c) : (i < c);
-    double v = 0.0;
-    if (in && i < nb && c < nb) v = flip ? T[(long)c + (long)i * ldt] : T[(long)i + (long)c * ldt];
-    Ms[e] = v;
-  }
-  for (int c = threadIdx.x; c < TB; c += 256)
-    dg[c] = (unit || c >= nb) ? 1.0 : T[(long)c * (ldt + 1)];
-  __syncthreads();
-  const int q = blockIdx.x * 256 + threadIdx.x;
-  if (q >= nrhs) return;
-  double x[TB];
-#pragma unroll
-  for (int c = 0; c < TB; ++c)
-    x[c] = (c < nb) ? (ROWS ? B[(long)q + (long)c * ldb] : B[(long)c + (long)q * ldb]) : 0.0;
-#pragma unroll
-  for (int cc = 0; cc < TB; ++cc) {
-    const int c = MLOWER ? cc : TB - 1 - cc;
-    if (c < nb) {
-      if (!unit) x[c] = ROWS ? x[c] * (1.0 / dg[c]) : x[c] / dg[c];
-      if (MLOWER) {
-#pragma unroll
-        for (int i = c + 1; i < TB; ++i) x[i] -= x[c] * Ms[c * TB + i];
-      } else {
-#pragma unroll
-        for (int i = 0; i < c; ++i) x[i] -= x[c] * Ms[c * TB + i];
-      }
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < TB; ++c)
-    if (c < nb) {
-      if (ROWS)
-        B[(long)q + (long)c * ldb] = x[c];
-      else
-        B[(long)c + (long)q * ldb] = x[c];
-    }
-}
-
 // A12 := inv(L11) * A12 for L11 unit lower of order 128 (ld ldl), in place:
 // one wave per 16 columns, 16-row blocks,
 //   X_i = inv(L_ii) (B_i - sum_{k<i} L_ik X_k),
@@ -377,31 +321,6 @@ int launch_trtri_blocks(hipStream_t s, int na, const double* A, long lda, bool u
   return FLA_HIP_OK;
 }
 
-// Solves the nb x nb diagonal block T (ld ldt) of a triangle against nrhs
-// right-hand sides of B in place (left: B is nb x nrhs; right: nrhs x nb).
-static int launch_diag_subst(hipStream_t s, bool left, bool upper, bool trans, bool unit, int nb,
-                             const double* T, long ldt, double* B, long ldb, int nrhs) {
-  if (nb <= 0 || nrhs <= 0) return FLA_HIP_OK;
-  const int flip = (left == trans) ? 1 : 0;
-  const bool mlower = (!upper && !flip) || (upper && flip);
-  const dim3 grid((unsigned)((nrhs + 255) / 256));
-  const int u = unit ? 1 : 0;
-  if (mlower && left)
-    hipLaunchKernelGGL((trsm_diag_subst_kernel<true, false>), grid, dim3(256), 0, s, nrhs, nb, T,
-                       ldt, flip, u, B, ldb);
-  else if (mlower)
-    hipLaunchKernelGGL((trsm_diag_subst_kernel<true, true>), grid, dim3(256), 0, s, nrhs, nb, T,
-                       ldt, flip, u, B, ldb);
-  else if (left)
-    hipLaunchKernelGGL((trsm_diag_subst_kernel<false, false>), grid, dim3(256), 0, s, nrhs, nb, T,
-                       ldt, flip, u, B, ldb);
-  else
-    hipLaunchKernelGGL((trsm_diag_subst_kernel<false, true>), grid, dim3(256), 0, s, nrhs, nb, T,
-                       ldt, flip, u, B, ldb);
-  FLA_HIP_CHECK(hipGetLastError());
-  return FLA_HIP_OK;
-}
-
 static bool is_trans(int t) { return t == kTrans || t == kConjTrans; }
 
 // Scales B by alpha (m x n) when alpha != 1: one MFMA-free elementwise pass.
@@ -422,13 +341,13 @@ static int dtrsm_args_ok(int side, int uplo, int m, int n, int lda, int ldb) {
   return (lda >= na && ldb >= m) ? 1 : 0;
 }
 
-// The few-right-hand-side path (the only one that needs a workspace).
+// The few-right-hand-side path.
 static bool dtrsm_narrow(int side, int n, int na) {
   return side == kLeft && n <= kNarrowRhs && na <= kUcSolveRows;
 }
 
 // Doubles of workspace dtrsm_body needs for a triangle of order na: the
-// inverted 128-blocks, then int words: the wait counter, the wait-failure
+// inverted (few right-hand sides) or reordered 128-blocks, then int words: the wait counter, the wait-failure
 // flag and one condition flag per block.
 static size_t dtrsm_workspace_doubles(int na) {
   const size_t nblk = (size_t)((na + TB - 1) / TB);
@@ -469,64 +388,7 @@ static int dtrsm_body(int side, int uplo, int trans, int diag, int m, int n, dou
     FLA_HIP_CHECK(hipStreamSynchronize(s));
     return herr ? FLA_HIP_ESPIN : FLA_HIP_OK;
   }
-  auto blk = [&](int idx) { return idx * TB; };
-  if (side == kLeft) {
-    // op(A) X = B.  Forward when op(A) is lower.
-    for (int q = 0; q < nblk; ++q) {
-      const int kb = op_lower ? q : (nblk - 1 - q);
-      const int r0 = blk(kb);
-      const int nbk = (na - r0) < TB ? (na - r0) : TB;
-      // X_k := inv(op(T_kk)) * B_k by substitution, in place
-      FLA_TRY(launch_diag_subst(s, true, upper, tr, unit, nbk, A + (long)r0 * (lda + 1), lda,
-                                B + r0, ldb, n));
-      // B_rest -= op(A)[rest, k] * X_k
-      if (op_lower) {
-        const int rr = r0 + nbk, mr = na - rr;
-        if (mr > 0) {
-          // op(A)(i, c) for i in rest, c in block: N -> A[i + c*lda]; T -> A[c + i*lda]
-          const double* Ap = tr ? A + (long)r0 + (long)rr * lda : A + (long)rr + (long)r0 * lda;
-          FLA_TRY(launch_dgemm_mfma(s, tr, false, 0, mr, n, nbk, -1.0, Ap, lda, B + r0, ldb, 1.0,
-                                    B + rr, ldb, nullptr));
-        }
-      } else {
-        const int mr = r0;  // rows above
-        if (mr > 0) {
-          const double* Ap = tr ? A + (long)r0 : A + (long)r0 * lda;
-          FLA_TRY(launch_dgemm_mfma(s, tr, false, 0, mr, n, nbk, -1.0, Ap, lda, B + r0, ldb, 1.0,
-                                    B, ldb, nullptr));
-        }
-      }
-    }
-  } else {
-    // X op(A) = B.  Forward over columns when op(A) is upper.
-    const bool fwd = !op_lower;
-    for (int q = 0; q < nblk; ++q) {
-      const int kb = fwd ? q : (nblk - 1 - q);
-      const int c0 = blk(kb);
-      const int nbk = (na - c0) < TB ? (na - c0) : TB;
-      double* Bk = B + (long)c0 * ldb;
-      // X_k := B_k * inv(op(T_kk)) by substitution, in place
-      FLA_TRY(launch_diag_subst(s, false, upper, tr, unit, nbk, A + (long)c0 * (lda + 1), lda, Bk,
-                                ldb, m));
-      if (fwd) {
-        const int cc = c0 + nbk, nr = na - cc;
-        if (nr > 0) {
-          // B[:, rest] -= X_k * op(A)[k, rest];  op(A)(c, j): N -> A[c + j*lda], T -> A[j + c*lda]
-          const double* Ap = tr ? A + (long)cc + (long)c0 * lda : A + (long)c0 + (long)cc * lda;
-          FLA_TRY(launch_dgemm_mfma(s, false, tr, 0, m, nr, nbk, -1.0, Bk, ldb, Ap, lda, 1.0,
-                                    B + (long)cc * ldb, ldb, nullptr));
-        }
-      } else {
-        const int nr = c0;
-        if (nr > 0) {
-          const double* Ap = tr ? A + (long)c0 * lda : A + (long)c0;
-          FLA_TRY(launch_dgemm_mfma(s, false, tr, 0, m, nr, nbk, -1.0, Bk, ldb, Ap, lda, 1.0, B,
-                                    ldb, nullptr));
-        }
-      }
-    }
-  }
-  return FLA_HIP_OK;
+  return trsm_wide(s, side == kLeft, upper, tr, unit, m, n, A, lda, B, ldb, W);
 }
 
 extern "C" int fla_hip_dtrsm(int side, int uplo, int trans, int diag, int m, int n, double alpha,
@@ -537,8 +399,7 @@ extern "C" int fla_hip_dtrsm(int side, int uplo, int trans, int diag, int m, int
   if (m == 0 || n == 0) return FLA_HIP_OK;
   const int na = (side == kLeft) ? m : n;
   void* w = nullptr;
-  if (dtrsm_narrow(side, n, na))
-    FLA_TRY(fla_workspace(dtrsm_workspace_doubles(na) * sizeof(double), &w));
+  FLA_TRY(fla_workspace(dtrsm_workspace_doubles(na) * sizeof(double), &w));
   return dtrsm_body(side, uplo, trans, diag, m, n, alpha, A, lda, B, ldb,
                     static_cast<double*>(w));
 }

@@ -1,0 +1,41 @@
+"""The triangular solve with many right-hand sides at the sizes where it can go
+wrong: edges of the 16-column blocks, the 128-blocks and the groups of four,
+ragged ends in both directions, and right-hand-side counts around a wave's 16
+rows.  Integer solutions of integer systems must come out exactly."""
+import numpy as np
+import pytest
+
+import libflame_amd as fla
+from tests.cases import exact_tri
+from tests.gpu_util import gpu_trsm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    fla.FLA_Init()
+    yield
+
+
+@pytest.mark.parametrize("n,nrhs", [(1, 33), (15, 64), (17, 40), (127, 33), (129, 65), (143, 100),
+                                    (512, 49), (513, 40), (700, 37)])
+@pytest.mark.parametrize("left", [True, False])
+@pytest.mark.parametrize("lower", [True, False])
+@pytest.mark.parametrize("trans", [True, False])
+def test_exact(n, nrhs, left, lower, trans):
+    unit = bool((n + nrhs) & 1)
+    T = exact_tri(n, seed=n, lower=lower, unit=unit)
+    # sparse off-diagonal part: the exact solutions stay small
+    T = np.where(np.eye(n, dtype=bool) | (np.random.default_rng(n).random((n, n)) < 0.05), T, 0.0)
+    X = np.random.default_rng(nrhs).integers(-4, 5, size=(n, nrhs) if left else (nrhs, n))
+    op = T.T if trans else T
+    B = op @ X if left else X @ op
+    S = T.copy()
+    if unit:
+        np.fill_diagonal(S, 7.0)  # a unit diagonal is not read
+    out = gpu_trsm(fla.FLA_LEFT if left else fla.FLA_RIGHT,
+                   fla.FLA_LOWER_TRIANGULAR if lower else fla.FLA_UPPER_TRIANGULAR,
+                   fla.FLA_TRANSPOSE if trans else fla.FLA_NO_TRANSPOSE,
+                   fla.FLA_UNIT_DIAG if unit else fla.FLA_NONUNIT_DIAG, S, B.astype(np.float64))
+    assert np.array_equal(out, X)

@@ -404,6 +404,16 @@ int chol_panel_f64(hipStream_t s, int n, double* A, long lda, int k, int kb, int
   return FLA_HIP_OK;
 }
 
+// Trailing order from which the updates move to the stream that leaves CUs to
+// the panels.  A CU mask costs the update an eighth of its rate even if it
+// takes 8 of 256 CUs (the XCDs' shader engines get equal shares of the
+// workgroups and the one with fewer CUs is last: 58.5 against 66.9 TFLOP/s),
+// but a panel kernel then never waits for CUs.  FLA_Chol with 0, 6000, 9000,
+// 13000, 20000: n = 32768 199.1, 199.5, 199.0, 198.4, 199.1 ms; n = 16384
+// 32.7, 32.3, 32.0, 31.6, 32.0 ms; n = 8192 7.07, 6.73, 6.63, 6.62, 6.62 ms
+// (all updates on a stream that leaves 8 CUs: 212.0, 32.5 and 6.9 ms).
+constexpr int kMaskedOrder = 13000;
+
 // Lower blocked Cholesky with look-ahead: the panel of step k+1 runs on
 // s_panel while the bulk of step k's trailing update runs on s_update.
 static int chol_lower(int n, double* A, long lda, int* dinfo) {
@@ -429,6 +439,13 @@ static int chol_lower(int n, double* A, long lda, int* dinfo) {
     const int k2 = k + kb;      // first column of the trailing matrix
     const int m2 = n - k2;      // its order
     if (m2 <= 0) break;
+    if (su == c.s_update && m2 <= kMaskedOrder) {
+      // from here on the panel chain outlasts the update: it gets CUs of its own
+      hipEvent_t sw = next_event();
+      FLA_HIP_CHECK(hipEventRecord(sw, su));
+      su = c.s_update_lp;
+      FLA_HIP_CHECK(hipStreamWaitEvent(su, sw, 0));
+    }
     const double* P = A + (long)k2 + (long)k * lda;  // m2 x kb, the factored panel
     const int kb2 = m2 < nb ? m2 : nb;             // width of the next panel
     // (a) next panel's columns: rows k2.., columns [k2, k2+kb2) (lower part)
@@ -455,7 +472,12 @@ static int chol_lower(int n, double* A, long lda, int* dinfo) {
   // Join: s_update waits for the last panel.
   hipEvent_t fin = next_event();
   FLA_HIP_CHECK(hipEventRecord(fin, sp));
-  FLA_HIP_CHECK(hipStreamWaitEvent(su, fin, 0));
+  FLA_HIP_CHECK(hipStreamWaitEvent(c.s_update, fin, 0));
+  if (su != c.s_update) {
+    hipEvent_t last = next_event();
+    FLA_HIP_CHECK(hipEventRecord(last, su));
+    FLA_HIP_CHECK(hipStreamWaitEvent(c.s_update, last, 0));
+  }
   return FLA_HIP_OK;
 }
 

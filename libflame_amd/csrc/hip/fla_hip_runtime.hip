@@ -18,11 +18,10 @@ int g_tile_group = 4;
 
 FlaHipCtx& fla_ctx() { return g_ctx; }
 
-// The update stream may leave the last `reserved` CUs to the panel stream:
-// the trailing update launches thousands of LDS-heavy workgroups, and a
-// single-workgroup panel kernel that needs a whole CU's LDS would otherwise
-// wait for a CU to drain completely.
-static int g_reserved_cus = 8;
+// The update stream may leave the last `reserved` CUs to the panel stream.
+// None by default: eight (one of each XCD) cost an eighth of the update's
+// rate, since every shader engine gets the same share of its workgroups.
+static int g_reserved_cus = 0;
 // The second update stream leaves 32 CUs (four of each XCD) to the panels.
 // It carries the reduced-precision factor's updates and the LU's bulk
 // updates, whose panel kernel needs one whole CU per 1024 rows with all its

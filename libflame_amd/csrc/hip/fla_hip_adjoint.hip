@@ -91,8 +91,7 @@ extern "C" int fla_hip_dchol_adjoint(int n, const double* L, int ldl, const doub
                      (long)n);
   FLA_HIP_CHECK(hipGetLastError());
   // Abar (lower) := L^T Lbar ; only the lower triangle is needed
-  FLA_TRY(launch_dgemm_mfma(s, true, false, 1, n, n, n, 1.0, Lc, n, Lb, n, 0.0, Abar, ldab,
-                            nullptr));
+  FLA_TRY(launch_dgemm_tri_tn(s, n, Lc, n, Lb, n, Abar, ldab));
   hipLaunchKernelGGL(phi_kernel, dim3(nblk(nn)), dim3(256), 0, s, n, Abar, (long)ldab);
   FLA_HIP_CHECK(hipGetLastError());
   // G = L^-T P L^-1

@@ -375,6 +375,155 @@ int launch_kp(hipStream_t s, bool vec, int mode, int m, int n, int k, double alp
   return FLA_HIP_OK;
 }
 
+// The same tiling and LDS layout for any transposition and any size.  An
+// operand whose tile rows are contiguous (A, or B') is loaded as above; one
+// whose k are contiguous (A', or B) needs no pairing: one 16-byte load is an
+// LDS entry (8 lanes read a row's 128 bytes).  EDGE: rows past the matrix read
+// its last row (never stored), k past its end is zero.  ktri: op(A)(i, k) = 0
+// for k < i (a lower triangle transposed), so a tile's sum starts at its row.
+typedef kp_d2 kp_d2u __attribute__((aligned(8)));
+template <bool TA, bool TB, bool EDGE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void dgemm_kp_kernel(
+    int mode, int ktri, int m, int n, int k, double alpha, const double* A, long lda,
+    const double* B, long ldb, double beta, double* C, long ldc, int Tm, int Tn, int rpc,
+    const int* __restrict__ abort_flag) {
+  constexpr int BK = KP_BK, WM = 2, WN = 4, NT = 512, NKP = BK / 2, KP_LD = KP_BM + 4;
+  constexpr int TM = KP_BM / WM / 16, TN = KP_BM / WN / 16;
+  if (abort_flag && *abort_flag >= 0) return;
+  __shared__ kp_d2 As[2][NKP * KP_LD];
+  __shared__ kp_d2 Bs[2][NKP * KP_LD];
+  int ti, tj;
+  fla_tile_of(blockIdx.x, gridDim.x, mode, Tm, Tn, rpc, ti, tj);
+  const int i0 = ti * KP_BM, j0 = tj * KP_BM;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int wr = wave / WN, wc = wave % WN;
+  const int li = lane & 15, lk = lane >> 4;
+  // Rows contiguous: row tid % 128, k pairs tid / 128 + 4 q.  k contiguous: k
+  // pair tid % 8, rows tid / 8 + 64 q.  32-bit lane offsets from a uniform base.
+  const int rA = TA ? tid / NKP : tid & (KP_BM - 1), kA = TA ? tid % NKP : tid / KP_BM;
+  const int rB = TB ? tid & (KP_BM - 1) : tid / NKP, kB = TB ? tid / KP_BM : tid % NKP;
+  unsigned oa[2], ob[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    int ra = rA + (TA ? 64 * q : 0), rb = rB + (TB ? 0 : 64 * q);
+    if (EDGE) {
+      ra = min(ra, m - 1 - i0);
+      rb = min(rb, n - 1 - j0);
+    }
+    oa[q] = TA ? (unsigned)(2 * kA) + (unsigned)ra * (unsigned)lda
+               : (unsigned)ra + (unsigned)(2 * kA + 8 * q) * (unsigned)lda;
+    ob[q] = TB ? (unsigned)rb + (unsigned)(2 * kB + 8 * q) * (unsigned)ldb
+               : (unsigned)(2 * kB) + (unsigned)rb * (unsigned)ldb;
+  }
+  const int sA = kA * KP_LD + rA, sB = kB * KP_LD + rB;
+  const int dA = TA ? 64 : 4 * KP_LD, dB = TB ? 4 * KP_LD : 64;
+  v4d acc[TM][TN];
+#pragma unroll
+  for (int a = 0; a < TM; ++a)
+#pragma unroll
+    for (int b = 0; b < TN; ++b) acc[a][b] = v4d{0.0, 0.0, 0.0, 0.0};
+  const double* const Ab = A + (TA ? (long)i0 * lda : (long)i0);
+  const double* const Bb = B + (TB ? (long)j0 : (long)j0 * ldb);
+  kp_d2 ra[2], rb[2];
+  auto load = [&](int kc) {
+    const double* const a0 = Ab + (TA ? (long)kc * BK : (long)kc * BK * lda);
+    const double* const b0 = Bb + (TB ? (long)kc * BK * ldb : (long)kc * BK);
+    if (!EDGE || (kc + 1) * BK <= k) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        if constexpr (TA)
+          ra[q] = *reinterpret_cast<const kp_d2u*>(a0 + oa[q]);
+        else
+          ra[q] = kp_d2{a0[oa[q]], (a0 + lda)[oa[q]]};
+        if constexpr (TB)
+          rb[q] = kp_d2{b0[ob[q]], (b0 + ldb)[ob[q]]};
+        else
+          rb[q] = *reinterpret_cast<const kp_d2u*>(b0 + ob[q]);
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int ka = kc * BK + 2 * (TA ? kA : kA + 4 * q), kb = kc * BK + 2 * (TB ? kB + 4 * q : kB);
+        ra[q].x = ka < k ? a0[oa[q]] : 0.0;
+        ra[q].y = ka + 1 < k ? (a0 + (TA ? 1 : lda))[oa[q]] : 0.0;
+        rb[q].x = kb < k ? b0[ob[q]] : 0.0;
+        rb[q].y = kb + 1 < k ? (b0 + (TB ? ldb : 1))[ob[q]] : 0.0;
+      }
+    }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      As[buf][sA + q * dA] = ra[q];
+      Bs[buf][sB + q * dB] = rb[q];
+    }
+  };
+  const int nk = EDGE ? (k + BK - 1) / BK : k / BK;
+  const int kt0 = ktri ? i0 / BK : 0;
+  if (kt0 < nk) {
+    load(kt0);
+    store(0);
+  }
+  __syncthreads();
+  for (int kt = kt0; kt < nk; ++kt) {
+    const int cur = (kt - kt0) & 1;
+    const bool more = kt + 1 < nk;
+    if (more) load(kt + 1);
+    const kp_d2* as = As[cur];
+    const kp_d2* bs = Bs[cur];
+#pragma unroll
+    for (int p = 0; p < NKP / 4; ++p) {
+      kp_d2 fa[TM], fb[TN];
+#pragma unroll
+      for (int t = 0; t < TM; ++t) fa[t] = as[(4 * p + lk) * KP_LD + wr * (KP_BM / WM) + t * 16 + li];
+#pragma unroll
+      for (int t = 0; t < TN; ++t) fb[t] = bs[(4 * p + lk) * KP_LD + wc * (KP_BM / WN) + t * 16 + li];
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[b].x, fa[a].x, acc[a][b], 0, 0, 0);
+#pragma unroll
+      for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[b].y, fa[a].y, acc[a][b], 0, 0, 0);
+    }
+    if (more) store(cur ^ 1);
+    __syncthreads();
+  }
+  store_tile<KP_BM, KP_BM, WM, WN, TM, TN>(acc, mode, m, n, alpha, beta, C, ldc, i0, j0, wr, wc,
+                                           li, lk);
+}
+
+template <bool TA, bool TB>
+int launch_kp_any(hipStream_t s, int mode, int ktri, int m, int n, int k, double alpha,
+                  const double* A, long lda, const double* B, long ldb, double beta, double* C,
+                  long ldc, const int* abort_flag) {
+  const int Tm = (m + KP_BM - 1) / KP_BM, Tn = (n + KP_BM - 1) / KP_BM;
+  const long nblk = (mode == 0) ? (long)Tm * Tn : (long)Tn * Tm - (long)Tn * (Tn - 1) / 2;
+  if (nblk > 0x7fffffffL) return FLA_HIP_EARG;
+  if ((TA || !TB) && m % KP_BM == 0 && n % KP_BM == 0 && k % KP_BK == 0)
+    hipLaunchKernelGGL((dgemm_kp_kernel<TA, TB, !(TA || !TB)>), dim3((unsigned)nblk), dim3(512), 0, s,
+                       mode, ktri, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, Tm, Tn,
+                       g_tile_group, abort_flag);
+  else
+    hipLaunchKernelGGL((dgemm_kp_kernel<TA, TB, true>), dim3((unsigned)nblk), dim3(512), 0, s,
+                       mode, ktri, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, Tm, Tn,
+                       g_tile_group, abort_flag);
+  FLA_HIP_CHECK(hipGetLastError());
+  return FLA_HIP_OK;
+}
+
+int launch_kp_any(hipStream_t s, bool ta, bool tb, int mode, int ktri, int m, int n, int k,
+                  double alpha, const double* A, long lda, const double* B, long ldb, double beta,
+                  double* C, long ldc, const int* abort_flag) {
+  auto f = ta ? (tb ? launch_kp_any<true, true> : launch_kp_any<true, false>)
+              : (tb ? launch_kp_any<false, true> : launch_kp_any<false, false>);
+  return f(s, mode, ktri, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, abort_flag);
+}
+
 // C := alpha*A*B' + beta*C for shapes whose 128 x 128 tiles would leave most
 // of the chip idle: 64 x 64 of C per workgroup of 4 waves, each 32 x 32 = 2 x 2
 // MFMA blocks, operands straight from memory into registers (a fragment load
@@ -563,11 +712,21 @@ int launch_dgemm_mfma(hipStream_t s, bool ta, bool tb, int mode, int m, int n, i
     if (t128 <= fla_ctx().num_cus)
       return launch_direct(s, mode, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, abort_flag);
   }
-  // Default (0) and 12..15: the k-pair kernel wherever it applies (A and B
-  // with the tile rows contiguous, full tiles, K a multiple of the chunk),
-  // measured on MI355X at 54.9 TFLOP/s on the n = 32768 Cholesky update
-  // against 51.0 for the 8-byte-layout kernel (configuration 2).
-  if (g_gemm_cfg == 0 || g_gemm_cfg >= 12) {
+  // The pair kernel of whole tiles where both operands are row-contiguous
+  // (n = 30720, K = 1024 lower update: 68.2 TFLOP/s with 2 x 4 waves, 66.9
+  // with 4 x 2), else its general form (FLA_Chol_adjoint n = 8192 34.9 ->
+  // 28.0 ms with it in place of the 8-byte layout below, which keeps K = 0
+  // and leading dimensions past 2^24).
+  if (g_gemm_cfg == 0 && !ta && tb && m % KP_BM == 0 && n % KP_BM == 0 && k % KP_BK == 0 &&
+      k > 0 && lda < (1L << 26) && ldb < (1L << 26))
+    return launch_kp<16, 2, 4>(s, false, mode, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
+                               abort_flag);
+  if (g_gemm_cfg == 0 && k > 0 && lda < (1L << 24) && ldb < (1L << 24))
+    return launch_kp_any(s, ta, tb, mode, 0, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc,
+                         abort_flag);
+  // 12..19: alternatives of the k-pair kernel where both operands have
+  // the tile rows contiguous, full tiles, K a multiple of the chunk.
+  if (g_gemm_cfg >= 12) {
     const int bk = (g_gemm_cfg == 15) ? 32 : KP_BK;
     if (!ta && tb && m % KP_BM == 0 && n % KP_BM == 0 && k % bk == 0 && k > 0 &&
         lda < (1L << 26) && ldb < (1L << 26)) {
@@ -649,6 +808,14 @@ int launch_dgemm_mfma(hipStream_t s, bool ta, bool tb, int mode, int m, int n, i
       return launch_cfg<128, 128, 16, 4, 2>(s, ta, tb, mode, m, n, k, alpha, A, lda, B, ldb, beta,
                                             C, ldc, abort_flag);
   }
+}
+
+// C (lower n x n) := A' B with A and B lower triangles whose strictly upper
+// parts are zero: the sums start at the tile's row.
+int launch_dgemm_tri_tn(hipStream_t s, int n, const double* A, long lda, const double* B, long ldb,
+                        double* C, long ldc) {
+  if (n <= 0) return FLA_HIP_OK;
+  return launch_kp_any(s, true, false, 1, 1, n, n, n, 1.0, A, lda, B, ldb, 0.0, C, ldc, nullptr);
 }
 
 static bool is_trans(int t) { return t == kTrans || t == kConjTrans; }

@@ -211,6 +211,8 @@ constexpr int kNarrowRhs = 32;
 int launch_trsm_left_narrow(hipStream_t s, bool op_lower, bool trans, int na, int nrhs,
                             const double* T, long ldt, const double* W, double* X, long ldx,
                             int* done, int* err, const int* ill = nullptr, bool unit = false);
+int launch_dgemm_tri_tn(hipStream_t s, int n, const double* A, long lda, const double* B, long ldb,
+                        double* C, long ldc);
 // The triangular solve with many right-hand sides: op(A) X = B (left) or
 // X op(A) = B in place on the m x n B.  W: 128 x 128 doubles per 128-block of A.
 int trsm_wide(hipStream_t s, bool left, bool upper, bool tr, bool unit, int m, int n,

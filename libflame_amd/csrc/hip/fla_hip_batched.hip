@@ -5,30 +5,24 @@
 // is ordered by decreasing n, so the large matrices start first and the
 // small ones fill the tail), factors its matrix alone and, when right-hand
 // sides are given, solves with them before taking the next index.  The
-// algorithms follow the right-looking blocked forms of FLA_Chol_l_blk_var3
-// (src/lapack/dec/chol/l/flamec/FLA_Chol_l_blk_var3.c) and FLA_LU_piv_blk_var5
-// (src/lapack/dec/lu/piv/vars/flamec/FLA_LU_piv_blk_var5.c) with a panel of
-// NB columns held in LDS:
-//   Cholesky: unblocked right-looking factor of the m x NB panel in LDS
-//     (dpotf2 order: sqrt, invscal, rank-1 update), then the trailing update
-//     A22 -= L21 L21^T on MFMA (lower 32 x 32 tiles, read-modify-write).
-//   LU: per column of the panel the pivot is the first maximal |a| of the
-//     column (idamax_, src/flablas/f2c/idamax.c:40-46, NaN rule included),
-//     rows are swapped across the whole matrix (FLAME-native relative
-//     pivots), the column scaled by the reciprocal of the pivot and the
-//     panel updated; then A12 := inv(L11) A12 and A22 -= L21 A12 on MFMA.
-// The forward substitution of the solve runs inside the factorization,
-// panel by panel, while L's panel is in LDS; the backward substitution reads
-// the factor once more from memory, with the right-hand sides staged in LDS.
-// Both solve 16 rows at a time: one wave sweeps the diagonal block with the
-// right-hand sides in registers (lanes exchange values by shuffles, no
-// barrier per column), then every thread updates the remaining rows.
+// algorithms follow the blocked forms of FLA_Chol_l_blk_var3
+// (src/lapack/dec/chol/l/flamec/FLA_Chol_l_blk_var3.c; here left-looking over
+// 16 x 16 blocks, fla_hip_posv.h) and FLA_LU_piv_blk_var5
+// (src/lapack/dec/lu/piv/vars/flamec/FLA_LU_piv_blk_var5.c), the latter with
+// a panel of NB columns held in LDS: per column of the panel the pivot is the
+// first maximal |a| of the column (idamax_, src/flablas/f2c/idamax.c:40-46,
+// NaN rule included), rows are swapped across the whole matrix (FLAME-native
+// relative pivots), the column scaled by the reciprocal of the pivot and the
+// panel updated; then A12 := inv(L11) A12 and A22 -= L21 A12 on MFMA.
+// The forward substitution of the solve runs inside the factorization; the
+// backward substitution reads the factor once more from memory.
 //
 // Element types: double (v_mfma_f64_16x16x4f64) and float
 // (v_mfma_f32_16x16x4f32).  Info per matrix: FLA_SUCCESS, or the 0-based
 // failing column (Cholesky) / first null pivot (LU, factorization continues
 // as FLA_LU_piv does).
 #include "fla_hip_internal.h"
+#include "fla_hip_posv.h"
 
 #include <algorithm>
 #include <cmath>
@@ -402,198 +396,6 @@ __device__ __forceinline__ void rows_update(const T* P, int p0, int sb, int i0, 
   }
 }
 
-// Forward substitution with the factored Cholesky panel in LDS (element
-// (i, j) at P[i + j*MAXN], m rows, kb columns): the panel's rows of B (B
-// points at the panel's first row) are solved against the diagonal block
-// and the rows below are updated, 16 columns at a time.  Each wave solves 8
-// right-hand sides per pass; the update subtracts one term at a time in
-// column order (dtrsm_'s order for B := inv(L) B).
-template <typename T>
-__device__ __forceinline__ void chol_panel_forward(const T* P, int kb, int m, T* B, long ldb,
-                                                   int nrhs, T* Ys, int t) {
-  const int w = t >> 6, lane = t & 63, r = lane & 15, g = lane >> 4;
-  for (int s0 = 0; s0 < kb; s0 += 16) {
-    const int sb = min(16, kb - s0), row = s0 + r;
-    for (int cg = 0; cg < nrhs; cg += 32) {
-      const int ncg = min(32, nrhs - cg);
-      if (8 * w < ncg) {
-        T cf[16];
-#pragma unroll
-        for (int j = 0; j < 16; ++j) cf[j] = (r < sb && j < sb) ? P[row + (s0 + j) * MAXN] : (T)0;
-        const T dg = r < sb ? P[row + row * MAXN] : (T)1;
-        T x[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int cc = 8 * w + g + 4 * q;
-          x[q] = (r < sb && cc < ncg) ? B[row + (long)(cg + cc) * ldb] : (T)0;
-        }
-        wave_trsv16<T, true>(x, cf, dg, r, g, sb);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int cc = 8 * w + g + 4 * q;
-          if (r < sb && cc < ncg) {
-            B[row + (long)(cg + cc) * ldb] = x[q];
-            Ys[r + cc * 16] = x[q];
-          }
-        }
-      }
-      __syncthreads();
-      rows_update<T, 16>(P, s0, sb, s0 + sb, m, B, ldb, cg, ncg, Ys, t);
-      __syncthreads();
-    }
-  }
-}
-
-// Column J of the register-resident Cholesky panel (compile-time J keeps
-// v in registers): the threads of rows < kb publish their column-J values,
-// then each thread scales its rows' column J and updates its rows' columns
-// J+1..min(r, kb-1).  jfail: the first column with a non-positive (or NaN)
-// diagonal; the later columns are skipped.
-template <typename T, int NB, int J>
-__device__ __forceinline__ void chol_reg_column(T (&v)[2][NB], T (*colb)[NB], int kb, int m, int t,
-                                                int& jfail) {
-  if (J < kb && jfail < 0) {
-    if (t < kb) colb[J & 1][t] = v[0][J];
-    __syncthreads();
-    const T d = colb[J & 1][J];
-    if (!(d > (T)0)) {
-      jfail = J;
-      return;
-    }
-    const T sd = sqrt(d);
-    const T inv = (T)1 / sd;
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int r = t + 256 * q;
-      if (r == J) {
-        v[q][J] = sd;
-      } else if (r > J && r < m) {
-        const T lr = v[q][J] * inv;
-        v[q][J] = lr;
-#pragma unroll
-        for (int c = J + 1; c < NB; ++c)
-          if (c < kb && c <= r) v[q][c] -= lr * (colb[J & 1][c] * inv);
-      }
-    }
-  }
-}
-template <typename T, int NB, int... J>
-__device__ __forceinline__ void chol_reg_columns(T (&v)[2][NB], T (*colb)[NB], int kb, int m,
-                                                 int t, int& jfail,
-                                                 std::integer_sequence<int, J...>) {
-  (chol_reg_column<T, NB, J>(v, colb, kb, m, t, jfail), ...);
-}
-
-// ---- Cholesky of one matrix (lower), fused forward substitution -----------
-template <typename T, int NB>
-__device__ int chol_one(T* A, long lda, int n, T* B, long ldb, int nrhs, T* P, T* Ys, int t) {
-  __shared__ T colb[2][NB];  // the published column, by column parity
-  int fail = -1;
-  for (int k = 0; k < n; k += NB) {
-    const int kb = min(NB, n - k), m = n - k;
-    // The panel A[k:n, k:k+kb] in registers: thread t owns rows t and
-    // t + 256.  Per column j, the threads of rows < kb publish their current
-    // column-j values (double-buffered by column parity, one barrier); every
-    // thread then scales its rows' column j (l = a * (1/d)) and updates its
-    // rows' columns j+1..min(r, kb-1) with l * (a_cj * (1/d)), the
-    // multipliers of the top rows formed from the published values.  These
-    // are dpotf2's operations in its order, per element.
-    T v[2][NB];
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        const int r = t + 256 * q;
-        v[q][c] = (r < m && c < kb) ? A[(k + r) + (long)(k + c) * lda] : (T)0;
-      }
-    int jfail = -1;
-    chol_reg_columns<T, NB>(v, colb, kb, m, t, jfail, std::make_integer_sequence<int, NB>{});
-    if (jfail >= 0) fail = k + jfail;
-    // the factored panel to LDS (trailing update, forward solve) and, lower
-    // part, back to A
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        const int r = t + 256 * q;
-        if (r < m && c < kb) {
-          P[r + c * MAXN] = v[q][c];
-          if (r >= c) A[(k + r) + (long)(k + c) * lda] = v[q][c];
-        }
-      }
-    __syncthreads();
-    if (fail >= 0) return fail;
-    // forward substitution with this panel: Y_k = L_kk^-1 B_k, B_rest -= L21 Y_k
-    if (nrhs > 0) chol_panel_forward<T>(P, kb, m, B + k, ldb, nrhs, Ys, t);
-    // trailing update
-    if (m > kb)
-      tile_update<T, true, NB, false>(m - kb, m - kb, kb, P + kb, P + kb, 1, MAXN,
-                           A + (k + kb) + (long)(k + kb) * lda, lda, t);
-    __syncthreads();
-  }
-  return fail;
-}
-
-// Backward substitution X := L^-T Y (L lower in A) for up to 8 right-hand
-// sides, staged in LDS (X, ld MAXN).  From the bottom, 16 rows at a time:
-// one wave solves the diagonal block in registers, then every thread
-// updates the rows above with the block's solution.
-template <typename T>
-__device__ void chol_back(const T* A, long lda, int n, T* B, long ldb, int nrhs, T* X, int t) {
-  const int w = t >> 6, lane = t & 63, r = lane & 15, g = lane >> 4;
-  for (int e = t; e < n * nrhs; e += 256) X[e % n + (e / n) * MAXN] = B[e % n + (long)(e / n) * ldb];
-  __syncthreads();
-  for (int k = ((n - 1) / 16) * 16; k >= 0; k -= 16) {
-    const int kb = min(16, n - k);
-    // the rows-above update's multipliers, loaded before the block solve
-    T l[2][16];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int i = t + 256 * q;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) l[q][j] = (i < k && j < kb) ? A[(k + j) + (long)i * lda] : (T)0;
-    }
-    if (w == 0) {
-      // row r of the block of L^T: L[k + j, k + r]
-      T cf[16];
-#pragma unroll
-      for (int j = 0; j < 16; ++j)
-        cf[j] = (r < kb && j < kb) ? A[(k + j) + (long)(k + r) * lda] : (T)0;
-      const T dg = r < kb ? A[(k + r) + (long)(k + r) * lda] : (T)1;
-      T x[2];
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int c = g + 4 * q;
-        x[q] = (r < kb && c < nrhs) ? X[(k + r) + c * MAXN] : (T)0;
-      }
-      wave_trsv16<T, false>(x, cf, dg, r, g, kb);
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int c = g + 4 * q;
-        if (r < kb && c < nrhs) X[(k + r) + c * MAXN] = x[q];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int i = t + 256 * q;
-      if (i < k) {
-#pragma unroll 1
-        for (int c = 0; c < nrhs; ++c) {
-          T v = X[i + c * MAXN];
-#pragma unroll
-          for (int j = 0; j < 16; ++j)
-            if (j < kb) v -= l[q][j] * X[(k + j) + c * MAXN];
-          X[i + c * MAXN] = v;
-        }
-      }
-    }
-    __syncthreads();
-  }
-  for (int e = t; e < n * nrhs; e += 256) B[e % n + (long)(e / n) * ldb] = X[e % n + (e / n) * MAXN];
-  __syncthreads();
-}
-
 // ---- LU with partial pivoting of one square matrix, fused forward solve ----
 template <typename T, int NB>
 __device__ int lu_one(T* A, long lda, int n, int* ipiv, T* B, long ldb, int nrhs, T* P,
@@ -895,23 +697,18 @@ __device__ void lu_back(const BatchItem* itp, int c0, int nrhs,
   __syncthreads();
 }
 
-// Persistent driver: OP 0 Cholesky (lower), 1 LU with partial pivoting.
-// As many workgroups share a CU (up to 4) as the panel's LDS allows; the
-// register budget is held to that occupancy.
-template <typename T, int OP, int NB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
-    (160 * 1024) / ((MAXN + 32) * NB * sizeof(T) + 1024) >= 4
-        ? 4
-        : ((160 * 1024) / ((MAXN + 32) * NB * sizeof(T) + 1024) >= 2 ? 2 : 1)))) void batched_kernel(const BatchItem* __restrict__ items,
-                                                      int count, int* counter, int* info,
-                                                      int max_rhs) {
+// Persistent driver of the general systems: LU with partial pivoting, two
+// 256-thread workgroups a CU (what the panel's LDS allows; the register
+// budget is held to it).
+template <typename T, int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gesv_kernel(
+    const BatchItem* __restrict__ items, int count, int* counter, int* info) {
   __shared__ T P[MAXN * NB];
   __shared__ T Ys[NB * 32];  // solved rows of the right-hand sides, 32 columns
   __shared__ AmaxSum red[8];
   __shared__ int spiv[NB];
   __shared__ int cur;
   const int t = threadIdx.x;
-  (void)max_rhs;
   for (;;) {
     if (t == 0) cur = atomicAdd(counter, 1);
     __syncthreads();
@@ -919,28 +716,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
     __syncthreads();
     if (idx >= count) break;
     const BatchItem it = items[idx];
-    // global pointers for the LU; the Cholesky kernels measured faster with
-    // the generic ones
-    T* A = OP == 1 ? global_field<T>(&items[idx].A) : static_cast<T*>(it.A);
-    T* B = OP == 1 ? global_field<T>(&items[idx].B) : static_cast<T*>(it.B);
+    T* A = global_field<T>(&items[idx].A);
+    T* B = global_field<T>(&items[idx].B);
     const int nr = it.B ? it.nrhs : 0;
-    int r;
-    if (OP == 0) {
-      r = chol_one<T, NB>(A, it.lda, it.n, B, it.ldb, nr, P, Ys, t);
-      __syncthreads();
-      if (r < 0 && nr > 0) {
-        for (int c0 = 0; c0 < nr; c0 += 8)
-          chol_back<T>(A, it.lda, it.n, B + (long)c0 * it.ldb, it.ldb, min(8, nr - c0), P, t);
-      }
-    } else {
-      r = lu_one<T, NB>(A, it.lda, it.n, global_field<int>((void* const*)&items[idx].ipiv), B,
-                        it.ldb, nr, P, red, spiv, Ys, t);
-      __syncthreads();
-      if (r < 0 && nr > 0) {
-        for (int c0 = 0; c0 < nr; c0 += 8)
-          lu_back<T>(&items[idx], c0, min(8, nr - c0), (__attribute__((address_space(3))) T*)P, t);
-      }
+    const int r = lu_one<T, NB>(A, it.lda, it.n, global_field<int>((void* const*)&items[idx].ipiv),
+                                B, it.ldb, nr, P, red, spiv, Ys, t);
+    __syncthreads();
+    if (r < 0 && nr > 0) {
+      for (int c0 = 0; c0 < nr; c0 += 8)
+        lu_back<T>(&items[idx], c0, min(8, nr - c0), (__attribute__((address_space(3))) T*)P, t);
     }
+    if (t == 0) info[it.index] = r < 0 ? kSuccess : r;
+    __syncthreads();
+  }
+}
+
+// Persistent driver of the SPD systems: one 512-thread workgroup per matrix;
+// one a CU in FP64 (226 VGPRs; held to 128 it spills and ran 6.8 instead of 6.3
+// ms on the batch below), two in FP32.  Bound: the chain of a matrix's block
+// columns (diagonal factor, substitution, memory round trips) with eight or
+// sixteen waves a CU.  4096 matrices of n ~ U{32..512} with 1-8 right-hand
+// sides, with the copies in: FP64 10.4 -> 6.4 ms, FP32 6.1 -> 3.6 ms against a
+// right-looking kernel of 16-column panels in LDS.
+template <typename T>
+__global__ __launch_bounds__(64 * fla_posv::NW, sizeof(T) == 8 ? 2 : 4) void posv_kernel(
+    const BatchItem* __restrict__ items, int count, int* counter, int* info) {
+  __shared__ fla_posv::Shared<T> S;
+  __shared__ int cur;
+  const int t = threadIdx.x;
+  for (;;) {
+    if (t == 0) cur = atomicAdd(counter, 1);
+    __syncthreads();
+    const int idx = __builtin_amdgcn_readfirstlane(cur);
+    __syncthreads();
+    if (idx >= count) break;
+    const BatchItem it = items[idx];
+    const int r = fla_posv::posv_one<T>(global_field<T>(&items[idx].A), it.lda, it.n,
+                                        global_field<T>(&items[idx].B), it.ldb,
+                                        it.B ? it.nrhs : 0, S, t);
     if (t == 0) info[it.index] = r < 0 ? kSuccess : r;
     __syncthreads();
   }
@@ -951,7 +764,7 @@ __global__ void reset_counter_kernel(int* c) { *c = 0; }
 // ---- host side: schedule, configurations, autotuner, graph replay ----------
 
 struct BatchConfig {
-  int nb = 32;        // panel width
+  int nb = 16;        // panel width of the LU kernel
   int wg_per_cu = 1;  // persistent workgroups per CU
 };
 
@@ -1011,38 +824,36 @@ BatchConfig lookup_config(int kind, const Signature& sig) {
   return default_config(kind);
 }
 
-template <typename T, int OP, int NB>
-int launch_batched(hipStream_t s, int grid, const BatchItem* items, int count, int* counter,
-                   int* info) {
-  hipLaunchKernelGGL((batched_kernel<T, OP, NB>), dim3(grid), dim3(256), 0, s, items, count,
-                     counter, info, 0);
-  FLA_HIP_CHECK(hipGetLastError());
-  return FLA_HIP_OK;
-}
-
 int launch_kind(hipStream_t s, int kind, const BatchConfig& cfg, int count, int* info) {
   const int grid = std::max(1, std::min(count, fla_ctx().num_cus * cfg.wg_per_cu));
   hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(1), 0, s, g_counter);
   FLA_HIP_CHECK(hipGetLastError());
-  if (kind == kDpotrf) {
-    if (cfg.nb == 16) return launch_batched<double, 0, 16>(s, grid, g_items_dev, count, g_counter, info);
-    return launch_batched<double, 0, 32>(s, grid, g_items_dev, count, g_counter, info);
+  if (kind != kDgetrf) {
+    if (kind == kDpotrf)
+      hipLaunchKernelGGL(posv_kernel<double>, dim3(grid), dim3(64 * fla_posv::NW), 0, s,
+                         g_items_dev, count, g_counter, info);
+    else
+      hipLaunchKernelGGL(posv_kernel<float>, dim3(grid), dim3(64 * fla_posv::NW), 0, s,
+                         g_items_dev, count, g_counter, info);
+    FLA_HIP_CHECK(hipGetLastError());
+    return FLA_HIP_OK;
   }
-  if (kind == kSpotrf) {
-    if (cfg.nb == 16) return launch_batched<float, 0, 16>(s, grid, g_items_dev, count, g_counter, info);
-    return launch_batched<float, 0, 32>(s, grid, g_items_dev, count, g_counter, info);
-  }
-  return launch_batched<double, 1, 16>(s, grid, g_items_dev, count, g_counter, info);
+  hipLaunchKernelGGL((gesv_kernel<double, 16>), dim3(grid), dim3(256), 0, s, g_items_dev, count,
+                     g_counter, info);
+  FLA_HIP_CHECK(hipGetLastError());
+  return FLA_HIP_OK;
 }
 
-// Panel widths: 16 or 32 for the Cholesky kinds, 16 for the LU (wider LU
-// panels spill registers and measured slower).
+// Panel widths: 16 for the LU (wider panels spill registers and measured
+// slower); the Cholesky kernel works in 16-column blocks under both accepted
+// values.
 bool valid_nb(int kind, int nb) {
   if (kind == kDgetrf) return nb == 16;
   return nb == 16 || nb == 32;
 }
 
-// Workgroups per CU that the panel's LDS allows (at most 4).
+// Most workgroups per CU worth a try (at most 4): those a 32- or 16-column
+// panel of the largest matrix in LDS allows.
 int max_wg_per_cu(int kind, int nb) {
   const int bytes = (MAXN + 32) * nb * (kind == kSpotrf ? 4 : 8) + 1024;
   return std::max(1, std::min(4, (160 * 1024) / bytes));
@@ -1260,13 +1071,11 @@ extern "C" int fla_hip_batched_tune(int kind, int count, const int* n, const int
     Pp[i] = ipiv_base + (size_t)i * MAXN;
   }
   std::vector<BatchConfig> cands;
-  for (int nb : (kind == kDgetrf ? std::vector<int>{16} : std::vector<int>{16, 32}))
-    for (int wg = 1; wg <= max_wg_per_cu(kind, nb); wg *= 2) {
-      BatchConfig c;
-      c.nb = nb;
-      c.wg_per_cu = wg;
-      cands.push_back(c);
-    }
+  for (int wg = 1; wg <= max_wg_per_cu(kind, BatchConfig().nb); wg *= 2) {
+    BatchConfig c;
+    c.wg_per_cu = wg;
+    cands.push_back(c);
+  }
   hipEvent_t e0, e1;
   FLA_HIP_CHECK(hipEventCreate(&e0));
   FLA_HIP_CHECK(hipEventCreate(&e1));

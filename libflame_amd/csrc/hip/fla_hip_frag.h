@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 namespace fla_frag {
 
 constexpr int FB = 128;        // order of a triangular block
@@ -12,6 +14,19 @@ constexpr int NT16 = FB / 16;  // its 16-blocks per side
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ double readlane_d(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Barrier that orders LDS accesses only: __syncthreads would also wait for
+// the global stores in flight.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
 
 // 16 x 16 blocks in fragment order.  v_mfma_f64_16x16x4f64 leaves D(x, y) in
 // lane 16*(x%4) + y, register x/4; with x the column and y the row of a
@@ -138,6 +153,145 @@ __device__ __forceinline__ void solve_rows(const d2* __restrict__ W, d4 (&c)[NT1
     done(jb);
     __builtin_amdgcn_sched_barrier(0);
   }
+}
+
+// One wave factors a 16 x 16 symmetric block.  Lane li of each row of 16 lanes
+// holds row li (x[c] = a(li, c)).  Column j: d = sqrt(a_jj), x_j *= 1/d, then
+// x_c -= x_j l_cj, with l_cj broadcast from lane c by the update instruction
+// itself (DPP row_newbcast).  (Through lane reads the pivot alone took 80
+// cycles from its update to its first use, and every multiplier two reads.)
+// A VALU result is a DPP source only two wait states later: the statements
+// below keep other instructions in between, or carry the s_nop.
+template <int C>
+__device__ __forceinline__ void sweep_update(double& x, double xs, double nx) {
+  asm volatile("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+               : "+v"(x)
+               : "v"(xs), "v"(nx), "i"(C));
+}
+// Updates of the columns C0 <= C < C1 (none past 15).
+template <int C0, int C1>
+__device__ __forceinline__ void sweep_updates(double (&x)[16], double xs, double nx) {
+  if constexpr (C0 < C1 && C0 < 16) {
+    sweep_update<C0>(x[C0], xs, nx);
+    sweep_updates<C0 + 1, C1>(x, xs, nx);
+  }
+}
+template <int J>
+__device__ __forceinline__ double bcast16(double x) {
+  double a;
+  asm volatile("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+               : "=v"(a)
+               : "v"(x), "i"(J));
+  return a;
+}
+
+// Column J with the pivot a already broadcast.  The root by Goldschmidt's
+// iteration from v_rsq_f64 (g -> sqrt(a), h -> 1/(2 sqrt(a))) and a residual
+// correction, the reciprocal by a Newton step against the rounded root
+// (Markstein): exact roots and reciprocals come out exact, as the reference's
+// sqrt and division give them.  The updates of column J - 1 right of column J
+// (xsp, nxp) fill the chain's latencies; column J + 1 is updated first, so
+// that the next pivot is on its way at the end.  piv, pinv: lane J's root and
+// reciprocal.
+template <int J>
+__device__ __forceinline__ void sweep_column(double (&x)[16], int li, double& piv, double& pinv,
+                                             double& a, double& xsp, double& nxp) {
+  constexpr int N = J > 0 ? 15 - J : 0, C1 = J + 1 + (N + 2) / 3, C2 = J + 1 + (2 * N + 2) / 3;
+  const double y = __builtin_amdgcn_rsq(a);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (J > 0) sweep_updates<J + 1, C1>(x, xsp, nxp);
+  __builtin_amdgcn_sched_barrier(0);
+  double g = a * y, h = 0.5 * y;
+  double e = fma(-h, g, 0.5);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (J > 0) sweep_updates<C1, C2>(x, xsp, nxp);
+  __builtin_amdgcn_sched_barrier(0);
+  h = fma(h, e, h);
+  g = fma(g, e, g);
+  e = fma(-g, g, a);
+  const double h2 = h + h;
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (J > 0) sweep_updates<C2, 16>(x, xsp, nxp);
+  __builtin_amdgcn_sched_barrier(0);
+  const double d = fma(e, h, g);
+  const double inv = fma(fma(-d, h2, 1.0), h2, h2);
+  xsp = x[J] * inv;
+  nxp = -xsp;
+  asm volatile("s_nop 1" : "+v"(xsp));
+  if constexpr (J < 15) {
+    sweep_update<J + 1>(x[J + 1], xsp, nxp);
+    a = bcast16<J + 1>(x[J + 1]);
+  }
+  x[J] = li == J ? d : xsp;
+  piv = li == J ? d : piv;
+  pinv = li == J ? inv : pinv;
+}
+template <int... J>
+__device__ __forceinline__ void sweep16(double (&x)[16], int li, double& piv, double& pinv,
+                                        std::integer_sequence<int, J...>) {
+  double a = bcast16<0>(x[0]), xsp = 0.0, nxp = 0.0;
+  (sweep_column<J>(x, li, piv, pinv, a, xsp, nxp), ...);
+}
+
+// A factored 16 x 16 diagonal block in LDS: rows 0..15 hold L (below and on
+// the diagonal), row 16 the reciprocals of its diagonal.  The row length keeps
+// 16-byte accesses aligned and spreads the rows over the banks.
+constexpr int ZLD = 18;
+
+// The sweep with the library's root and division, any pivot range, in place
+// in LDS (rare: it takes no registers from the fast one); returns the first
+// column whose pivot is <= 0 or NaN (bl1_dsqrte's rule), else -1.
+__device__ __forceinline__ int sweep16_any(double* z, int lane) {
+  const int li = lane & 15;
+  int f = -1;
+#pragma unroll 1
+  for (int j = 0; j < 16; ++j) {
+    const double a = z[j * ZLD + j];
+    if (f < 0 && !(a > 0.0)) f = j;
+    const double d = sqrt(a), inv = 1.0 / d;
+    const double xs = z[li * ZLD + j] * inv;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (lane < 16) {
+      if (li > j) z[li * ZLD + j] = xs;
+      if (li == j) {
+        z[j * ZLD + j] = d;
+        z[16 * ZLD + j] = inv;
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll 1
+    for (int c = j + 1; c < 16; ++c)
+      if (lane < 16 && li >= c) z[li * ZLD + c] = fma(-xs, z[c * ZLD + j], z[li * ZLD + c]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  return __builtin_amdgcn_readfirstlane(f);
+}
+
+// Factors the symmetric block dg (fragment order) into z, one wave.  Returns
+// the first failing column or -1.  Pivots outside [2^-700, 2^1000] (products
+// of the fast sweep could under- or overflow) and failing ones take the
+// general sweep.
+__device__ __forceinline__ int factor16(d4 dg, double* z, int lane) {
+  const int li = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) z[li * ZLD + lk + 4 * r] = dg[r];
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  double x[16], piv = 0.0, pinv = 0.0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const d2 v = *reinterpret_cast<const d2*>(z + li * ZLD + 2 * q);
+    x[2 * q] = v.x;
+    x[2 * q + 1] = v.y;
+  }
+  sweep16(x, li, piv, pinv, std::make_integer_sequence<int, 16>{});
+  if (!__all(piv >= 0x1p-350 && piv <= 0x1p500)) return sweep16_any(z, lane);
+  if (lane < 16) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      *reinterpret_cast<d2*>(z + lane * ZLD + 2 * q) = d2{x[2 * q], x[2 * q + 1]};
+    z[16 * ZLD + lane] = pinv;
+  }
+  return -1;
 }
 
 }  // namespace fla_frag

@@ -1,0 +1,84 @@
+"""The left-looking batched Cholesky and solve where it can go wrong: orders
+around the 16-row blocks and the eight waves' turns, leading dimensions larger
+than the order, right-hand-side counts around 16, and failing columns.  Exact
+integer systems: factors and solutions must come out bit for bit."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import libflame_amd as fla
+from tests.cases import exact_spd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    fla.FLA_Init()
+    yield
+
+
+def _run(dtype, mats, rhs, pad):
+    cnt = len(mats)
+    dA, dB = [], []
+    for a, b in zip(mats, rhs):
+        n = a.shape[0]
+        A = np.full((n + pad, n), 77.0, order="F")
+        A[:n] = a
+        B = np.full((n + pad, b.shape[1]), 55.0, order="F")
+        B[:n] = b
+        dA.append(fla.DeviceMatrix.from_host(A, dtype))
+        dB.append(fla.DeviceMatrix.from_host(B, dtype))
+    ptr = lambda v: (C.c_void_p * cnt)(*[x.ptr.value for x in v])  # noqa: E731
+    ints = lambda v: (C.c_int * cnt)(*[int(x) for x in v])  # noqa: E731
+    info = fla.DeviceMatrix(cnt, 1, np.int32)
+    L = fla.lib()
+    f = L.fla_hip_dposv_batched if dtype == np.float64 else L.fla_hip_sposv_batched
+    fla.check(f(C.c_int(cnt), ints([a.shape[0] for a in mats]), ptr(dA), ints([d.ld for d in dA]),
+                ptr(dB), ints([d.ld for d in dB]), ints([b.shape[1] for b in rhs]), info.ptr))
+    fla.synchronize()
+    return [d.download() for d in dA], [d.download() for d in dB], info.download().ravel()
+
+
+def _spd(n, seed):
+    """A sparse closed form, so that FP32 stays exact and solutions small."""
+    _, F = exact_spd(n, seed)
+    keep = np.random.default_rng(seed).random((n, n)) < 0.06
+    F = np.where(keep | np.eye(n, dtype=bool), F, 0.0)
+    return F @ F.T, F
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("pad", [0, 3])
+def test_exact(dtype, pad):
+    ns = [1, 15, 16, 17, 31, 33, 48, 49, 127, 128, 129, 143, 145, 257, 497, 511, 512]
+    rs = [1, 2, 8, 15, 16, 17, 31, 33, 40]
+    mats, facs, xs = [], [], []
+    for i, n in enumerate(ns):
+        A, F = _spd(n, n + 1)
+        mats.append(A)
+        facs.append(F)
+        # only a few nonzeros: the triangular systems' intermediate values stay small
+        X = np.zeros((n, rs[i % len(rs)]))
+        X[:: max(1, n // 5)] = np.random.default_rng(n).integers(-2, 3, size=X[:: max(1, n // 5)].shape)
+        xs.append(X)
+    out, sol, info = _run(dtype, mats, [a @ x for a, x in zip(mats, xs)], pad)
+    assert np.all(info == fla.FLA_SUCCESS)
+    for n, A, F, X, o, s in zip(ns, mats, facs, xs, out, sol):
+        assert np.array_equal(np.tril(o[:n]), F), n
+        assert np.array_equal(np.triu(o[:n], 1), np.triu(A, 1)), n
+        assert np.all(o[n:] == 77.0) and np.all(s[n:] == 55.0), n
+        assert np.array_equal(s[:n], X), n
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_failing_column(dtype):
+    cols = [0, 5, 15, 16, 31, 47, 100]
+    mats = []
+    for k in cols:
+        A, F = _spd(101, 7)
+        A[k, k] -= F[k, k] ** 2 + 1.0
+        mats.append(A)
+    _, _, info = _run(dtype, mats, [np.ones((101, 2))] * len(cols), 0)
+    assert list(info) == cols

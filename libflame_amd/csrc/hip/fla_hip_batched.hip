@@ -736,7 +736,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
 // ms on the batch below), two in FP32.  Bound: the chain of a matrix's block
 // columns (diagonal factor, substitution, memory round trips) with eight or
 // sixteen waves a CU.  4096 matrices of n ~ U{32..512} with 1-8 right-hand
-// sides, with the copies in: FP64 10.4 -> 6.4 ms, FP32 6.1 -> 3.6 ms against a
+// sides, with the copies in: FP64 10.4 -> 6.5 ms, FP32 6.1 -> 3.6 ms against a
 // right-looking kernel of 16-column panels in LDS.
 template <typename T>
 __global__ __launch_bounds__(64 * fla_posv::NW, sizeof(T) == 8 ? 2 : 4) void posv_kernel(

@@ -898,7 +898,8 @@ int stage_items(int count, const int* n, void* const* A, const int* lda, int* co
     it.n = n[i];
     it.index = i;
     it.ipiv = need_ipiv ? ipiv[i] : nullptr;
-    const int r = (B && nrhs) ? nrhs[i] : 0;
+    // the kernels take right-hand sides of a matrix with rows, and a count >= 0
+    const int r = (B && nrhs && n[i] > 0) ? std::max(0, nrhs[i]) : 0;
     it.nrhs = r;
     it.B = r > 0 ? B[i] : nullptr;
     it.ldb = r > 0 ? ldb[i] : 1;

@@ -176,7 +176,8 @@ struct Row {
 };
 
 // Factor (lower) of the n x n A and, with nrhs > 0, B := inv(A) B.  Returns
-// the first failing column or -1.
+// the first failing column or -1.  n >= 1, or n = 0 and nrhs = 0 (the staging
+// of the items sees to it).
 template <typename T>
 __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<T>& S, int t) {
   typedef typename Frag<T>::V V;

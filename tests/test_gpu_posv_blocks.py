@@ -82,3 +82,29 @@ def test_failing_column(dtype):
         mats.append(A)
     _, _, info = _run(dtype, mats, [np.ones((101, 2))] * len(cols), 0)
     assert list(info) == cols
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_empty_matrices_and_negative_counts(dtype):
+    """An item of order 0 touches nothing, whatever its matrix pointer and
+    right-hand-side count; a negative count is no right-hand sides."""
+    A, F = _spd(40, 7)
+    X = np.full((40, 2), 3.0)
+    ns, rs = [40, 0, 40, 0], [2, 5, -40, 1]
+    dA = [fla.DeviceMatrix.from_host(np.asfortranarray(A), dtype) for _ in ns]
+    dB = [fla.DeviceMatrix.from_host(np.asfortranarray(A @ X), dtype) for _ in ns]
+    pA = (C.c_void_p * 4)(dA[0].ptr.value, None, dA[2].ptr.value, dA[3].ptr.value)
+    pB = (C.c_void_p * 4)(*[b.ptr.value for b in dB])
+    ints = lambda v: (C.c_int * 4)(*v)  # noqa: E731
+    info = fla.DeviceMatrix(4, 1, np.int32)
+    L = fla.lib()
+    f = L.fla_hip_dposv_batched if dtype == np.float64 else L.fla_hip_sposv_batched
+    fla.check(f(C.c_int(4), ints(ns), pA, ints([40] * 4), pB, ints([40] * 4), ints(rs), info.ptr))
+    fla.synchronize()
+    assert np.all(info.download() == fla.FLA_SUCCESS)
+    assert np.array_equal(np.tril(dA[0].download()), F)
+    assert np.array_equal(np.tril(dA[2].download()), F)
+    assert np.array_equal(dA[3].download(), A)
+    assert np.array_equal(dB[0].download(), X)
+    for q in (1, 2, 3):
+        assert np.array_equal(dB[q].download(), A @ X), q

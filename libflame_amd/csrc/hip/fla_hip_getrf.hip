@@ -484,13 +484,15 @@ __global__ __launch_bounds__(NT, 2) void lu_sub_kernel(int M, int W, double* __r
         l[0] = lane > j ? l[0] : x[0];
       }
       if (select) {
+        // the whole update of this wave's rows; what follows then adds zeros
 #pragma unroll
         for (int c = 0; c < SW; ++c) {
-          const double y = fma(-l[0], u[c], v[0][c]);
-          if (c > pos && c < 8 * nlive && lane > j) v[0][c] = y;
-          if (c == pos + 1) x[0] = v[0][c];
+          const bool live = c > pos && c < 8 * nlive;
+          const double y0 = fma(nl[0], u[c], v[0][c]), y1 = fma(nl[1], u[c], v[1][c]);
+          if (live && lane > j) v[0][c] = y0;
+          if (live) v[1][c] = y1;
         }
-        nl[0] = 0.0;
+        nl[0] = nl[1] = 0.0;
         u0 = fabs(u0) < __builtin_inf() ? u0 : 0.0;
         u1 = fabs(u1) < __builtin_inf() ? u1 : 0.0;
       }

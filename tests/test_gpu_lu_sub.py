@@ -51,3 +51,20 @@ def test_infinite_row_keeps_finished_rows(orc, m):
     assert np.array_equal(np.isfinite(out[:, :c]), np.isfinite(ref[:, :c]))
     k = next(i for i in range(n) if not np.isfinite(ref[i, c]))
     assert np.all(np.isfinite(out[:k, :]))
+
+
+@pytest.mark.parametrize("m", [600, 1500])
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+def test_non_finite_pivot_row_reaches_every_row(orc, m, value):
+    """A pivot row holding an infinity or NaN updates every row below it, those
+    of a thread's second register row (512 and up) too, and the pivots chosen
+    from them follow."""
+    n, c = 32, 9
+    A = np.asfortranarray(orc.gen_lu_c2(5, m, n))
+    A[0, 0] = 8.0  # the first pivot
+    A[0, c] = value
+    out, pv, _ = gpu_lu(A)
+    ref, pref, _ = orc.lu_piv(A)
+    assert np.array_equal(pv, pref)
+    assert np.array_equal(np.isfinite(out), np.isfinite(ref))
+    assert np.array_equal(np.isnan(out), np.isnan(ref))

@@ -83,14 +83,11 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
         l[s] = -z[li * ZLD + cc];  // above the diagonal never used
         cf[s][0] = z[16 * ZLD + cc];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) {
-          const double v = z[cc * ZLD + 4 * s + q];
-          cf[s][1 + q] = lk > q ? -v : 0.0;
-        }
+        for (int q = 0; q < 3; ++q) cf[s][1 + q] = -z[cc * ZLD + 4 * s + q];
       }
       d4 cur = c[0];
       if (b > 0) cur = mfma_block(Xf[par ^ 1][b][0][lane], Xf[par ^ 1][b][1][lane], xr, cur);
-      const d4 xn = solve_block(l, cf, cur, li, lk);
+      const d4 xn = solve_block(l, cf, cur, lk);
       const d2 n0 = d2{-xn[0], -xn[1]}, n1 = d2{-xn[2], -xn[3]};
       Xf[par][w][0][lane] = n0;
       Xf[par][w][1][lane] = n1;

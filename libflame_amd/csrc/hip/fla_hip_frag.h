@@ -63,23 +63,33 @@ __device__ __forceinline__ double row_to_all(double x) {
 // order (x_j *= 1/l_jj, then t_c -= x_j l_cj).  The four columns 4r..4r+3 sit
 // in register r of the four rows of 16 lanes: within them the solved column
 // is copied across the rows, then one matrix step updates the later columns.
-// l: -L; cf[r]: of the lane's column c = lk + 4r the reciprocal 1/l_cc and
-// -l_cj for j = 4r..4r+2 (0 where c <= j).  About 1100 cycles; a matrix step
-// per column, whose result has to come back through the vector unit each
-// time, took 3200.
-__device__ __forceinline__ d4 solve_block(d4 l, const d4 (&cf)[4], d4 t, int li, int lk) {
+// Columns already solved are kept by selects and by taking only the matrix
+// step's later registers, not by zero multipliers: x_j may be infinite.
+// l: -L (any value on and above the diagonal); cf[r]: of the lane's column
+// c = lk + 4r the reciprocal 1/l_cc and -l_cj for j = 4r..4r+2 (any value
+// where c <= j).  About 1100 cycles; a
+// matrix step per column, whose result has to come back through the vector
+// unit each time, took 3200.
+__device__ __forceinline__ d4 solve_block(d4 l, const d4 (&cf)[4], d4 t, int lk) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    double x = t[r];
+    double x = t[r], y;
     x *= lk == 0 ? cf[r][0] : 1.0;
-    x = fma(cf[r][1], row_to_all<0>(x), x);
+    y = fma(cf[r][1], row_to_all<0>(x), x);
+    x = lk > 0 ? y : x;
     x *= lk == 1 ? cf[r][0] : 1.0;
-    x = fma(cf[r][2], row_to_all<1>(x), x);
+    y = fma(cf[r][2], row_to_all<1>(x), x);
+    x = lk > 1 ? y : x;
     x *= lk == 2 ? cf[r][0] : 1.0;
-    x = fma(cf[r][3], row_to_all<2>(x), x);
+    y = fma(cf[r][3], row_to_all<2>(x), x);
+    x = lk > 2 ? y : x;
     x *= lk == 3 ? cf[r][0] : 1.0;
     t[r] = x;
-    if (r < 3) t = mfma_step(li >= 4 * (r + 1) ? l[r] : 0.0, x, t);
+    if (r < 3) {
+      const d4 u = mfma_step(l[r], x, t);
+#pragma unroll
+      for (int q = r + 1; q < 4; ++q) t[q] = u[q];
+    }
   }
   return t;
 }
@@ -114,7 +124,7 @@ __device__ __forceinline__ void solve_rows(const d2* __restrict__ W, d4 (&c)[NT1
                                            F done) {
   constexpr int PF = 6;
   constexpr Stream kStream = make_stream();
-  const int li = lane & 15, lk = lane >> 4;
+  const int lk = lane >> 4;
   d2 ring[PF][2];
   d4 cf[4];
   const d2* const Wl = W + lane;
@@ -142,7 +152,7 @@ __device__ __forceinline__ void solve_rows(const d2* __restrict__ W, d4 (&c)[NT1
       if (k < jb)
         c[jb] = mfma_block(l0, l1, c[k], c[jb]);
       else
-        c[jb] = solve_block(d4{l0.x, l0.y, l1.x, l1.y}, cf, c[jb], li, lk);
+        c[jb] = solve_block(d4{l0.x, l0.y, l1.x, l1.y}, cf, c[jb], lk);
       if (q + PF < NQ) {
         ring[q % PF][0] = Wl[kStream.block[q + PF] * 128];
         ring[q % PF][1] = Wl[kStream.block[q + PF] * 128 + 64];

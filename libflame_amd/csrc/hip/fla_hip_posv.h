@@ -64,47 +64,47 @@ template <typename T>
 struct Tri {
   typename Frag<T>::V l, cf[4];
 };
-// at(i, j): L(i, j) for j < i; inv(i): 1 / L(i, i).
+// at(i, j): L(i, j) for j < i, any value for j >= i (never used); inv(i):
+// 1 / L(i, i).
 template <typename T, typename At, typename Inv>
 __device__ __forceinline__ void load_tri(Tri<T>& t, int li, int lk, At at, Inv inv) {
   constexpr bool D = sizeof(T) == 8;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int c = Frag<T>::col(lk, r);
-    t.l[r] = c < li ? -at(li, c) : (T)0;
+    t.l[r] = -at(li, c);
     t.cf[r][0] = inv(c);
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int j = (D ? 4 * r : 4 * lk) + q;
-      t.cf[r][1 + q] = j < c ? -at(c, j) : (T)0;
-    }
+    for (int q = 0; q < 3; ++q) t.cf[r][1 + q] = -at(c, (D ? 4 * r : 4 * lk) + q);
   }
 }
 
 // X := X inv(L)' by substitution (x_j *= 1/l_jj, then x_c -= x_j l_cj).
-__device__ __forceinline__ Frag<double>::V solve(const Tri<double>& t, Frag<double>::V x, int li,
+__device__ __forceinline__ Frag<double>::V solve(const Tri<double>& t, Frag<double>::V x,
                                                  int lk) {
-  return fla_frag::solve_block(t.l, t.cf, x, li, lk);
+  return fla_frag::solve_block(t.l, t.cf, x, lk);
 }
-__device__ __forceinline__ Frag<float>::V solve(const Tri<float>& t, Frag<float>::V x, int li,
-                                                int lk) {
+__device__ __forceinline__ Frag<float>::V solve(const Tri<float>& t, Frag<float>::V x, int lk) {
   // columns 4q..4q+3 sit in the registers of the lanes with lk == q: solved
-  // there, then four matrix steps with that k slot update the later columns
+  // there, then four matrix steps with that k slot (the others zero on both
+  // sides) update the later columns; the solved ones are kept as they are
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     const bool me = lk == q;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
+      float y = x[r];
 #pragma unroll
-      for (int p = 0; p < r; ++p) x[r] = fmaf(me ? t.cf[r][1 + p] : 0.0f, x[p], x[r]);
-      x[r] *= me ? t.cf[r][0] : 1.0f;
+      for (int p = 0; p < r; ++p) y = fmaf(t.cf[r][1 + p], x[p], y);
+      x[r] = me ? y * t.cf[r][0] : x[r];
     }
     if (q < 3) {
       Frag<float>::V y = x;
 #pragma unroll
       for (int s = 0; s < 4; ++s)
-        y = Frag<float>::step(me && li >= 4 * (q + 1) ? t.l[s] : 0.0f, x[s], y);
-      x = y;
+        y = Frag<float>::step(me ? t.l[s] : 0.0f, me ? x[s] : 0.0f, y);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) x[r] = lk > q ? y[r] : x[r];
     }
   }
   return x;
@@ -285,7 +285,7 @@ __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<
       if (i >= nb + nr) break;  // uniform
       if (i == b) continue;
       const Row<T> p = block_row(i);
-      const V x = solve(tri, acc[u], li, lk);
+      const V x = solve(tri, acc[u], lk);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (p.in && (!ragb || 16 * b + c0 + CS * r < n)) *p.at(b, r) = x[r];
@@ -336,7 +336,7 @@ __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<
         load_tri<T>(
             tri, li, lk, [&](int i, int j) { return S.z[par][i * ZLD + j]; },
             [&](int i) { return S.z[par][16 * ZLD + i]; });
-        x = solve(tri, x, li, lk);
+        x = solve(tri, x, lk);
         S.x[par][lane] = x;
 #pragma unroll
         for (int r = 0; r < 4; ++r)

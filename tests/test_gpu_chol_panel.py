@@ -41,3 +41,14 @@ def test_scaled_pivots_exact(n, e):
     out, r = gpu_chol(S)
     assert r == fla.FLA_SUCCESS
     assert np.array_equal(np.tril(out), np.ldexp(F, e))
+
+
+@pytest.mark.parametrize("n,i,j", [(100, 40, 9), (100, 40, 20), (300, 250, 5), (300, 250, 137)])
+def test_entries_before_an_infinity_stay(n, i, j):
+    """An infinity at (i, j) makes row i fail; what the row holds left of
+    column j is the factor's, in the same 16 columns too."""
+    A, F = exact_spd(n, seed=n)
+    A[i, j] = np.inf
+    out, r = gpu_chol(A)
+    assert r == i
+    assert np.array_equal(out[i, :j], F[i, :j])

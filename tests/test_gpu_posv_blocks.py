@@ -108,3 +108,20 @@ def test_empty_matrices_and_negative_counts(dtype):
     assert np.array_equal(dB[0].download(), X)
     for q in (1, 2, 3):
         assert np.array_equal(dB[q].download(), A @ X), q
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_entries_before_an_infinity_stay(dtype):
+    """An infinity at (i, j) makes row i fail; what the row holds left of
+    column j is the factor's, in the same 16 columns too."""
+    at = [(40, 9), (40, 20), (95, 3), (99, 70)]
+    A, F = _spd(101, 7)
+    mats = []
+    for i, j in at:
+        M = A.copy()
+        M[i, j] = np.inf
+        mats.append(M)
+    out, _, info = _run(dtype, mats, [np.ones((101, 2))] * len(at), 0)
+    assert list(info) == [i for i, _ in at]
+    for (i, j), o in zip(at, out):
+        assert np.array_equal(o[i, :j], F[i, :j]), (i, j)

@@ -39,3 +39,58 @@ def test_exact(n, nrhs, left, lower, trans):
                    fla.FLA_TRANSPOSE if trans else fla.FLA_NO_TRANSPOSE,
                    fla.FLA_UNIT_DIAG if unit else fla.FLA_NONUNIT_DIAG, S, B.astype(np.float64))
     assert np.array_equal(out, X)
+
+
+def _reference(T, B, left, lower, trans, unit):
+    """dtrsm_'s substitution, one component at a time."""
+    op = T.T if trans else T
+    M, X = (op, B.copy()) if left else (op.T, B.T.copy())  # M X = B
+    n = M.shape[0]
+    fwd = lower != trans if left else lower == trans
+    with np.errstate(divide="ignore", invalid="ignore"):
+        for j in range(n) if fwd else range(n - 1, -1, -1):
+            if not unit:
+                X[j] /= M[j, j]
+            rest = slice(j + 1, n) if fwd else slice(0, j)
+            X[rest] -= np.outer(M[rest, j], X[j])
+    return X if left else X.T
+
+
+def _solve(T, B, left, lower, trans, unit=False):
+    return gpu_trsm(fla.FLA_LEFT if left else fla.FLA_RIGHT,
+                    fla.FLA_LOWER_TRIANGULAR if lower else fla.FLA_UPPER_TRIANGULAR,
+                    fla.FLA_TRANSPOSE if trans else fla.FLA_NO_TRANSPOSE,
+                    fla.FLA_UNIT_DIAG if unit else fla.FLA_NONUNIT_DIAG, T, B)
+
+
+def _sparse_tri(n, lower):
+    T = exact_tri(n, seed=n, lower=lower)
+    return np.where(np.eye(n, dtype=bool) | (np.random.default_rng(n).random((n, n)) < 0.05), T, 0.0)
+
+
+@pytest.mark.parametrize("at", [3, 9, 137])
+@pytest.mark.parametrize("what", ["diagonal", "rhs"])
+@pytest.mark.parametrize("left", [True, False])
+@pytest.mark.parametrize("lower", [True, False])
+@pytest.mark.parametrize("trans", [True, False])
+def test_components_before_an_infinity_stay(at, what, left, lower, trans):
+    """A zero on the diagonal or an infinite right-hand side at the at-th
+    component solved changes that one and the later ones only."""
+    n, nrhs = 200, 40
+    T = _sparse_tri(n, lower)
+    fwd = lower != trans if left else lower == trans
+    j = at if fwd else n - 1 - at
+    B = np.random.default_rng(at).integers(1, 5, size=(n, nrhs) if left else (nrhs, n)).astype(float)
+    if what == "diagonal":
+        T[j, j] = 0.0
+    elif left:
+        B[j, :] = np.inf
+    else:
+        B[:, j] = np.inf
+    ref = _reference(T, B, left, lower, trans, False)
+    out = _solve(T, B, left, lower, trans)
+    done = [k if fwd else n - 1 - k for k in range(at)]
+    ahead = ref[done] if left else ref[:, done]
+    assert np.all(np.isfinite(ahead))
+    assert np.array_equal(out[done] if left else out[:, done], ahead)
+    assert np.array_equal(np.isfinite(out), np.isfinite(ref))

@@ -53,13 +53,15 @@ def test_infinite_row_keeps_finished_rows(orc, m):
     assert np.all(np.isfinite(out[:k, :]))
 
 
-@pytest.mark.parametrize("m", [600, 1500])
+@pytest.mark.parametrize("m", [560, 600, 1500])
 @pytest.mark.parametrize("value", [np.inf, np.nan])
-def test_non_finite_pivot_row_reaches_every_row(orc, m, value):
+@pytest.mark.parametrize("c", [1, 9])
+def test_non_finite_pivot_row_reaches_every_row(orc, m, value, c):
     """A pivot row holding an infinity or NaN updates every row below it, those
     of a thread's second register row (512 and up) too, and the pivots chosen
-    from them follow."""
-    n, c = 32, 9
+    from them follow (in the next column a finite row among NaNs would be
+    chosen, or be scaled to zero by an infinite pivot)."""
+    n = 32
     A = np.asfortranarray(orc.gen_lu_c2(5, m, n))
     A[0, 0] = 8.0  # the first pivot
     A[0, c] = value

@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void trsm_rlt_kernel(int m, const d2* __res
   for (int k = 0; k < NT16; ++k)
 #pragma unroll
     for (int r = 0; r < 4; ++r) c[k][r] = xp[(long)(16 * k + 4 * r) * ldx];
-  solve_rows(W, c, lane, [&](int jb) {
+  solve_rows<ByReciprocal>(W, c, lane, [&](int jb) {
     if (in) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) xp[(long)(16 * jb + 4 * r) * ldx] = c[jb][r];

@@ -59,31 +59,46 @@ __device__ __forceinline__ double row_to_all(double x) {
                           (int)row_to_all<Q>((unsigned)__double2loint(x)));
 }
 
+// What a substitution does with the diagonal entry of the lane's column when
+// that column's turn comes (me); the other columns keep their value.
+// Multiplies by the reciprocal c (dtrsm_ from the right, dpotrf_).
+struct ByReciprocal {
+  static __device__ __forceinline__ double apply(double x, double c, bool me) {
+    return x * (me ? c : 1.0);
+  }
+};
+// Divides by the diagonal entry c (dtrsm_ from the left).
+struct ByDivision {
+  static __device__ __forceinline__ double apply(double x, double c, bool me) {
+    return x / (me ? c : 1.0);
+  }
+};
+
 // X := T inv(L)' for a block T by substitution, dtrsm_'s operations in its
-// order (x_j *= 1/l_jj, then t_c -= x_j l_cj).  The four columns 4r..4r+3 sit
-// in register r of the four rows of 16 lanes: within them the solved column
-// is copied across the rows, then one matrix step updates the later columns.
-// Columns already solved are kept by selects and by taking only the matrix
-// step's later registers, not by zero multipliers: x_j may be infinite.
-// l: -L (any value on and above the diagonal); cf[r]: of the lane's column
-// c = lk + 4r the reciprocal 1/l_cc and -l_cj for j = 4r..4r+2 (any value
-// where c <= j).  About 1100 cycles; a
-// matrix step per column, whose result has to come back through the vector
-// unit each time, took 3200.
+// order (x_j *= 1/l_jj or x_j /= l_jj, then t_c -= x_j l_cj).  The four
+// columns 4r..4r+3 sit in register r of the four rows of 16 lanes: within them
+// the solved column is copied across the rows, then one matrix step updates
+// the later columns.  Columns already solved are kept by selects and by taking
+// only the matrix step's later registers, not by zero multipliers: x_j may be
+// infinite.  l: -L (any value on and above the diagonal); cf[r]: of the lane's
+// column c = lk + 4r what SCALE takes and -l_cj for j = 4r..4r+2 (any value
+// where c <= j).  About 1100 cycles with reciprocals; a matrix step per column,
+// whose result has to come back through the vector unit each time, took 3200.
+template <typename SCALE = ByReciprocal>
 __device__ __forceinline__ d4 solve_block(d4 l, const d4 (&cf)[4], d4 t, int lk) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     double x = t[r], y;
-    x *= lk == 0 ? cf[r][0] : 1.0;
+    x = SCALE::apply(x, cf[r][0], lk == 0);
     y = fma(cf[r][1], row_to_all<0>(x), x);
     x = lk > 0 ? y : x;
-    x *= lk == 1 ? cf[r][0] : 1.0;
+    x = SCALE::apply(x, cf[r][0], lk == 1);
     y = fma(cf[r][2], row_to_all<1>(x), x);
     x = lk > 1 ? y : x;
-    x *= lk == 2 ? cf[r][0] : 1.0;
+    x = SCALE::apply(x, cf[r][0], lk == 2);
     y = fma(cf[r][3], row_to_all<2>(x), x);
     x = lk > 2 ? y : x;
-    x *= lk == 3 ? cf[r][0] : 1.0;
+    x = SCALE::apply(x, cf[r][0], lk == 3);
     t[r] = x;
     if (r < 3) {
       const d4 u = mfma_step(l[r], x, t);
@@ -119,7 +134,7 @@ constexpr Stream make_stream() {
 // the 128 columns and is overwritten by c inv(L)'; W: L's blocks.  They are
 // read PF blocks ahead of their use (88 KB, shared by every wave through the
 // caches); done(jb) is called when column block jb is final.
-template <typename F>
+template <typename SCALE, typename F>
 __device__ __forceinline__ void solve_rows(const d2* __restrict__ W, d4 (&c)[NT16], int lane,
                                            F done) {
   constexpr int PF = 6;
@@ -152,7 +167,7 @@ __device__ __forceinline__ void solve_rows(const d2* __restrict__ W, d4 (&c)[NT1
       if (k < jb)
         c[jb] = mfma_block(l0, l1, c[k], c[jb]);
       else
-        c[jb] = solve_block(d4{l0.x, l0.y, l1.x, l1.y}, cf, c[jb], lk);
+        c[jb] = solve_block<SCALE>(d4{l0.x, l0.y, l1.x, l1.y}, cf, c[jb], lk);
       if (q + PF < NQ) {
         ring[q % PF][0] = Wl[kStream.block[q + PF] * 128];
         ring[q % PF][1] = Wl[kStream.block[q + PF] * 128 + 64];

@@ -8,10 +8,12 @@
 // (the right-hand sides are the rows), and a descending one has its indices
 // reversed.  One launch per solve writes the diagonal blocks in that form and
 // in the order the solve reads them; one wave then solves 16 right-hand sides
-// by substitution (dtrsm_'s update order, the reciprocal of the diagonal
-// multiplied in).
+// by substitution (dtrsm_'s update order; its division by the diagonal from the
+// left, its multiplication by the reciprocal from the right).
 #include "fla_hip_frag.h"
 #include "fla_hip_internal.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -24,10 +26,11 @@ constexpr int kGroup = 4;
 
 // Diagonal block kb = blockIdx.x of the triangle A: L(i, j) = U(j, i) for
 // ascending solves x U = b (U upper), reversed otherwise; U(k, c) =
-// swap ? A(c, k) : A(k, c).  Identity beyond the block's order.
+// swap ? A(c, k) : A(k, c).  Identity beyond the block's order.  recip: the
+// diagonal's reciprocals among the coefficients, else the diagonal.
 __global__ __launch_bounds__(512) void pack_blocks_kernel(int n, const double* __restrict__ A,
                                                           long lda, int swap, int rev, int unit,
-                                                          double* __restrict__ W) {
+                                                          int recip, double* __restrict__ W) {
   __shared__ double S[FB * (FB + 1)];  // A's block: (i, j) at S[j * (FB + 1) + i]
   const int r0 = blockIdx.x * FB, nb = min(FB, n - r0);
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -65,7 +68,7 @@ __global__ __launch_bounds__(512) void pack_blocks_kernel(int n, const double* _
   const int r = lane & 12, q = (lane & 3) - 1, c = 16 * w + lk + r;
   double v = 0.0;
   if (q < 0)
-    v = 1.0 / at(c, c);
+    v = recip ? 1.0 / at(c, c) : at(c, c);
   else if (lk > q)
     v = -at(c, 16 * w + r + q);
   Wk[(long)(frag_q0(w) + w + 1) * 256 + lane] = v;
@@ -98,7 +101,8 @@ __global__ __launch_bounds__(256, 2) void solve_block_kernel(int nrhs, int nb, i
       const double v = bp[(j < 0 ? 0 : j) * cs];
       c[k][r] = j < 0 ? 0.0 : v;
     }
-  solve_rows(W, c, lane, [&](int jb) {
+  // dtrsm_ divides from the left and multiplies by the reciprocal from the right
+  solve_rows<std::conditional_t<LEFT, ByDivision, ByReciprocal>>(W, c, lane, [&](int jb) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int j = col(jb, r);
@@ -117,7 +121,7 @@ int trsm_wide(hipStream_t s, bool left, bool upper, bool tr, bool unit, int m, i
   const bool fwd = left ? op_lower : !op_lower;
   const int swap = left ? !tr : tr;
   hipLaunchKernelGGL(pack_blocks_kernel, dim3((unsigned)nblk), dim3(512), 0, s, na, A, lda, swap,
-                     fwd ? 0 : 1, unit ? 1 : 0, W);
+                     fwd ? 0 : 1, unit ? 1 : 0, left ? 0 : 1, W);
   FLA_HIP_CHECK(hipGetLastError());
   // B[lo:hi) -= its product with the solved part [c0, c0 + k) of the triangle
   auto update = [&](int lo, int hi, int c0, int k) -> int {

@@ -94,3 +94,24 @@ def test_components_before_an_infinity_stay(at, what, left, lower, trans):
     assert np.all(np.isfinite(ahead))
     assert np.array_equal(out[done] if left else out[:, done], ahead)
     assert np.array_equal(np.isfinite(out), np.isfinite(ref))
+
+
+@pytest.mark.parametrize("lower", [True, False])
+@pytest.mark.parametrize("trans", [True, False])
+def test_left_solves_divide(lower, trans):
+    """Exact quotients of a solve from the left come out exactly whatever the
+    diagonal: by odd integers (49 (1/49) is not 1), by subnormal numbers
+    (their reciprocals overflow) and by those whose reciprocals are subnormal."""
+    n, nrhs = 150, 40
+    rng = np.random.default_rng(n)
+    T = _sparse_tri(n, lower)
+    np.fill_diagonal(T, rng.choice([3.0, 49.0, 98.0, 103.0, -107.0], size=n))
+    X = rng.integers(-4, 5, size=(n, nrhs)).astype(np.float64)
+    out = _solve(T, (T.T if trans else T) @ X, True, lower, trans)
+    assert np.array_equal(out, X)
+    d = rng.choice([3 * 2.0**-1040, -7 * 2.0**-1060, 1.75 * 2.0**1023, 49.0], size=n)
+    X = np.where(abs(d) < 1e-300, 2.0**40, 0.25)[:, None] * rng.integers(1, 4, size=(n, nrhs))
+    B = d[:, None] * X
+    assert np.array_equal(B / d[:, None], X) and np.all(np.isfinite(B))
+    out = _solve(np.diag(d), B, True, lower, trans)
+    assert np.array_equal(out, X)

@@ -60,17 +60,36 @@ __device__ __forceinline__ double row_to_all(double x) {
 }
 
 // What a substitution does with the diagonal entry of the lane's column when
-// that column's turn comes (me); the other columns keep their value.
+// that column's turn comes (me); the other columns keep their value.  c and d:
+// the column's coefficients.
 // Multiplies by the reciprocal c (dtrsm_ from the right, dpotrf_).
 struct ByReciprocal {
-  static __device__ __forceinline__ double apply(double x, double c, bool me) {
+  static __device__ __forceinline__ double apply(double x, double c, double, bool me) {
     return x * (me ? c : 1.0);
   }
 };
 // Divides by the diagonal entry c (dtrsm_ from the left).
 struct ByDivision {
-  static __device__ __forceinline__ double apply(double x, double c, bool me) {
+  static __device__ __forceinline__ double apply(double x, double c, double, bool me) {
     return x / (me ? c : 1.0);
+  }
+};
+// The quotient x / d from c = 1 / d rounded, where neither is subnormal: the
+// product corrected by its residual, which rounds correctly (Markstein).  Of an
+// infinite or NaN product the residual is NaN or infinite; held finite, it
+// leaves the product as it is.
+__device__ __forceinline__ double quotient(double x, double c, double d) {
+  const double q = x * c, y = fma(fma(-d, q, x), c, q);
+  return fabs(q) < __builtin_inf() ? y : q;
+}
+__device__ __forceinline__ float quotient(float x, float c, float d) {
+  const float q = x * c;
+  return fmaf(__builtin_amdgcn_fmed3f(fmaf(-d, q, x), -0x1p126f, 0x1p126f), c, q);
+}
+struct ByQuotient {
+  static __device__ __forceinline__ double apply(double x, double c, double d, bool me) {
+    const double q = quotient(x, c, d);
+    return me ? q : x;
   }
 };
 
@@ -82,23 +101,25 @@ struct ByDivision {
 // only the matrix step's later registers, not by zero multipliers: x_j may be
 // infinite.  l: -L (any value on and above the diagonal); cf[r]: of the lane's
 // column c = lk + 4r what SCALE takes and -l_cj for j = 4r..4r+2 (any value
-// where c <= j).  About 1100 cycles with reciprocals; a matrix step per column,
+// where c <= j); d[r]: SCALE's second coefficient.  About 1100 cycles with
+// reciprocals; a matrix step per column,
 // whose result has to come back through the vector unit each time, took 3200.
 template <typename SCALE = ByReciprocal>
-__device__ __forceinline__ d4 solve_block(d4 l, const d4 (&cf)[4], d4 t, int lk) {
+__device__ __forceinline__ d4 solve_block(d4 l, const d4 (&cf)[4], d4 t, int lk,
+                                          d4 d = d4{}) {
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     double x = t[r], y;
-    x = SCALE::apply(x, cf[r][0], lk == 0);
+    x = SCALE::apply(x, cf[r][0], d[r], lk == 0);
     y = fma(cf[r][1], row_to_all<0>(x), x);
     x = lk > 0 ? y : x;
-    x = SCALE::apply(x, cf[r][0], lk == 1);
+    x = SCALE::apply(x, cf[r][0], d[r], lk == 1);
     y = fma(cf[r][2], row_to_all<1>(x), x);
     x = lk > 1 ? y : x;
-    x = SCALE::apply(x, cf[r][0], lk == 2);
+    x = SCALE::apply(x, cf[r][0], d[r], lk == 2);
     y = fma(cf[r][3], row_to_all<2>(x), x);
     x = lk > 2 ? y : x;
-    x = SCALE::apply(x, cf[r][0], lk == 3);
+    x = SCALE::apply(x, cf[r][0], d[r], lk == 3);
     t[r] = x;
     if (r < 3) {
       const d4 u = mfma_step(l[r], x, t);

@@ -18,6 +18,8 @@
 
 #include "fla_hip_frag.h"
 
+#include <type_traits>
+
 namespace fla_posv {
 
 using fla_frag::lds_barrier;
@@ -46,6 +48,12 @@ struct Frag<float> {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(c, r, a, 0, 0, 0);
   }
 };
+// The steps' result with the wait states (10) that the vector unit needs before
+// it reads it: where only branches follow, the compiler can leave them out.
+__device__ __forceinline__ Frag<float>::V settled(Frag<float>::V a) {
+  asm("s_nop 9" : "+v"(a));
+  return a;
+}
 // acc + R C'
 template <typename T>
 __device__ __forceinline__ typename Frag<T>::V product(typename Frag<T>::V c, typename Frag<T>::V r,
@@ -78,13 +86,28 @@ __device__ __forceinline__ void load_tri(Tri<T>& t, int li, int lk, At at, Inv i
     for (int q = 0; q < 3; ++q) t.cf[r][1 + q] = -at(c, (D ? 4 * r : 4 * lk) + q);
   }
 }
-
-// X := X inv(L)' by substitution (x_j *= 1/l_jj, then x_c -= x_j l_cj).
-__device__ __forceinline__ Frag<double>::V solve(const Tri<double>& t, Frag<double>::V x,
-                                                 int lk) {
-  return fla_frag::solve_block(t.l, t.cf, x, lk);
+// Right-hand sides are divided by the diagonal (dtrsm_ from the left), rows of
+// the matrix multiplied by its reciprocal (dpotf2_).  The diagonal is a root,
+// so that it and its reciprocal are in the normal range.
+template <typename T>
+__device__ __forceinline__ typename Frag<T>::V load_diag(const T* z, int lk) {
+  typename Frag<T>::V d;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) d[r] = z[Frag<T>::col(lk, r) * (ZLD + 1)];
+  return d;
 }
-__device__ __forceinline__ Frag<float>::V solve(const Tri<float>& t, Frag<float>::V x, int lk) {
+
+// X := X inv(L)' by substitution (x_j *= 1/l_jj, or with DIV x_j /= l_jj, d
+// holding the diagonal; then x_c -= x_j l_cj).
+template <bool DIV>
+__device__ __forceinline__ Frag<double>::V solve(const Tri<double>& t, Frag<double>::V x, int lk,
+                                                 Frag<double>::V d) {
+  using S = std::conditional_t<DIV, fla_frag::ByQuotient, fla_frag::ByReciprocal>;
+  return fla_frag::solve_block<S>(t.l, t.cf, x, lk, d);
+}
+template <bool DIV>
+__device__ __forceinline__ Frag<float>::V solve(const Tri<float>& t, Frag<float>::V x, int lk,
+                                                Frag<float>::V d) {
   // columns 4q..4q+3 sit in the registers of the lanes with lk == q: solved
   // there, then four matrix steps with that k slot (the others zero on both
   // sides) update the later columns; the solved ones are kept as they are
@@ -96,13 +119,15 @@ __device__ __forceinline__ Frag<float>::V solve(const Tri<float>& t, Frag<float>
       float y = x[r];
 #pragma unroll
       for (int p = 0; p < r; ++p) y = fmaf(t.cf[r][1 + p], x[p], y);
-      x[r] = me ? y * t.cf[r][0] : x[r];
+      y = DIV ? fla_frag::quotient(y, t.cf[r][0], d[r]) : y * t.cf[r][0];
+      x[r] = me ? y : x[r];
     }
     if (q < 3) {
       Frag<float>::V y = x;
 #pragma unroll
       for (int s = 0; s < 4; ++s)
         y = Frag<float>::step(me ? t.l[s] : 0.0f, me ? x[s] : 0.0f, y);
+      y = settled(y);
 #pragma unroll
       for (int r = 0; r < 4; ++r) x[r] = lk > q ? y[r] : x[r];
     }
@@ -140,6 +165,9 @@ __device__ __forceinline__ void sweep_f(float (&x)[16], int li, float& pinv, int
   (sweep_column_f<J>(x, li, pinv, f, std::make_integer_sequence<int, 15 - J>{}), ...);
 }
 __device__ __forceinline__ int factor(Frag<float>::V dg, float* z, int lane) {
+  // LDS addresses formed here: kept from one block column to the next they
+  // are spilled, and the reload waits for memory inside the chain
+  asm volatile("" : "+v"(lane));
   const int li = lane & 15, lk = lane >> 4;
 #pragma unroll
   for (int r = 0; r < 4; ++r) z[li * ZLD + Frag<float>::col(lk, r)] = dg[r];
@@ -282,10 +310,23 @@ __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<
 #pragma unroll
     for (int u = 0; u < TMAX; ++u) {
       const int i = i0 + NW * u;
-      if (i >= nb + nr) break;  // uniform
+      if (i >= nb) break;  // uniform
       if (i == b) continue;
       const Row<T> p = block_row(i);
-      const V x = solve(tri, acc[u], lk);
+      const V x = solve<false>(tri, acc[u], lk, V{});
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (p.in && (!ragb || 16 * b + c0 + CS * r < n)) *p.at(b, r) = x[r];
+    }
+    // the right-hand sides (usually one block row, of one wave)
+    const V dg = load_diag(S.z[0], lk);
+    for (int i = nb + ((w - nb) & (NW - 1)); i < nb + nr; i += NW) {
+      V x = acc[0];
+#pragma unroll
+      for (int u = 1; u < TMAX; ++u)
+        if (i0 + NW * u == i) x = acc[u];
+      x = solve<true>(tri, x, lk, dg);
+      const Row<T> p = block_row(i);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (p.in && (!ragb || 16 * b + c0 + CS * r < n)) *p.at(b, r) = x[r];
@@ -336,7 +377,7 @@ __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<
         load_tri<T>(
             tri, li, lk, [&](int i, int j) { return S.z[par][i * ZLD + j]; },
             [&](int i) { return S.z[par][16 * ZLD + i]; });
-        x = solve(tri, x, lk);
+        x = solve<true>(tri, x, lk, load_diag(S.z[par], lk));
         S.x[par][lane] = x;
 #pragma unroll
         for (int r = 0; r < 4; ++r)

@@ -125,3 +125,15 @@ def test_entries_before_an_infinity_stay(dtype):
     assert list(info) == [i for i, _ in at]
     for (i, j), o in zip(at, out):
         assert np.array_equal(o[i, :j], F[i, :j]), (i, j)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_solves_divide(dtype):
+    """Exact quotients come out exactly (49 (1/49) is not 1)."""
+    d = np.resize([3.0, 49.0, 98.0, 103.0, 107.0], 40)
+    X = np.random.default_rng(3).integers(-4, 5, size=(40, 9)).astype(float)
+    A = np.diag(d * d)
+    out, sol, info = _run(dtype, [A], [A @ X], 0)
+    assert info[0] == fla.FLA_SUCCESS
+    assert np.array_equal(out[0], np.diag(d))
+    assert np.array_equal(sol[0], X)

@@ -29,7 +29,9 @@ constexpr int PB = FB;  // panel sub-block width (diagonal block order)
 // block (w, b), solves it against the factored diagonal block b, applies it
 // to its own diagonal block, and publishes it through LDS; wave b + 1 then
 // factors its diagonal block (factor16) while the others apply the previous
-// step's update to their remaining blocks.
+// step's update to their remaining blocks.  An update sums its sixteen terms
+// from zero: subtracted from the block one by one they left the factor of
+// B B'/n + I, n = 128, 2.1e-16 off (1.0e-16 from zero in a model of both).
 // Bound: the serial chain of 128 pivots (broadcast, root, reciprocal, scale,
 // update: about 200 cycles each) plus a block substitution and its updates
 // (about 3000 cycles) per 16 columns.  128 columns take 26 us alone, 73
@@ -86,12 +88,12 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
         for (int q = 0; q < 3; ++q) cf[s][1 + q] = -z[cc * ZLD + 4 * s + q];
       }
       d4 cur = c[0];
-      if (b > 0) cur = mfma_block(Xf[par ^ 1][b][0][lane], Xf[par ^ 1][b][1][lane], xr, cur);
+      if (b > 0) cur += mfma_block(Xf[par ^ 1][b][0][lane], Xf[par ^ 1][b][1][lane], xr, d4{});
       const d4 xn = solve_block(l, cf, cur, lk);
       const d2 n0 = d2{-xn[0], -xn[1]}, n1 = d2{-xn[2], -xn[3]};
       Xf[par][w][0][lane] = n0;
       Xf[par][w][1][lane] = n1;
-      dg = mfma_block(n0, n1, xn, dg);
+      dg += mfma_block(n0, n1, xn, d4{});
       if (w == b + 1) {
         __builtin_amdgcn_s_setprio(3);
         const int f = factor16(dg, Z[par ^ 1], lane);
@@ -102,9 +104,9 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
 #pragma unroll
       for (int i = 1; i < NT16 - 1; ++i) {
         if (i >= w - b) break;  // uniform
-        c[i - 1] = b > 0 ? mfma_block(Xf[par ^ 1][b + i][0][lane], Xf[par ^ 1][b + i][1][lane], xr,
-                                      c[i])
-                         : c[i];
+        c[i - 1] = c[i];
+        if (b > 0)
+          c[i - 1] += mfma_block(Xf[par ^ 1][b + i][0][lane], Xf[par ^ 1][b + i][1][lane], xr, d4{});
       }
       xr = xn;
       d2* const Wq = W + (frag_q0(w) + b) * 128;

@@ -52,3 +52,25 @@ def test_entries_before_an_infinity_stay(n, i, j):
     out, r = gpu_chol(A)
     assert r == i
     assert np.array_equal(out[i, :j], F[i, :j])
+
+
+@pytest.mark.parametrize("n", [100, 128])
+def test_sums_of_sixteen_terms(n):
+    """The diagonal factor sums sixteen terms from zero before it subtracts
+    them.  A model of its operations in that order is 0.9e-16 to 1.1e-16 off
+    a wider-precision factor of these matrices, one that subtracts term by term
+    1.7e-16 to 2.3e-16."""
+    for seed in range(4):
+        B = np.random.default_rng(seed).standard_normal((n, n))
+        A = B @ B.T / n + np.eye(n)
+        A = np.asfortranarray((A + A.T) / 2)
+        R = A.astype(np.longdouble)
+        for j in range(n):
+            R[j, j] = np.sqrt(R[j, j])
+            R[j + 1:, j] /= R[j, j]
+            R[j + 1:, j + 1:] -= np.outer(R[j + 1:, j], R[j + 1:, j])
+        R = np.tril(R)
+        out, r = gpu_chol(A)
+        assert r == fla.FLA_SUCCESS
+        err = np.linalg.norm((np.tril(out) - R).astype(float)) / np.linalg.norm(R.astype(float))
+        assert err < 1.4e-16, (seed, err)

@@ -45,11 +45,12 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
   if (*info >= 0) return;
   __shared__ d2 Xf[2][NT16][2][64];  // the solved blocks (negated) of a block column, by parity
   __shared__ __attribute__((aligned(16))) double Z[2][17 * ZLD];
-  __shared__ int fail;
+  // the failing column found in block b's factor, or -1, by b's parity: read
+  // only after the barrier that follows the write
+  __shared__ int fail[2];
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int li = lane & 15, lk = lane >> 4;
-  if (t == 0) fail = -1;
   // c[i]: block (w, b + i) at step b (i < w - b); dg: block (w, w)
   d4 c[NT16 - 1], dg;
   const int row = 16 * w + li;
@@ -68,14 +69,15 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
   }
   if (w == 0) {
     const int f = factor16(dg, Z[0], lane);
-    if (lane == 0 && f >= 0) fail = f;
+    if (lane == 0) fail[0] = f;
   }
+  int flim = -1;
   d4 xr = {0.0, 0.0, 0.0, 0.0};  // this row's block of the previous block column
   for (int b = 0; b < NT16; ++b) {
     lds_barrier();
     const int par = b & 1;
     const double* const z = Z[par];
-    const int flim = fail;
+    flim = fail[par];
     if (w > b && flim < 0) {
       __builtin_amdgcn_s_setprio(2);
       d4 l, cf[4];
@@ -97,7 +99,7 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
       if (w == b + 1) {
         __builtin_amdgcn_s_setprio(3);
         const int f = factor16(dg, Z[par ^ 1], lane);
-        if (lane == 0 && f >= 0) fail = 16 * w + f;
+        if (lane == 0) fail[par ^ 1] = f < 0 ? -1 : 16 * w + f;
       }
       __builtin_amdgcn_s_setprio(0);
       // the previous step's update of the blocks right of b, moved one place
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restri
     }
     if (flim >= 0) break;
   }
-  if (t == 0 && fail >= 0) *info = col_offset + fail;
+  if (t == 0 && flim >= 0) *info = col_offset + flim;
 }
 
 // Exchanges A(i,j) and A(j,i) for all i > j, 32x32 tile pairs through LDS.

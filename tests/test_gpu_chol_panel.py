@@ -74,3 +74,16 @@ def test_sums_of_sixteen_terms(n):
         assert r == fla.FLA_SUCCESS
         err = np.linalg.norm((np.tril(out) - R).astype(float)) / np.linalg.norm(R.astype(float))
         assert err < 1.4e-16, (seed, err)
+
+
+@pytest.mark.parametrize("k", [5, 16, 40, 63, 95, 111, 127, 135])
+def test_failing_column_keeps_finished_blocks(k):
+    """Column k's pivot fails: the 16-column blocks before it are the factor's
+    in all rows of the diagonal block."""
+    n = 200
+    A, F = exact_spd(n, seed=11)
+    A[k, k] -= F[k, k] ** 2 + 1.0
+    out, r = gpu_chol(A)
+    assert r == k
+    rows, cols = 128 * (k // 128) + 128, k // 16 * 16
+    assert np.array_equal(np.tril(out)[:rows, :cols], F[:rows, :cols])

@@ -204,8 +204,8 @@ struct Row {
 };
 
 // Factor (lower) of the n x n A and, with nrhs > 0, B := inv(A) B.  Returns
-// the first failing column or -1.  n >= 1, or n = 0 and nrhs = 0 (the staging
-// of the items sees to it).
+// the first failing column or -1; the columns before it are the factor's.
+// n >= 1, or n = 0 and nrhs = 0 (the staging of the items sees to it).
 template <typename T>
 __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<T>& S, int t) {
   typedef typename Frag<T>::V V;
@@ -302,7 +302,7 @@ __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<
         if (c <= li && pb.in && c < jend) *pb.at(b, r) = S.z[0][li * ZLD + c];
       }
     }
-    if (fail >= 0) return fail;
+    // (from a failing column on it holds anything, which no earlier one reads)
     Tri<T> tri;
     load_tri<T>(
         tri, li, lk, [&](int i, int j) { return S.z[0][i * ZLD + j]; },
@@ -316,8 +316,9 @@ __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<
       const V x = solve<false>(tri, acc[u], lk, V{});
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (p.in && (!ragb || 16 * b + c0 + CS * r < n)) *p.at(b, r) = x[r];
+        if (p.in && c0 + CS * r < jend) *p.at(b, r) = x[r];
     }
+    if (fail >= 0) return fail;
     // the right-hand sides (usually one block row, of one wave)
     const V dg = load_diag(S.z[0], lk);
     for (int i = nb + ((w - nb) & (NW - 1)); i < nb + nr; i += NW) {

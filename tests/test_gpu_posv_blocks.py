@@ -137,3 +137,20 @@ def test_solves_divide(dtype):
     assert info[0] == fla.FLA_SUCCESS
     assert np.array_equal(out[0], np.diag(d))
     assert np.array_equal(sol[0], X)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_failing_matrix_keeps_finished_columns(dtype):
+    """The columns before the failing one are the factor's in every row, those
+    of its own 16-column block too."""
+    cols = [5, 15, 16, 21, 47, 100]
+    A, F = _spd(101, 7)
+    mats = []
+    for k in cols:
+        M = A.copy()
+        M[k, k] -= F[k, k] ** 2 + 1.0
+        mats.append(M)
+    out, _, info = _run(dtype, mats, [np.ones((101, 2))] * len(cols), 0)
+    assert list(info) == cols
+    for k, o in zip(cols, out):
+        assert np.array_equal(np.tril(o)[:, :k], F[:, :k]), k

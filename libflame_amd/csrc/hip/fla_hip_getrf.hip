@@ -247,8 +247,16 @@ __global__ __launch_bounds__(NT, 2) void lu_sub_kernel(int M, int W, double* __r
                                                        int flip, int first,
                                                        int* __restrict__ pmoved,
                                                        unsigned tagbase) {
-  // A wait that expired in an earlier launch of this factorization aborts all later ones.
-  if (__hip_atomic_load(cm.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
+  // A wait that expired in an earlier launch of this factorization aborts all
+  // later ones; their move lists are empty (an older, taller panel's would
+  // move rows past this one's last).
+  if (__hip_atomic_load(cm.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      __hip_atomic_store(&cm.submoved[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (pmoved) __hip_atomic_store(&pmoved[0], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return;
+  }
   constexpr int NW = NT / 64;
   __shared__ __attribute__((aligned(16))) double crow[2][SW];  // the candidate's row, by parity
   __shared__ __attribute__((aligned(16))) double jrow[2][SW];  // row j before the interchange

@@ -1,6 +1,8 @@
 """The LU sub-panel kernel where it can go wrong: heights around the 512
 threads and the 1024 rows of a workgroup, ragged last sub-panels, and NaN or
 infinite entries in workgroups other than the pivot's."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -70,3 +72,40 @@ def test_non_finite_pivot_row_reaches_every_row(orc, m, value, c):
     assert np.array_equal(pv, pref)
     assert np.array_equal(np.isfinite(out), np.isfinite(ref))
     assert np.array_equal(np.isnan(out), np.isnan(ref))
+
+
+def test_after_an_expired_wait_no_rows_move(orc):
+    """Panels launched after a bounded wait of the factorization expired (here:
+    its flag is set beforehand) do nothing, and the interchanges queued behind
+    them move no rows, though the lists held a taller panel's before."""
+    L = fla.lib()
+    setup = L["_Z18fla_lu_panel_setupiPi"]
+    run = L["_Z16fla_lu_panel_runP12ihipStream_tiiiPdliPiS2_"]
+    gather = L["_Z18fla_lu_gather_rowsP12ihipStream_tiiPdl"]
+    setup.argtypes = [C.c_int, C.c_void_p]
+    run.argtypes = [C.c_void_p] + [C.c_int] * 3 + [C.c_void_p, C.c_long, C.c_int] + [C.c_void_p] * 2
+    gather.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_long]
+    hip = C.CDLL("libamdhip64.so")
+    w, piv = 128, fla.DeviceMatrix(128, 1, np.int32)
+    flags = fla.DeviceMatrix(2, 1, np.int32)  # expired, info
+
+    def panel(A, expired):
+        flags.upload(np.array([[expired], [-1]], dtype=np.int32))
+        d = fla.DeviceMatrix.from_host(A)
+        fla.check(setup(d.ld, flags.ptr))
+        m = A.shape[0] - 40  # the last 40 rows stay outside
+        fla.check(run(None, 0, m, w, d.ptr, d.ld, 0, piv.ptr, flags.ptr.value + 4))
+        c = fla.DeviceMatrix.from_host(A)
+        fla.check(gather(None, 0, w, c.ptr, c.ld))
+        assert hip.hipDeviceSynchronize() == 0
+        return d.download(), c.download()
+
+    tall = np.asfortranarray(orc.gen_lu_c2(3, 3040, w))
+    _, moved = panel(tall, 0)
+    assert not np.array_equal(moved, tall)  # its lists move rows
+    low = np.asfortranarray(orc.gen_lu_c2(4, 340, w))
+    out, moved = panel(low, 1)
+    assert np.array_equal(moved, low)
+    assert np.array_equal(out[300:], low[300:])
+    _, moved = panel(low, 0)
+    assert not np.array_equal(moved, low) and np.array_equal(moved[300:], low[300:])

@@ -82,7 +82,10 @@ int fla_hip_dgemm(int transa, int transb, int m, int n, int k, double alpha,
 /* C := alpha*op(A)*op(A)' + beta*C on the uplo triangle only. */
 int fla_hip_dsyrk(int uplo, int trans, int n, int k, double alpha, const double* A,
                   int lda, double beta, double* C, int ldc);
-/* B := alpha*inv(op(A))*B (left) or alpha*B*inv(op(A)) (right). */
+/* B := alpha*inv(op(A))*B (left) or alpha*B*inv(op(A)) (right).  With more
+   than 32 columns of B, or from the right, nothing is allocated and the call
+   can be captured into a graph; its workspace is the library's, so a replay
+   must not overlap other calls of the library. */
 int fla_hip_dtrsm(int side, int uplo, int trans, int diag, int m, int n, double alpha,
                   const double* A, int lda, double* B, int ldb);
 /* fla_hip_dtrsm without any device allocation.  No counterpart in the

@@ -63,11 +63,15 @@ struct FlaHipCtx {
   char* uc = nullptr;
   // The current Cholesky diagonal block as the panel solve reads it.
   double* dlinv = nullptr;
+  // kWideBlocks diagonal blocks as the triangular solve with many right-hand
+  // sides reads them.
+  double* wide_blocks = nullptr;
   int chol_nb = 0;  // 0: chosen from n (fla_chol_nb)
   int mp_nb = 0;    // reduced-precision factor block; 0: fla_chol_nb
   int lu_nb = 256;  // <= 128: panel width; 256: blocks of two 128-column panels
 };
 
+constexpr int kWideBlocks = 64;
 constexpr size_t kUcLuBytes = 4u << 20;
 constexpr long kUcSolveRows = 131072;
 constexpr size_t kUcBytes = kUcLuBytes + (size_t)kUcSolveRows * 16 * sizeof(double);
@@ -214,7 +218,7 @@ int launch_trsm_left_narrow(hipStream_t s, bool op_lower, bool trans, int na, in
 int launch_dgemm_tri_tn(hipStream_t s, int n, const double* A, long lda, const double* B, long ldb,
                         double* C, long ldc);
 // The triangular solve with many right-hand sides: op(A) X = B (left) or
-// X op(A) = B in place on the m x n B.  W: 128 x 128 doubles per 128-block of A.
+// X op(A) = B in place on the m x n B.  W: kWideBlocks 128 x 128 blocks.
 int trsm_wide(hipStream_t s, bool left, bool upper, bool tr, bool unit, int m, int n,
               const double* A, long lda, double* B, long ldb, double* W);
 // Inverts the 128x128 diagonal blocks of a triangle (lower or upper storage)

@@ -97,6 +97,8 @@ extern "C" int fla_hip_init(void) {
     FLA_HIP_CHECK(hipEventCreateWithFlags(&g_ctx.ev_user[i], hipEventDisableTiming));
   FLA_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&g_ctx.dscratch), 4096));
   FLA_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&g_ctx.dlinv), 128 * 128 * sizeof(double)));
+  FLA_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&g_ctx.wide_blocks),
+                          kWideBlocks * 128 * 128 * sizeof(double)));
   // uncached exchange memory: allocated once per process, never freed
   static char* uc = nullptr;
   if (!uc) {
@@ -129,6 +131,8 @@ extern "C" int fla_hip_finalize(void) {
   g_ctx.dscratch = nullptr;
   if (g_ctx.dlinv) FLA_HIP_CHECK(hipFree(g_ctx.dlinv));
   g_ctx.dlinv = nullptr;
+  if (g_ctx.wide_blocks) FLA_HIP_CHECK(hipFree(g_ctx.wide_blocks));
+  g_ctx.wide_blocks = nullptr;
   for (int i = 0; i < FlaHipCtx::kEvents; ++i) FLA_HIP_CHECK(hipEventDestroy(g_ctx.ev[i]));
   for (int i = 0; i < 4; ++i) FLA_HIP_CHECK(hipEventDestroy(g_ctx.ev_user[i]));
   FLA_HIP_CHECK(hipStreamDestroy(g_ctx.s_update));

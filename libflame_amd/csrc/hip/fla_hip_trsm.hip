@@ -4,12 +4,12 @@
 // src/flablas/f2c/dtrsm.c, used by FLA_Trsm_external and the solve paths
 // FLA_Chol_solve / FLA_LU_piv_solve / dpotrs_ / dgetrs_), blocked by 128:
 //   X_k := inv(op(T_kk)) * (B_k - sum_{j<k} op(T)_kj X_j)
-// The diagonal-block solves substitute in dtrsm_'s order (block staged in
-// LDS, one lane per right-hand side); the updates are MFMA GEMMs.  With at
-// most 32 right-hand sides on the left, one persistent launch per 16 columns
-// (fla_hip_trsv.hip) does the whole solve; it multiplies by the inverted
-// diagonal blocks (inverted in parallel, one workgroup per block) where their
-// condition number is at most kInvCondMax and substitutes through the rest.
+// The diagonal-block solves substitute in dtrsm_'s order (fla_hip_trsm_wide.hip);
+// the updates are MFMA GEMMs.  With at most 32 right-hand sides on the left,
+// one persistent launch per 16 columns (fla_hip_trsv.hip) does the whole
+// solve; it multiplies by the inverted diagonal blocks (inverted in parallel,
+// one workgroup per block) where their condition number is at most
+// kInvCondMax and substitutes through the rest.
 //
 // LU panel: A12 := inv(tril_unit(L11)) * A12 (FLA_LU_piv_blk_var5.c:88-91,
 // dtrsm_('L','L','N','U')): for a full 128-column panel, a blocked
@@ -341,21 +341,22 @@ static int dtrsm_args_ok(int side, int uplo, int m, int n, int lda, int ldb) {
   return (lda >= na && ldb >= m) ? 1 : 0;
 }
 
-// The few-right-hand-side path.
+// The few-right-hand-side path (the only one whose workspace depends on na).
 static bool dtrsm_narrow(int side, int n, int na) {
   return side == kLeft && n <= kNarrowRhs && na <= kUcSolveRows;
 }
 
-// Doubles of workspace dtrsm_body needs for a triangle of order na: the
-// inverted (few right-hand sides) or reordered 128-blocks, then int words: the wait counter, the wait-failure
-// flag and one condition flag per block.
+// Doubles of workspace the few-right-hand-side path needs for a triangle of
+// order na: the inverted 128-blocks, then int words: the wait counter, the
+// wait-failure flag and one condition flag per block.
 static size_t dtrsm_workspace_doubles(int na) {
   const size_t nblk = (size_t)((na + TB - 1) / TB);
   return nblk * TB * TB + 32 + nblk;
 }
 
 // dtrsm on checked, non-empty arguments with the caller's workspace W
-// (dtrsm_workspace_doubles(na) doubles of device memory).
+// (dtrsm_workspace_doubles(na) doubles of device memory, or, with many
+// right-hand sides, kWideBlocks 128 x 128 blocks).
 static int dtrsm_body(int side, int uplo, int trans, int diag, int m, int n, double alpha,
                       const double* A, int lda, double* B, int ldb, double* W) {
   const int na = (side == kLeft) ? m : n;  // order of A
@@ -398,8 +399,11 @@ extern "C" int fla_hip_dtrsm(int side, int uplo, int trans, int diag, int m, int
   if (!dtrsm_args_ok(side, uplo, m, n, lda, ldb)) return FLA_HIP_EARG;
   if (m == 0 || n == 0) return FLA_HIP_OK;
   const int na = (side == kLeft) ? m : n;
-  void* w = nullptr;
-  FLA_TRY(fla_workspace(dtrsm_workspace_doubles(na) * sizeof(double), &w));
+  // With many right-hand sides nothing is allocated, whatever the order: a
+  // first call can be captured, and a captured one keeps its workspace.
+  void* w = fla_ctx().wide_blocks;
+  if (dtrsm_narrow(side, n, na))
+    FLA_TRY(fla_workspace(dtrsm_workspace_doubles(na) * sizeof(double), &w));
   return dtrsm_body(side, uplo, trans, diag, m, n, alpha, A, lda, B, ldb,
                     static_cast<double*>(w));
 }
@@ -420,6 +424,7 @@ namespace {
 constexpr int kNoAllocMaxOrder = 8192;
 constexpr size_t kNoAllocDoubles = (size_t)(kNoAllocMaxOrder / TB) * TB * TB + 32 +
                                    kNoAllocMaxOrder / TB;
+static_assert(kNoAllocDoubles >= (size_t)kWideBlocks * TB * TB, "the wide solve's blocks fit");
 __device__ __align__(256) double scratch[kNoAllocDoubles];
 constexpr int kNoAllocDevices = 64;
 double* g_scratch_ptr[kNoAllocDevices] = {};

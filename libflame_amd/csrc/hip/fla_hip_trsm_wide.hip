@@ -6,8 +6,8 @@
 // Every case is one solve of row vectors with a lower-triangular block L on
 // the right, x L' = b, ascending: a solve from the left is its transpose
 // (the right-hand sides are the rows), and a descending one has its indices
-// reversed.  One launch per solve writes the diagonal blocks in that form and
-// in the order the solve reads them; one wave then solves 16 right-hand sides
+// reversed.  One launch per kWideBlocks diagonal blocks writes them in that
+// form and in the order the solve reads them; one wave then solves 16 right-hand sides
 // by substitution (dtrsm_'s update order; its division by the diagonal from the
 // left, its multiplication by the reciprocal from the right).
 #include "fla_hip_frag.h"
@@ -24,15 +24,18 @@ constexpr long kBlockStride = (long)FB * FB;  // doubles of workspace per diagon
 // over 512, so that the right-hand sides are read and written n / 512 times.
 constexpr int kGroup = 4;
 
-// Diagonal block kb = blockIdx.x of the triangle A: L(i, j) = U(j, i) for
+static_assert(kWideBlocks % kGroup == 0, "a group's blocks are written together");
+
+// Diagonal block k0 + blockIdx.x of the triangle A: L(i, j) = U(j, i) for
 // ascending solves x U = b (U upper), reversed otherwise; U(k, c) =
 // swap ? A(c, k) : A(k, c).  Identity beyond the block's order.  recip: the
 // diagonal's reciprocals among the coefficients, else the diagonal.
-__global__ __launch_bounds__(512) void pack_blocks_kernel(int n, const double* __restrict__ A,
-                                                          long lda, int swap, int rev, int unit,
-                                                          int recip, double* __restrict__ W) {
+__global__ __launch_bounds__(512) void pack_blocks_kernel(int n, int k0,
+                                                          const double* __restrict__ A, long lda,
+                                                          int swap, int rev, int unit, int recip,
+                                                          double* __restrict__ W) {
   __shared__ double S[FB * (FB + 1)];  // A's block: (i, j) at S[j * (FB + 1) + i]
-  const int r0 = blockIdx.x * FB, nb = min(FB, n - r0);
+  const int r0 = (k0 + blockIdx.x) * FB, nb = min(FB, n - r0);
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const int li = lane & 15, lk = lane >> 4;
   for (int q0 = 0; q0 < FB * FB / 512; q0 += 8) {
@@ -120,9 +123,6 @@ int trsm_wide(hipStream_t s, bool left, bool upper, bool tr, bool unit, int m, i
   const bool op_lower = upper == tr;
   const bool fwd = left ? op_lower : !op_lower;
   const int swap = left ? !tr : tr;
-  hipLaunchKernelGGL(pack_blocks_kernel, dim3((unsigned)nblk), dim3(512), 0, s, na, A, lda, swap,
-                     fwd ? 0 : 1, unit ? 1 : 0, left ? 0 : 1, W);
-  FLA_HIP_CHECK(hipGetLastError());
   // B[lo:hi) -= its product with the solved part [c0, c0 + k) of the triangle
   auto update = [&](int lo, int hi, int c0, int k) -> int {
     if (hi <= lo) return FLA_HIP_OK;
@@ -136,7 +136,15 @@ int trsm_wide(hipStream_t s, bool left, bool upper, bool tr, bool unit, int m, i
                              1.0, B + (long)lo * ldb, ldb, nullptr);
   };
   const dim3 grid((unsigned)((nrhs + 63) / 64));
+  int k0 = 0;  // the first diagonal block in W
   for (int q0 = 0; q0 < nblk; q0 += kGroup) {
+    if (q0 % kWideBlocks == 0) {
+      const int nw = nblk - q0 < kWideBlocks ? nblk - q0 : kWideBlocks;
+      k0 = fwd ? q0 : nblk - q0 - nw;
+      hipLaunchKernelGGL(pack_blocks_kernel, dim3((unsigned)nw), dim3(512), 0, s, na, k0, A, lda,
+                         swap, fwd ? 0 : 1, unit ? 1 : 0, left ? 0 : 1, W);
+      FLA_HIP_CHECK(hipGetLastError());
+    }
     const int q1 = q0 + kGroup < nblk ? q0 + kGroup : nblk;
     // the group's rows (columns) of the triangle
     const int g0 = (fwd ? q0 : nblk - q1) * FB;
@@ -144,7 +152,7 @@ int trsm_wide(hipStream_t s, bool left, bool upper, bool tr, bool unit, int m, i
     for (int q = q0; q < q1; ++q) {
       const int kb = fwd ? q : nblk - 1 - q;
       const int c0 = kb * FB, nb = na - c0 < FB ? na - c0 : FB;
-      const d2* w = reinterpret_cast<const d2*>(W + kb * kBlockStride);
+      const d2* w = reinterpret_cast<const d2*>(W + (kb - k0) * kBlockStride);
       if (left)
         hipLaunchKernelGGL(solve_block_kernel<true>, grid, dim3(256), 0, s, nrhs, nb, fwd ? 0 : 1,
                            w, B + c0, ldb);

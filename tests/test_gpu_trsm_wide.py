@@ -2,6 +2,8 @@
 wrong: edges of the 16-column blocks, the 128-blocks and the groups of four,
 ragged ends in both directions, and right-hand-side counts around a wave's 16
 rows.  Integer solutions of integer systems must come out exactly."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -114,4 +116,43 @@ def test_left_solves_divide(lower, trans):
     B = d[:, None] * X
     assert np.array_equal(B / d[:, None], X) and np.all(np.isfinite(B))
     out = _solve(np.diag(d), B, True, lower, trans)
+    assert np.array_equal(out, X)
+
+
+def test_wide_solve_allocates_nothing():
+    """A solve with many right-hand sides takes its block workspace from the
+    library's start, at any order: the free device memory does not change, so
+    the first call of a size can be captured."""
+    hip = C.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = C.c_size_t(0), C.c_size_t(0)
+        assert hip.hipDeviceSynchronize() == 0
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    n, nrhs = 40000, 33
+    dT, dB = fla.DeviceMatrix(n, n), fla.DeviceMatrix(n, nrhs)
+    before = free()
+    fla.check(fla.lib().fla_hip_dtrsm(fla.FLA_LEFT, fla.FLA_LOWER_TRIANGULAR, fla.FLA_NO_TRANSPOSE,
+                                      fla.FLA_UNIT_DIAG, n, nrhs, 1.0, dT.ptr, dT.ld, dB.ptr,
+                                      dB.ld))
+    assert free() == before
+
+
+@pytest.mark.parametrize("left,lower,trans", [(True, True, False), (True, True, True),
+                                              (False, True, False), (False, False, False)])
+def test_more_blocks_than_the_workspace_holds(left, lower, trans):
+    """Past 64 diagonal blocks the workspace is written again, in both directions."""
+    n, nrhs = 8192 + 700, 40
+    rng = np.random.default_rng(8)
+    T = np.zeros((n, n), order="F")
+    i, j = rng.integers(0, n, size=(2, 6 * n))
+    T[np.maximum(i, j), np.minimum(i, j)] = rng.integers(-2, 3, size=6 * n)
+    if not lower:
+        T = np.asfortranarray(T.T)
+    np.fill_diagonal(T, rng.choice([1.0, -2.0, 4.0], size=n))
+    X = rng.integers(-3, 4, size=(n, nrhs) if left else (nrhs, n)).astype(np.float64)
+    op = T.T if trans else T
+    out = _solve(T, op @ X if left else X @ op, left, lower, trans)
     assert np.array_equal(out, X)

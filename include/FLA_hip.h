@@ -198,7 +198,9 @@ int fla_hip_set_gemm_config(int cfg);
    that concurrently running tiles share operand panels in L2 (default 4). */
 int fla_hip_set_gemm_group(int G);
 /* CUs left out of the update stream's CU mask for the panel stream
-   (default 0: no mask). */
+   (default 0: no mask; then, and with the other stream's default, the steps of
+   FLA_Chol with at most 13000 trailing columns run on that stream, which leaves
+   32). */
 int fla_hip_set_reserved_cus(int reserved);
 
 /* ---- measurement ---- */
@@ -270,8 +272,9 @@ int fla_hip_mp_last_stats(double* out, int nout);
    with the diagonal factors' inverses.  One panel solve (blocked
    substitution) serves both, so the choice has no effect any more. */
 int fla_hip_mp_set_panel(int inverse);
-/* CUs left out of the reduced-precision factor's update stream for its panel
-   chain (default 32; 0 = no mask). */
+/* CUs left out of the second update stream for the panel chains beside it
+   (default 32; 0 = no mask): the reduced-precision factors' updates and the
+   bulk updates of FLA_LU_piv. */
 int fla_hip_mp_set_reserved_cus(int reserved);
 /* Outer block of the reduced-precision factor (multiple of 128; 0 = the
    FP64 Cholesky's choice for the order). */

@@ -291,7 +291,7 @@ static int chol_lower(int n, double* A, long lda, int* dinfo) {
     const int k2 = k + kb;      // first column of the trailing matrix
     const int m2 = n - k2;      // its order
     if (m2 <= 0) break;
-    if (su == c.s_update && m2 <= kMaskedOrder) {
+    if (su == c.s_update && m2 <= kMaskedOrder && fla_chol_tail_on_lp()) {
       // from here on the panel chain outlasts the update: it gets CUs of its own
       hipEvent_t sw = next_event();
       FLA_HIP_CHECK(hipEventRecord(sw, su));

@@ -32,10 +32,9 @@ struct FlaHipCtx {
   int num_cus = 0;
   hipStream_t s_update = nullptr;  // trailing updates (and the API's default stream)
   hipStream_t s_panel = nullptr;   // panel factorizations (look-ahead)
-  // Trailing updates of the reduced-precision factor: their panel chain, not
-  // the update, is the critical path, so this stream leaves more CUs free.
-  // 32 CUs left to the panels: the reduced-precision factor's updates and the
-  // LU's bulk updates beside its panel chain
+  // Updates whose panel chain, not the update, is the critical path, with 32 CUs
+  // left to the panels: the reduced-precision factors', the LU's bulk updates
+  // and the last steps of FLA_Chol.
   hipStream_t s_update_lp = nullptr;
   static constexpr int kEvents = 8;
   hipEvent_t ev[kEvents] = {};
@@ -82,6 +81,9 @@ FlaHipCtx& fla_ctx();
 // larger blocks raise the trailing update's arithmetic intensity).
 int fla_chol_nb(int n);
 int fla_ensure_ready();
+// The last steps of FLA_Chol may run on s_update_lp: while both update streams
+// leave as many CUs as the library chooses.
+bool fla_chol_tail_on_lp();
 // Orders a public entry point's device work after the work already queued on
 // the caller's stream (on construction) and that stream's later work after
 // the entry point's (on destruction), when a caller's stream is set.  Uses

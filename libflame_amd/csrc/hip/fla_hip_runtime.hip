@@ -5,8 +5,8 @@
 // (FLASH_Queue_bind_hip, src/base/flamec/supermatrix/hip/main/FLASH_Queue_hip.c:297-318);
 // here one process drives one GPU through three streams: s_update for trailing
 // updates, s_panel for the look-ahead panel chain, and s_update_lp (32 CUs
-// left to the panels) for the reduced-precision factor's updates and the
-// LU's bulk updates.
+// left to the panels) for the reduced-precision factor's updates, the LU's
+// bulk updates and the last steps of FLA_Chol.
 #include <cstdlib>
 #include <cstring>
 
@@ -23,8 +23,8 @@ FlaHipCtx& fla_ctx() { return g_ctx; }
 // rate, since every shader engine gets the same share of its workgroups.
 static int g_reserved_cus = 0;
 // The second update stream leaves 32 CUs (four of each XCD) to the panels.
-// It carries the reduced-precision factor's updates and the LU's bulk
-// updates, whose panel kernel needs one whole CU per 1024 rows with all its
+// It carries the reduced-precision factor's updates, the last steps of
+// FLA_Chol (kMaskedOrder) and the LU's bulk updates, whose panel kernel needs one whole CU per 1024 rows with all its
 // workgroups resident.  Measured at n = 16384 with 64, 48, 32, 24, 16 and 8
 // CUs left: FLA_LU_piv 120.0, 120.9, 116.6, 124.3, 126.2, 127.4 ms; the mixed
 // solve 32.0, 32.0, 30.5, 31.1, 31.7, 32.0 ms (n = 8000-8192: within 1 %).
@@ -32,7 +32,13 @@ static int g_reserved_cus = 0;
 // stream, fit the four hardware queues HIP gives a process: two busy streams
 // sharing a queue serialize (an LU with its bulk stream on the panel's queue
 // took 182 ms instead of 134 ms).
-static int g_lp_reserved_cus = 32;
+constexpr int kLpReservedCus = 32;
+static int g_lp_reserved_cus = kLpReservedCus;
+
+// The two counts are tuning values of other paths: a caller's own must not
+// decide where FLA_Chol's last steps run (with 224 CUs left out of the second
+// stream they would have 32).
+bool fla_chol_tail_on_lp() { return g_reserved_cus == 0 && g_lp_reserved_cus == kLpReservedCus; }
 
 static int create_masked_stream(hipStream_t* s, int reserved) {
   if (reserved <= 0 || reserved >= g_ctx.num_cus) {

@@ -116,3 +116,34 @@ def test_chol_host_buffer_staging(orc):
     assert fla.lib().FLA_Obj_is_device(o.o) == 0
     assert fla.FLA_Chol(fla.FLA_LOWER_TRIANGULAR, o) == fla.FLA_SUCCESS
     assert np.array_equal(np.tril(host), F)
+
+
+def test_tuning_of_other_streams_leaves_chol_alone():
+    """A CU count set for the reduced-precision factors' stream changes neither
+    the factor nor where it runs: with 224 of 256 CUs left out there, FLA_Chol
+    on that stream would take several times as long (32 CUs: 9 TFLOP/s at most,
+    37 ms for this order against about 10)."""
+    import time
+
+    n = 10000
+    A = fla.DeviceMatrix(n, n)
+    fla.check(fla.lib().fla_hip_gen_spd_reflectors(1, n, 2, 10.0, A.ptr, n))
+    F = fla.DeviceMatrix(n, n)
+
+    def factor():
+        best = 1e9
+        for _ in range(3):
+            fla.check(fla.lib().fla_hip_memcpy_d2d(F.ptr, A.ptr, 8 * n * n))
+            t = time.perf_counter()
+            assert fla.FLA_Chol(fla.FLA_LOWER_TRIANGULAR, F.obj()) == fla.FLA_SUCCESS
+            best = min(best, time.perf_counter() - t)
+        return best, F.download()
+
+    t0, L0 = factor()
+    fla.check(fla.lib().fla_hip_mp_set_reserved_cus(224))
+    try:
+        t1, L1 = factor()
+    finally:
+        fla.check(fla.lib().fla_hip_mp_set_reserved_cus(32))
+    assert np.array_equal(L0, L1)
+    assert t1 < 2 * t0, (t0, t1)

@@ -55,8 +55,9 @@ def dev_reflector_spd(seed, n, nrefl, kappa):
 
 @pytest.fixture
 def substitution_panel():
-    """Exact closed forms need the backward-stable panel solve: the factors of
-    these integer matrices have astronomically large inverses."""
+    """Exact closed forms need a backward-stable panel solve (the factors of these
+    integer matrices have astronomically large inverses): the one there is, under
+    either value of the switch."""
     fla.lib().fla_hip_mp_set_panel(0)
     yield
     fla.lib().fla_hip_mp_set_panel(1)
@@ -81,8 +82,8 @@ def test_mp_chol_exact_upper(precision, substitution_panel):
 
 @pytest.mark.parametrize("inverse", [0, 1])
 def test_mp_chol_panel_modes_agree(orc, inverse):
-    """Both panel solves give a factor of FP32 quality on a well-conditioned
-    matrix (the inverse of a diagonal factor is then well conditioned)."""
+    """Either value of the panel switch, which has no effect, is accepted and gives
+    a factor of FP32 quality."""
     n = 900
     A = orc.gen_spd_c2(12, n)
     fla.lib().fla_hip_mp_set_panel(inverse)

@@ -129,14 +129,18 @@ def test_entries_before_an_infinity_stay(dtype):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_solves_divide(dtype):
-    """Exact quotients come out exactly (49 (1/49) is not 1)."""
+    """Exact quotients come out exactly (49 (1/49) is not 1), and infinities, NaN
+    and overflowing quotients as a division gives them."""
     d = np.resize([3.0, 49.0, 98.0, 103.0, 107.0], 40)
     X = np.random.default_rng(3).integers(-4, 5, size=(40, 9)).astype(float)
     A = np.diag(d * d)
-    out, sol, info = _run(dtype, [A], [A @ X], 0)
-    assert info[0] == fla.FLA_SUCCESS
+    big = 0.75 * float(np.finfo(dtype).max)
+    special = np.array([[np.inf, -np.inf, np.nan, 0.0, big, -big]])
+    out, sol, info = _run(dtype, [A, np.array([[0.25]])], [A @ X, special], 0)
+    assert np.all(info == fla.FLA_SUCCESS)
     assert np.array_equal(out[0], np.diag(d))
     assert np.array_equal(sol[0], X)
+    assert np.array_equal(sol[1], [[np.inf, -np.inf, np.nan, 0.0, np.inf, -np.inf]], equal_nan=True)
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])

@@ -764,7 +764,7 @@ __global__ void reset_counter_kernel(int* c) { *c = 0; }
 // ---- host side: schedule, configurations, autotuner, graph replay ----------
 
 struct BatchConfig {
-  int nb = 16;        // panel width of the LU kernel
+  int nb = 16;        // the LU kernel's panel width; no effect on the Cholesky kernel
   int wg_per_cu = 1;  // persistent workgroups per CU
 };
 
@@ -805,8 +805,9 @@ Signature signature_of(int count, const int* n, const int* nrhs) {
   return s;
 }
 
-// The fastest configurations measured on 4096 matrices of n ~ U{32..512}
-// with 1-8 right-hand sides.
+// Workgroups launched per CU.  The Cholesky kernel's registers let one (FP64)
+// or two (FP32) run at a time, the LU kernel's LDS two; those beyond start when
+// one ends and find the queue empty.
 BatchConfig default_config(int kind) {
   BatchConfig c;
   c.nb = 16;
@@ -852,8 +853,9 @@ bool valid_nb(int kind, int nb) {
   return nb == 16 || nb == 32;
 }
 
-// Most workgroups per CU worth a try (at most 4): those a 32- or 16-column
-// panel of the largest matrix in LDS allows.
+// Most workgroups per CU that the tuner tries (at most 4): those that a panel of
+// nb columns of the largest matrix in LDS allows, which bounds the LU kernel
+// (the Cholesky kernel's registers allow fewer).
 int max_wg_per_cu(int kind, int nb) {
   const int bytes = (MAXN + 32) * nb * (kind == kSpotrf ? 4 : 8) + 1024;
   return std::max(1, std::min(4, (160 * 1024) / bytes));

@@ -34,9 +34,11 @@ constexpr int PB = FB;  // panel sub-block width (diagonal block order)
 // B B'/n + I, n = 128, 2.1e-16 off (1.0e-16 from zero in a model of both).
 // Bound: the serial chain of 128 pivots (broadcast, root, reciprocal, scale,
 // update: about 200 cycles each) plus a block substitution and its updates
-// (about 3000 cycles) per 16 columns.  128 columns take 26 us alone, 73
+// (about 3000 cycles) per 16 columns.  128 columns take 27 us alone, 73
 // with the block in LDS, lane reads for the multipliers and three barriers
-// per 32 columns.
+// per 32 columns.  Its registers are a whole CU's: beside an update without a
+// CU mask it waits for a CU to drain (n = 32768: 399 us on average, 15 ms at
+// most, hidden while the update is the longer chain).
 // W receives the blocks of L for the panel solve (see frag_q0).  A failed
 // block leaves its columns from the failing one on unwritten.
 __global__ __launch_bounds__(512) void potrf_blk_kernel(int nb, double* __restrict__ A, long lda,

@@ -404,7 +404,8 @@ __device__ int posv_one(T* A, long lda, int n, T* B, long ldb, int nrhs, Shared<
         if (j >= b) break;
         // accumulated by the matrix steps themselves: as y -= L x the
         // subtraction opens the block behind the next pass's branch, where the
-        // compiler left out the wait for the steps' last register
+        // compiler left out the wait for the steps' last register (a test
+        // searches the built code for such reads)
         y[u] = product<T>(-lb[u], x, y[u]);
       }
     }

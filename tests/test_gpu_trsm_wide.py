@@ -156,3 +156,35 @@ def test_more_blocks_than_the_workspace_holds(left, lower, trans):
     op = T.T if trans else T
     out = _solve(T, op @ X if left else X @ op, left, lower, trans)
     assert np.array_equal(out, X)
+
+
+def test_captured_call_replays():
+    """A solve captured on the caller's stream gives the eager result on every
+    replay, with the program's own copies and synchronisations in between."""
+    hip, L = C.CDLL("libamdhip64.so"), fla.lib()
+    n, nrhs = 700, 96
+    T = _sparse_tri(n, True)
+    B = np.asfortranarray(T @ np.random.default_rng(1).integers(-4, 5, size=(n, nrhs)))
+    want = _solve(T, B, True, True, False)
+    dT, dB = fla.DeviceMatrix.from_host(T), fla.DeviceMatrix.from_host(B)
+    s, g, x = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreate(C.byref(s)) == 0
+    fla.check(L.fla_hip_set_stream(s))
+    try:
+        assert hip.hipStreamBeginCapture(s, 1) == 0  # thread local
+        st = L.fla_hip_dtrsm(fla.FLA_LEFT, fla.FLA_LOWER_TRIANGULAR, fla.FLA_NO_TRANSPOSE,
+                             fla.FLA_NONUNIT_DIAG, n, nrhs, 1.0, dT.ptr, dT.ld, dB.ptr, dB.ld)
+        assert hip.hipStreamEndCapture(s, C.byref(g)) == 0
+        fla.check(st)
+    finally:
+        fla.check(L.fla_hip_set_stream(None))
+    assert np.array_equal(dB.download(), B)  # captured, not run
+    assert hip.hipGraphInstantiate(C.byref(x), g, None, None, C.c_size_t(0)) == 0
+    for _ in range(3):
+        dB.upload(B)
+        assert hip.hipGraphLaunch(x, s) == 0
+        assert hip.hipStreamSynchronize(s) == 0
+        assert np.array_equal(dB.download(), want)
+        assert np.array_equal(_solve(T, B, True, True, False), want)
+    assert hip.hipGraphExecDestroy(x) == 0 and hip.hipGraphDestroy(g) == 0
+    assert hip.hipStreamDestroy(s) == 0
